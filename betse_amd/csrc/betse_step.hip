@@ -758,6 +758,9 @@ k_mem_cell(MemCellArgs A, KParams P) {
     else mem_cell_wave<NI, FT, WG, WG - 1, OBS>(A, P, tile, L);
 }
 
+// bits of the per-square flags the env kernel reads
+constexpr uint8_t SQ_LIVE = 1, SQ_HAS_MEM = 2;
+
 // ---------------------------------------------------------------------------
 // k_env_field: Gaussian + E field from u, then update_ecm for every ion
 // ---------------------------------------------------------------------------
@@ -775,7 +778,7 @@ struct FieldArgs {
     // diffuse mode: a square without membranes has no exchange, so its
     // post-diffusion value is already the step's new env state and goes to
     // c_env_out; squares with membranes go to c_mid for k_env_exchange
-    const uint8_t* live;      // per square: 1 if k_env_exchange updates it
+    const uint8_t* live;      // per square: SQ_LIVE if k_env_exchange updates it, SQ_HAS_MEM where sq_has_mem is set
     double* c_env_out;        // the step's env state buffer (never the one read here)
     const double* Phi_b = nullptr;   // applied boundary voltage per square (clusters with phib)
     // the exchange done by this kernel (k_mem_cell ran first: no ion's
@@ -784,7 +787,7 @@ struct FieldArgs {
     // sq_ptr[k+1])) to its diffused value, and the surface charge of the
     // step's env state goes to u_out (not u, which neighbouring tiles still
     // read); the block of tile 0 advances the step counters of ctr_mask
-    const int32_t* sq_ptr = nullptr; const uint8_t* has_mem = nullptr; const void* fsa = nullptr;
+    const int32_t* sq_ptr = nullptr; const void* fsa = nullptr;
     int fsa32 = 0;
     double* u_out = nullptr;
     long long* step_ctr = nullptr; unsigned ctr_mask = 0; int count_step = 0;
@@ -838,24 +841,122 @@ __device__ __forceinline__ double neg_flux_sum(const void* fsa, int fsa32, size_
                  : neg_seg_sum<double, W>(static_cast<const double*>(fsa) + row, a, b, S);
 }
 
-// FUSE: the first FUSE_PF membrane fluxes of a square's row, loaded at the
-// start of the ion's iteration so that their latency passes in its flux
-// stages; the rest FUSE_W at a time
-constexpr int FUSE_PF = 2;
+// FUSE: the membrane fluxes of FUSE_I ions of a square are summed together,
+// FUSE_W membranes of each loaded at a time (16 loads in flight)
+constexpr int FUSE_I = 2;
 constexpr int FUSE_W = 4;
 
-// LDS of one k_env_field tile, in doubles
-constexpr int ENV_UH = 6;                                        // u on tile +- 6
-constexpr int ENV_A1 = (TY + 2 * ENV_UH) * (TX + 2 * ENV_UH) + (TY + 4) * (TX + 2 * ENV_UH);
-constexpr int ENV_A2 = (TY + 4) * (TX + 4) + (TY + 2) * (TX + 2) + TY * (TX + 2) + (TY + 2) * TX;
+// Four consecutive fluxes of a row from an address aligned to one of them, by
+// 16-byte loads: the vector-memory address unit takes 16 cycles for a
+// wavefront's gather whether a lane asks for 8 bytes or 16, and it is what
+// bounds these kernels. A run may reach FSA_PAD values past a square's own
+// membranes (into the next square's, the next row, or the allocation's padding);
+// those are not used.
+constexpr int FSA_PAD = FUSE_W - 1;
+template <typename T>
+struct Run4 {
+    T x[4];
+};
+__device__ __forceinline__ Run4<double> load_run4(const double* p) {
+    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+    const d2 lo = *reinterpret_cast<const d2*>(p), hi = *reinterpret_cast<const d2*>(p + 2);
+    return {{lo.x, lo.y, hi.x, hi.y}};
+}
+__device__ __forceinline__ Run4<float> load_run4(const float* p) {
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    const f4 v = *reinterpret_cast<const f4*>(p);
+    return {{v.x, v.y, v.z, v.w}};
+}
+
+// The negated sums of a square's membrane fluxes over its membranes [a, b), in
+// membrane order, of every ion i in the mask (wave-uniform), to out[i * stride].
+template <typename T>
+__device__ __forceinline__ void neg_flux_sums(const T* fsa, int n_mems, unsigned mask, int a, int b, double* out,
+                                              int stride) {
+    while (mask) {
+        int ion[FUSE_I];
+        unsigned rest = mask;
+#pragma unroll
+        for (int s = 0; s < FUSE_I; ++s) {
+            ion[s] = __builtin_ctz(rest);
+            const unsigned less = rest & (rest - 1u);
+            rest = less ? less : rest;           // past the last ion: it again, to the same slot
+        }
+        double S[FUSE_I] = {};
+        for (int q0 = a; q0 < b; q0 += FUSE_W) {
+            Run4<T> t[FUSE_I];
+#pragma unroll
+            for (int s = 0; s < FUSE_I; ++s) t[s] = load_run4(fsa + (size_t)ion[s] * n_mems + q0);
+#pragma unroll
+            for (int s = 0; s < FUSE_I; ++s)
+#pragma unroll
+                for (int u = 0; u < FUSE_W; ++u)
+                    if (q0 + u < b) S[s] = S[s] + (-(double)t[s].x[u]);
+        }
+#pragma unroll
+        for (int s = 0; s < FUSE_I; ++s) out[ion[s] * stride] = S[s];
+#pragma unroll
+        for (int s = 0; s < FUSE_I; ++s) mask &= ~(1u << ion[s]);
+    }
+}
+
+// LDS of one k_env_field tile, in doubles: u on tile +- 6 and its axis-0 pass
+// (20 rows of 28), whose space the ion loop's two concentration and two D_env
+// buffers then take; v_env on tile +- 2; the cluster's uniform D_env per ion
+constexpr int ENV_UH = 6;
+constexpr int ENV_VR = TY + 4, ENV_VC = TX + 4, ENV_ER = TY + 2, ENV_EC = TX + 2;
+constexpr int ENV_A1 = (TY + 2 * ENV_UH) * (TX + 2 * ENV_UH) + ENV_VR * (TX + 2 * ENV_UH);
+constexpr int ENV_A2 = 2 * ENV_VR * ENV_VC + 2 * ENV_ER * ENV_EC;
 constexpr int ENV_POOL = ENV_A1 > ENV_A2 ? ENV_A1 : ENV_A2;
-constexpr int ENV_LDS = ENV_POOL + (TY + 4) * (TX + 4) + 2 * (TY + 2) * (TX + 2) + BT_MAX_IONS;
+constexpr int ENV_LDS = ENV_POOL + ENV_VR * ENV_VC + BT_MAX_IONS;
+
+// Where a square's difference stencils read along one axis, as offsets in
+// squares from it: its neighbours L and R (itself at the world's edge) and the
+// squares the gradients at L and R difference, with their factors (one-sided at
+// the edge, finitediff.py:1236-1266) and the divergence's, whose one-sided
+// edges carry the opposite sign (Q4, finitediff.py:1268-1311).
+struct EnvAxis {
+    int L, R, Llo, Lhi, Rlo, Rhi;
+    double fL, fR, fdiv;
+};
+__device__ __forceinline__ EnvAxis env_axis(int c, int n, double rdl, double rd2) {
+    EnvAxis a;
+    const int l = max(c - 1, 0), r = min(c + 1, n - 1);
+    a.L = l - c;
+    a.R = r - c;
+    a.Llo = max(l - 1, 0) - c;
+    a.Lhi = min(l + 1, n - 1) - c;
+    a.Rlo = max(r - 1, 0) - c;
+    a.Rhi = min(r + 1, n - 1) - c;
+    a.fL = (l == 0 || l == n - 1) ? rdl : rd2;
+    a.fR = (r == 0 || r == n - 1) ? rdl : rd2;
+    a.fdiv = (c == 0 || c == n - 1) ? -rdl : rd2;
+    return a;
+}
+// the same inside the world (2 <= c <= n - 3): constants
+__device__ __forceinline__ EnvAxis env_axis_inner(double rd2) {
+    return EnvAxis{-1, 1, -2, 0, 0, 2, rd2, rd2, rd2};
+}
 
 // One env tile's work for the ion group ion_id of n_groups (the ions
 // [ion_id * ipb, ion_id * ipb + ipb), ipb = ceil(n_ions / n_groups)), with
 // the block's LDS at lds (ENV_LDS doubles). With RATES the block's threads also
 // evaluate the gating-rate items rate_first, rate_first + rate_stride, ...
-template <bool DIFFUSE, bool RATES, bool FUSE = false>
+//
+// A thread owns one square. The divergence at a square needs the fluxes of its
+// four neighbours only, and each of those the two concentrations beside it, so
+// the thread evaluates the four fluxes itself from the staged concentrations:
+// one LDS buffer and one barrier per ion (two buffers alternate), where fluxes
+// staged in LDS took three barriers and a halo of their own. The field at the
+// four neighbours does not depend on the ion: it is differenced from v_env once
+// and stays in registers. Together with the 16-byte loads (a row's concentrations
+// and u in pairs, membrane fluxes in runs of four): with the exchange on the
+// 500k-cell batch 95.4 -> 84.8 us, 512x512 squares over six ions 21.0 -> 18.7 us,
+// 256x256 squares with two ions a block 10.2 -> 8.3 us.
+//
+// DVAR: some cluster's D_env varies over its squares (its values are staged
+// too; 20 VGPRs that a uniform D_env does without); OBS: an observed step.
+template <bool DIFFUSE, bool RATES, bool FUSE, bool DVAR, bool OBS>
 __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams& P, int tile_id, int ion_id,
                                                int n_groups, double* lds, int rate_first, int rate_stride,
                                                bool check_halt = true) {
@@ -865,32 +966,20 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // decided for the whole block passes check_halt = false)
     const bool stop = check_halt && halted(A.flags);
     constexpr int UH = ENV_UH, UR = TY + 2 * UH, UC = TX + 2 * UH;   // u on tile +- 6
-    constexpr int TR = TY + 4;                                  // row-blurred rows tile +- 2
-    constexpr int VR = TY + 4, VC = TX + 4;                     // v on tile +- 2
-    constexpr int ER = TY + 2, EC = TX + 2;                     // E on tile +- 1
-    // the Gaussian staging (sU, sT) is dead once v_env is built, so the
-    // diffusion staging (sC, sD, sFx, sFy) reuses its LDS
-    double* s_pool = lds;
-    double (&sV)[VR][VC] = *reinterpret_cast<double (*)[VR][VC]>(lds + ENV_POOL);
-    double (&sEx)[ER][EC] = *reinterpret_cast<double (*)[ER][EC]>(lds + ENV_POOL + VR * VC);
-    double (&sEy)[ER][EC] = *reinterpret_cast<double (*)[ER][EC]>(lds + ENV_POOL + VR * VC + ER * EC);
-    double* s_du = lds + ENV_POOL + VR * VC + 2 * ER * EC;
-    double (&sU)[UR][UC] = *reinterpret_cast<double (*)[UR][UC]>(s_pool);
-    double (&sT)[TR][UC] = *reinterpret_cast<double (*)[TR][UC]>(s_pool + UR * UC);
-    double (&sC)[VR][VC] = *reinterpret_cast<double (*)[VR][VC]>(s_pool);
-    double (&sD)[ER][EC] = *reinterpret_cast<double (*)[ER][EC]>(s_pool + VR * VC);
-    double (&sFx)[TY][TX + 2] = *reinterpret_cast<double (*)[TY][TX + 2]>(s_pool + VR * VC + ER * EC);
-    double (&sFy)[TY + 2][TX] =
-        *reinterpret_cast<double (*)[TY + 2][TX]>(s_pool + VR * VC + ER * EC + TY * (TX + 2));
+    constexpr int VR = ENV_VR, VC = ENV_VC;                     // v and concentrations on tile +- 2
+    constexpr int ER = ENV_ER, EC = ENV_EC;                     // D_env on tile +- 1
+    double* sU = lds;                                           // [UR][UC]
+    double* sT = lds + UR * UC;                                 // [VR][UC]
+    double* sV = lds + ENV_POOL;                                // [VR][VC]
+    double* s_du = sV + VR * VC;
     const int* et = A.env_tiles + 3 * tile_id;
-    const KCluster K = A.kcl[et[0]];
-    const int ny = K.ny, nx = K.nx, so = K.sq_off;
+    const KCluster* K = A.kcl + et[0];
+    const int ny = K->ny, nx = K->nx, so = K->sq_off;
     const int r0 = et[1], cc0 = et[2];
     const int tid = threadIdx.x;
-    const double dl = K.delta, d2 = K.two_delta;
-    const double rdl = 1.0 / dl, rd2 = 1.0 / d2;
-    auto per_dl = [&](double x) { return x * rdl; };
-    auto per_d2 = [&](double x) { return x * rd2; };
+    const double rdl = 1.0 / K->delta, rd2 = 1.0 / K->two_delta;
+    const double screen = K->screen;
+    const unsigned still_mem = K->still_mem;
 
     // ion group ion_id takes the ions [ion_id * ipb, ion_id * ipb + ipb), with
     // ipb = ceil(n_ions / n_groups), and rebuilds its tile's field for them
@@ -905,39 +994,38 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // through the previous ion's flux stages (barriers wait for LDS only).
     const int nc = P.n_cells;
     const int items = RATES ? P.n_chan * nc : 0;
-    const int nthr = rate_stride;
-    const int t_first = rate_first;
     double vm_first = 0.0;
-    if (RATES && t_first >= 0 && t_first < items) vm_first = A.vm[t_first % nc];
+    if (RATES && rate_first >= 0 && rate_first < items) vm_first = A.vm[rate_first % nc];
     double du_mine = 0.0;
-    if (DIFFUSE && tid < P.n_ions) du_mine = A.kcl[et[0]].denv_u[tid];
+    if (DIFFUSE && tid < P.n_ions) du_mine = K->denv_u[tid];
 
+    static_assert(TY == 16 && TX == 16, "a thread per square of a 16 x 16 tile");
+    const int lr = tid / TX, lc = tid % TX;                // own square in the tile
+    const int r_own = r0 + lr, c_own = cc0 + lc;
+    const bool own_in = r_own < ny && c_own < nx;
+    const int k_own = so + r_own * nx + c_own;
     // whether this thread's square goes to the exchange (c_mid) or is final (c_env_out)
     // (an empty asm at the store keeps the compiler from testing it, and so
     // waiting for every load issued before it, right after the load)
     unsigned live_b = 0;
     int fa = 0, fb = 0;             // FUSE: the square's membranes in fsa's rows
-    unsigned hm = 0;
-    if (DIFFUSE) {
-        const int r = r0 + tid / TX, cc = cc0 + tid % TX;
-        if (r < ny && cc < nx) {
-            live_b = A.live[so + r * nx + cc];
-            if (FUSE) {
-                fa = A.sq_ptr[so + r * nx + cc];
-                fb = A.sq_ptr[so + r * nx + cc + 1];
-                hm = A.has_mem[so + r * nx + cc];
-            }
+    if (DIFFUSE && own_in) {
+        live_b = A.live[k_own];
+        if (FUSE) {
+            typedef int i2 __attribute__((ext_vector_type(2), aligned(4)));
+            const i2 f = *reinterpret_cast<const i2*>(A.sq_ptr + k_own);
+            fa = f.x;
+            fb = f.y;
         }
     }
-    // The squares of ion data a thread stages: its own square of the tile
-    // (row tid / TX, column tid % TX) and one square of the ring around the
-    // tile, for the concentrations on tile +- 2 (the RC squares of the
-    // (TY + 4) x (TX + 4) block outside the tile: thread t < RC takes ring
-    // square t) and for D_env on tile +- 1 (RD squares, t < RD). Their
-    // clamped in-grid offsets, LDS slots and edge flags are set once per tile,
-    // so an ion's loads and staging take no index arithmetic.
-    static_assert(TY == 16 && TX == 16, "the halo flux mapping assumes 16 x 16 tiles");
-    constexpr int RC = VR * VC - TY * TX;
+    // The squares of ion data a thread stages: for the concentrations on tile
+    // +- 2 two neighbours of a row (thread t < VR * VC / 2 takes pair t of the
+    // block), so that an ion is one 16-byte load per thread; for a varying
+    // D_env on tile +- 1 its own square and one of the RD squares of the ring
+    // around the tile (t < RD). Their clamped in-grid offsets, LDS slots and
+    // edge flags are set once per tile, so an ion's loads and staging take no
+    // index arithmetic.
+    constexpr int NP = VR * VC / 2;
     constexpr int RD = ER * EC - TY * TX;
     // ring square t of the block of width w around the tile: the w top rows,
     // the w bottom rows, then the w left and w right squares of each tile row
@@ -958,47 +1046,60 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
         }
     };
     auto on_edge = [&](int r, int cc) { return r == 0 || r == ny - 1 || cc == 0 || cc == nx - 1; };
-    const int lr = tid / TX, lc = tid % TX;                // own square in the tile
-    const int r_own = r0 + lr, c_own = cc0 + lc;
-    const bool own_in = r_own < ny && c_own < nx;
-    const bool own_edge = on_edge(r_own, c_own);
     const int off_own = clampi(r_own, ny) * nx + clampi(c_own, nx);
-    int crs, ccs, drs, dcs;                                // ring squares in sC and sD
-    ring(min(tid, RC - 1), 2, crs, ccs);
+    int drs, dcs;                                          // ring square of the D_env block
     ring(min(tid, RD - 1), 1, drs, dcs);
-    const int rc_r = r0 - 2 + crs, rc_c = cc0 - 2 + ccs;
     const int rd_r = r0 - 1 + drs, rd_c = cc0 - 1 + dcs;
-    const bool cring_in = rc_r >= 0 && rc_r < ny && rc_c >= 0 && rc_c < nx;
-    const bool cring_edge = on_edge(rc_r, rc_c);
-    const bool dring_in = rd_r >= 0 && rd_r < ny && rd_c >= 0 && rd_c < nx;
-    const int off_cring = clampi(rc_r, ny) * nx + clampi(rc_c, nx);
     const int off_dring = clampi(rd_r, ny) * nx + clampi(rd_c, nx);
+    const int pt = min(tid, NP - 1);
+    const int prow = pt / (VC / 2), pcol = 2 * (pt % (VC / 2));
+    const int p_r = r0 - 2 + prow, p_c = cc0 - 2 + pcol;   // the pair's first square
+    const bool pe0 = on_edge(p_r, p_c), pe1 = on_edge(p_r, p_c + 1);
+    // a pair whose second square lies past the row's end is loaded one square
+    // to the left (the first square is then the loaded pair's second)
+    const bool p_last = p_c == nx - 1;
+    const int off_pair = clampi(p_r, ny) * nx + min(max(p_c, 0), nx - 2);
     // one ion's concentrations and D_env at those squares, from clamped
     // in-grid addresses (du: the cluster's D_env of the ion when it is one
-    // value, no loads; NaN when it varies)
-    double tc_own = 0.0, tc_ring = 0.0, td_own = 0.0, td_ring = 0.0;
+    // value, no loads; NaN when it varies). What lies outside the world is
+    // staged from the clamped square and never read.
+    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+    d2 tc = {0.0, 0.0};
+    double td_own = 0.0, td_ring = 0.0;
     auto load_ion = [&](int i, double du) {
         const double* cenv = A.c_env + (size_t)i * P.n_sq + so;
         const double* D = A.D_env + (size_t)i * P.n_sq + so;
-        tc_own = cenv[off_own];
-        tc_ring = cenv[off_cring];
-        if (!(du == du)) {
+        if (tid < NP) tc = *reinterpret_cast<const d2*>(cenv + off_pair);
+        if (DVAR && !(du == du)) {
             td_own = D[off_own];
             td_ring = D[off_dring];
         }
     };
-    if (DIFFUSE && i_lo < i_hi) load_ion(i_lo, A.kcl[et[0]].denv_u[i_lo]);
+    if (DIFFUSE && i_lo < i_hi) load_ion(i_lo, K->denv_u[i_lo]);
     // u last: its loads are the only unconditional ones, so the waits for
-    // them count the same on every path
-    constexpr int NIT = (UR * UC + TY * TX - 1) / (TY * TX);
-    double t[NIT];
+    // them count the same on every path. Pairs of a row (cc0 - UH is even, so
+    // a pair that starts left of the world lies outside it; one that ends past
+    // the batch's last square reads the buffer's padding).
+    static_assert(UC % 2 == 0 && UH % 2 == 0 && TX % 2 == 0, "u is staged in pairs");
+    constexpr int NU = UR * UC / 2;
+    constexpr int NIT = (NU + TY * TX - 1) / (TY * TX);
+    d2 t[NIT];
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int e = min(tid + it * TY * TX, UR * UC - 1);
+        const int e = 2 * min(tid + it * TY * TX, NU - 1);
         const int rr = r0 - UH + e / UC, cc = cc0 - UH + e % UC;
-        t[it] = A.u[so + clampi(rr, ny) * nx + clampi(cc, nx)];
+        t[it] = *reinterpret_cast<const d2*>(A.u + so + clampi(rr, ny) * nx + clampi(cc, nx));
     }
 
+    // FUSE: the square's membrane-flux sums of every moving ion, taken here, all
+    // ions' loads in flight together, while the field's loads are too; each
+    // thread keeps its own in LDS for the ion loop
+    double* s_sum = s_du + BT_MAX_IONS;
+    if (FUSE && live_b != 0) {
+        const unsigned moving = ~still_mem & ((1u << P.n_ions) - 1u);
+        if (A.fsa32) neg_flux_sums(static_cast<const float*>(A.fsa), P.n_mems, moving, fa, fb, s_sum + tid, TY * TX);
+        else neg_flux_sums(static_cast<const double*>(A.fsa), P.n_mems, moving, fa, fb, s_sum + tid, TY * TX);
+    }
     // the gating rates of every (channel, cell) for this step's k_mem_cell.
     // They depend on the cell's Vmem alone, so evaluating them here, one
     // (channel, cell) per thread, replaces one FP64 evaluation per membrane.
@@ -1006,64 +1107,57 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // with the block's first loads); run first, their registers would stay
     // live beside the prefetched loads and cost occupancy.
     auto gating_rates = [&]() {
-        for (int t_it = t_first; t_it >= 0 && t_it < items; t_it += nthr)
-            gate_coef_item(A, P, t_it, (t_it == t_first) ? vm_first : A.vm[t_it % nc]);
+        for (int t_it = rate_first; t_it >= 0 && t_it < items; t_it += rate_stride)
+            gate_coef_item(A, P, t_it, (t_it == rate_first) ? vm_first : A.vm[t_it % nc]);
     };
     if (DIFFUSE && tid < P.n_ions) s_du[tid] = du_mine;
 
     // u with zero padding outside the grid (gaussian_filter mode='constant')
-    {
 #pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int e = tid + it * TY * TX;
-            if (e < UR * UC) {
-                const int rr = r0 - UH + e / UC, cc = cc0 - UH + e % UC;
-                sU[e / UC][e % UC] = (rr >= 0 && rr < ny && cc >= 0 && cc < nx) ? t[it] : 0.0;
+    for (int it = 0; it < NIT; ++it) {
+        const int e = 2 * (tid + it * TY * TX);
+        if (e < UR * UC) {
+            const int rr = r0 - UH + e / UC, cc = cc0 - UH + e % UC;
+            const bool in = rr >= 0 && rr < ny && cc >= 0;
+            sU[e] = (in && cc < nx) ? t[it].x : 0.0;
+            sU[e + 1] = (in && cc + 1 < nx) ? t[it].y : 0.0;
+        }
+    }
+    lds_barrier();
+    // axis-0 pass (scipy correlate1d: centre tap, then pairs outermost first),
+    // two rows a thread: ten LDS reads for two squares instead of nine for one
+    for (int e = tid; e < (VR / 2) * UC; e += TY * TX) {
+        const double* x = sU + 2 * (e / UC) * UC + e % UC;      // row -4 of the first square
+        double w[10];
+#pragma unroll
+        for (int q = 0; q < 10; ++q) w[q] = x[q * UC];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            double o = w[4 + h] * P.gw[0];
+#pragma unroll
+            for (int q = 4; q >= 1; --q) o = o + (w[4 + h - q] + w[4 + h + q]) * P.gw[q];
+            sT[(2 * (e / UC) + h) * UC + e % UC] = o;
+        }
+    }
+    lds_barrier();
+    // axis-1 pass -> v_env (+ Phi_b, ion_current.py:104), two columns a thread
+    if (tid < VR * (VC / 2)) {
+        const int vr = tid / (VC / 2), vc = 2 * (tid % (VC / 2));
+        const double* x = sT + vr * UC + vc;                    // column -4 of the first square
+        double w[10];
+#pragma unroll
+        for (int q = 0; q < 10; ++q) w[q] = x[q];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            double o = w[4 + h] * P.gw[0];
+#pragma unroll
+            for (int q = 4; q >= 1; --q) o = o + (w[4 + h - q] + w[4 + h + q]) * P.gw[q];
+            if (K->phib) {
+                const int r = r0 - 2 + vr, cc = cc0 - 2 + vc + h;
+                if (r >= 0 && r < ny && cc >= 0 && cc < nx) o = o + A.Phi_b[so + r * nx + cc];
             }
+            sV[vr * VC + vc + h] = o;
         }
-    }
-    lds_barrier();
-    // axis-0 pass (scipy correlate1d: centre tap, then pairs outermost first)
-    for (int e = tid; e < TR * UC; e += TY * TX) {
-        const int lr = e / UC + 4, lc = e % UC;          // row in sU
-        double o = sU[lr][lc] * P.gw[0];
-#pragma unroll
-        for (int q = 4; q >= 1; --q) o = o + (sU[lr - q][lc] + sU[lr + q][lc]) * P.gw[q];
-        sT[e / UC][lc] = o;
-    }
-    lds_barrier();
-    // axis-1 pass -> v_env (+ Phi_b, ion_current.py:104)
-    for (int e = tid; e < VR * VC; e += TY * TX) {
-        const int lr = e / VC, lc = e % VC + 4;          // column in sT
-        double o = sT[lr][lc] * P.gw[0];
-#pragma unroll
-        for (int q = 4; q >= 1; --q) o = o + (sT[lr][lc - q] + sT[lr][lc + q]) * P.gw[q];
-        if (K.phib) {
-            const int r = r0 - 2 + lr, cc = cc0 - 2 + e % VC;
-            if (r >= 0 && r < ny && cc >= 0 && cc < nx) o = o + A.Phi_b[so + r * nx + cc];
-        }
-        sV[lr][e % VC] = o;
-    }
-    lds_barrier();
-    // E = -grad(screen * v_env), one-sided at the world edges (finitediff.py:1236-1266)
-    for (int e = tid; e < ER * EC; e += TY * TX) {
-        const int er = e / EC, ec = e % EC;
-        const int r = r0 - 1 + er, cc = cc0 - 1 + ec;
-        double ex = 0.0, ey = 0.0;
-        if (r >= 0 && r < ny && cc >= 0 && cc < nx) {
-            const int vr = er + 1, vc = ec + 1;         // (r, cc) in sV
-            double gx, gy;
-            if (cc == 0) gx = per_dl((K.screen * sV[vr][vc + 1] - K.screen * sV[vr][vc]));
-            else if (cc == nx - 1) gx = per_dl((K.screen * sV[vr][vc] - K.screen * sV[vr][vc - 1]));
-            else gx = per_d2(-(K.screen * sV[vr][vc - 1] - K.screen * sV[vr][vc + 1]));
-            if (r == 0) gy = per_dl((K.screen * sV[vr + 1][vc] - K.screen * sV[vr][vc]));
-            else if (r == ny - 1) gy = per_dl((K.screen * sV[vr][vc] - K.screen * sV[vr - 1][vc]));
-            else gy = per_d2(-(K.screen * sV[vr - 1][vc] - K.screen * sV[vr + 1][vc]));
-            ex = -gx;
-            ey = -gy;
-        }
-        sEx[er][ec] = ex;
-        sEy[er][ec] = ey;
     }
     lds_barrier();
     // a halted run writes nothing (every thread read the same flag)
@@ -1071,171 +1165,151 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     if (FUSE && A.count_step && tile_id == 0 && ion_id == 0 && tid == 0)
         for (int g = 0; g < BT_MAX_STREAMS; ++g)
             if (A.ctr_mask & (1u << g)) A.step_ctr[g] = A.step_ctr[g] + 1;
+    const int o = (lr + 2) * VC + lc + 2;                       // own square in sV and the staged ions
+    // grad(screen * v_env) along one axis (E = -grad, one-sided at the world
+    // edges), between the squares lo and hi (LDS offsets) with the factor f
+    auto vgrad = [&](int lo, int hi, double f) { return (screen * sV[o + hi] - screen * sV[o + lo]) * f; };
     if (!DIFFUSE) {
-        const int r = r0 + tid / TX, cc = cc0 + tid % TX;
-        if (r < ny && cc < nx) {
-            A.v_env[so + r * nx + cc] = sV[tid / TX + 2][tid % TX + 2];
-            A.Ex[so + r * nx + cc] = sEx[tid / TX + 1][tid % TX + 1];
-            A.Ey[so + r * nx + cc] = sEy[tid / TX + 1][tid % TX + 1];
+        if (own_in) {
+            const int xl = (c_own > 0) ? -1 : 0, xh = (c_own < nx - 1) ? 1 : 0;
+            const int yl = (r_own > 0) ? -VC : 0, yh = (r_own < ny - 1) ? VC : 0;
+            A.v_env[k_own] = sV[o];
+            A.Ex[k_own] = -vgrad(xl, xh, (xl && xh) ? rd2 : rdl);
+            A.Ey[k_own] = -vgrad(yl, yh, (yl && yh) ? rd2 : rdl);
         }
         return;
     }
 
-    double rho = 0.0;               // FUSE: the square's charge over the ions, in ion order
-    for (int i = i_lo; i < i_hi; ++i) {
-        const double cb = P.c_bound[i];
-        const double zi = P.zq[i];
-        const double zq_kt = (zi * P.q) / P.kbT;        // alpha = D * zq_kt
-        lds_barrier();
-        // concentrations of ion i (loaded one ion ahead) with the world
-        // boundary reset to c_env_bound (Q3), zero outside the grid
-        sC[lr + 2][lc + 2] = own_in ? (own_edge ? cb : tc_own) : 0.0;
-        if (tid < RC) sC[crs][ccs] = cring_in ? (cring_edge ? cb : tc_ring) : 0.0;
-        // D_env zero over the cluster (block-uniform): the Nernst-Planck flux
-        // is a signed zero everywhere and the update keeps the
-        // (boundary-reset) concentrations, so its stages are skipped. D_env
-        // one value over the cluster (block-uniform) is that value, with no
-        // staging; else it is staged on tile +- 1, zero outside the grid.
-        const double du_i = s_du[i];
-        const bool still = (du_i == 0.0);
-        const bool duni = (du_i == du_i);
-        // FUSE: this square's first membrane fluxes of ion i (none for a still
-        // ion, whose rows are zeros, or a square without membranes)
-        double pf[(FUSE && FUSE_PF > 0) ? FUSE_PF : 1];
-        const bool fsum = FUSE && FUSE_PF > 0 && live_b != 0 && fa < fb && !((K.still_mem >> i) & 1u);
-        if (FUSE && fsum) {
-            const size_t row = (size_t)i * P.n_mems;
-#pragma unroll
-            for (int u = 0; u < FUSE_PF; ++u) {
-                const int q = min(fa + u, fb - 1);
-                pf[u] = A.fsa32 ? (double)static_cast<const float*>(A.fsa)[row + q]
-                                : static_cast<const double*>(A.fsa)[row + q];
-            }
-        }
-        if (!still && !duni) {
-            sD[lr + 1][lc + 1] = own_in ? td_own : 0.0;
-            if (tid < RD) sD[drs][dcs] = dring_in ? td_ring : 0.0;
-        }
-        // the next ion's loads, in flight through this ion's flux stages
-        if (i + 1 < i_hi) load_ion(i + 1, s_du[i + 1]);
-        lds_barrier();
-        if (!still) {
-        // Nernst-Planck fluxes (sim_toolbox.py:409-411, gv = -E, u = 0, mu = 0)
-        // at the square (r, cc), which is (sr, sc) in sC and (er, ec) in sD, sEx and sEy
-        auto np_flux = [&](int r, int cc, int sr, int sc, int er, int ec, double& fx, double& fy, bool want_x,
-                           bool want_y) {
-            const double Dv = duni ? du_i : sD[er][ec];
-            const double alpha = Dv * zq_kt;
-            if (want_x) {
-                double g;
-                if (cc == 0) g = per_dl((sC[sr][sc + 1] - sC[sr][sc]));
-                else if (cc == nx - 1) g = per_dl((sC[sr][sc] - sC[sr][sc - 1]));
-                else g = per_d2(-(sC[sr][sc - 1] - sC[sr][sc + 1]));
-                fx = (-Dv) * g - (alpha * (-sEx[er][ec])) * sC[sr][sc];
-            }
-            if (want_y) {
-                double g;
-                if (r == 0) g = per_dl((sC[sr + 1][sc] - sC[sr][sc]));
-                else if (r == ny - 1) g = per_dl((sC[sr][sc] - sC[sr - 1][sc]));
-                else g = per_d2(-(sC[sr - 1][sc] - sC[sr + 1][sc]));
-                fy = (-Dv) * g - (alpha * (-sEy[er][ec])) * sC[sr][sc];
+    // The ion loop. EDGE: some square of the tile lies within two of the
+    // world's edge, where the stencils' offsets and factors vary by square;
+    // elsewhere they are constants (folded into the LDS instructions).
+    auto ions = [&](auto edge_c) {
+        constexpr bool EDGE = decltype(edge_c)::value;
+        // (an axis' offsets and factors are rebuilt for each use, behind an
+        // empty asm that keeps the compiler from holding them between the
+        // ions: held, they cost a quarter of the occupancy)
+        auto axis = [&](int at, int n) {
+            if constexpr (EDGE) {
+                int c = min(at, n - 1);
+                asm volatile("" : "+v"(c));
+                return env_axis(c, n, rdl, rd2);
+            } else {
+                return env_axis_inner(rd2);
             }
         };
+        double gxL, gxR, gyL, gyR;
         {
-            // both fluxes at the thread's own square
-            double fx = 0.0, fy = 0.0;
-            if (own_in) np_flux(r_own, c_own, lr + 2, lc + 2, lr + 1, lc + 1, fx, fy, true, true);
-            sFx[lr][lc + 1] = fx;
-            sFy[lr + 1][lc] = fy;
+            const EnvAxis a = axis(c_own, nx);
+            gxL = vgrad(a.Llo, a.Lhi, a.fL);
+            gxR = vgrad(a.Rlo, a.Rhi, a.fR);
         }
-        if (tid < 2 * TY + 2 * TX) {
-            // the halo the divergence also reads, by the first wavefront: fx
-            // in the columns left and right of the tile, fy in the rows above
-            // and below it
-            const bool xh = tid < 2 * TY;
-            const int t = xh ? tid : tid - 2 * TY;
-            const int a = t % TX, side = (t / TX) ? TX + 1 : 0;     // 16 squares per side
-            const int hr = xh ? a : side, hc = xh ? side : a;       // in sFy rows / sFx columns
-            const int r = xh ? r0 + a : r0 - 1 + side, cc = xh ? cc0 - 1 + side : cc0 + a;
-            double f = 0.0;
-            if (r >= 0 && r < ny && cc >= 0 && cc < nx) {
-                double fx = 0.0, fy = 0.0;
-                if (xh) np_flux(r, cc, a + 2, side + 1, a + 1, side, fx, fy, true, false);
-                else np_flux(r, cc, side + 1, a + 2, side, a + 1, fx, fy, false, true);
-                f = xh ? fx : fy;
+        {
+            const EnvAxis a = axis(r_own, ny);
+            gyL = vgrad(a.Llo * VC, a.Lhi * VC, a.fL);
+            gyR = vgrad(a.Rlo * VC, a.Rhi * VC, a.fR);
+        }
+        double rho = 0.0;               // FUSE: the square's charge over the ions, in ion order
+        for (int i = i_lo; i < i_hi; ++i) {
+            const double cb = P.c_bound[i];
+            const double zi = P.zq[i];
+            const double zq_kt = (zi * P.q) / P.kbT;        // alpha = D * zq_kt
+            double* sC = lds + ((i - i_lo) & 1) * (VR * VC);
+            double* sD = lds + 2 * VR * VC + ((i - i_lo) & 1) * (ER * EC);
+            // concentrations of ion i (loaded one ion ahead) with the world
+            // boundary reset to c_env_bound (Q3)
+            if (tid < NP) {
+                sC[2 * tid] = pe0 ? cb : (p_last ? tc.y : tc.x);
+                sC[2 * tid + 1] = pe1 ? cb : tc.y;
             }
-            if (xh) sFx[hr][hc] = f;
-            else sFy[hr][hc] = f;
-        }
-        lds_barrier();
-        }
-        // fd.divergence(-fx, -fy) with the sign-flipped one-sided edges (Q4), Euler step
-        {
-            const int lr = tid / TX, lc = tid % TX;
-            const int r = r0 + lr, cc = cc0 + lc;
-            if (r < ny && cc < nx) {
-                double cn = sC[lr + 2][lc + 2];
-                if (!still) {
-                    double gx, gy;
-                    if (cc == 0) gx = per_dl(((-sFx[lr][lc + 1]) - (-sFx[lr][lc + 2])));
-                    else if (cc == nx - 1) gx = per_dl(((-sFx[lr][lc]) - (-sFx[lr][lc + 1])));
-                    else gx = per_d2(-((-sFx[lr][lc]) - (-sFx[lr][lc + 2])));
-                    if (r == 0) gy = per_dl(-((-sFy[lr + 2][lc]) - (-sFy[lr + 1][lc])));
-                    else if (r == ny - 1) gy = per_dl(-((-sFy[lr + 1][lc]) - (-sFy[lr][lc])));
-                    else gy = per_d2(-((-sFy[lr][lc]) - (-sFy[lr + 2][lc])));
-                    const double div = gx + gy;
-                    cn = cn + div * P.dt;
+            // D_env zero over the cluster (block-uniform): the Nernst-Planck flux
+            // is a signed zero everywhere and the update keeps the
+            // (boundary-reset) concentrations, so its stages are skipped. D_env
+            // one value over the cluster (block-uniform) is that value, with no
+            // staging; else it is staged on tile +- 1.
+            const double du_i = s_du[i];
+            const bool still = (du_i == 0.0);
+            const bool duni = !DVAR || (du_i == du_i);
+            const bool mstill = (still_mem >> i) & 1u;
+            const int od = (lr + 1) * EC + lc + 1;
+            if (!still && !duni) {
+                sD[od] = td_own;
+                if (tid < RD) sD[drs * EC + dcs] = td_ring;
+            }
+            // the next ion's loads, in flight through this ion's flux stages
+            if (i + 1 < i_hi) load_ion(i + 1, s_du[i + 1]);
+            lds_barrier();
+            if (!own_in) continue;
+            double cn = sC[o], ofx = 0.0, ofy = 0.0;
+            if (!still) {
+                // Nernst-Planck flux (sim_toolbox.py:409-411, gv = -E, u = 0, mu = 0)
+                // at LDS offset s: -D grad c - alpha (-E) c, grad c between lo and hi
+                auto np_flux = [&](int s, int sd, int lo, int hi, double f, double ge) {
+                    const double Dv = duni ? du_i : sD[od + sd];
+                    const double g = (sC[o + hi] - sC[o + lo]) * f;
+                    return (-Dv) * g - ((Dv * zq_kt) * ge) * sC[o + s];
+                };
+                // fd.divergence(-fx, -fy), Euler step
+                double div;
+                {
+                    const EnvAxis a = axis(c_own, nx);
+                    const double fL = np_flux(a.L, a.L, a.Llo, a.Lhi, a.fL, gxL);
+                    const double fR = np_flux(a.R, a.R, a.Rlo, a.Rhi, a.fR, gxR);
+                    div = (fL - fR) * a.fdiv;
                 }
-                const size_t e = (size_t)i * P.n_sq + so + r * nx + cc;
-                unsigned lv = live_b;
-                asm volatile("" : "+v"(lv));
-                if (FUSE) {
-                    // the exchange of k_env_exchange for this square and ion:
-                    // a still ion's membrane fluxes are zeros, whose sum
-                    // would add a signed zero
-                    if (lv != 0 && !((K.still_mem >> i) & 1u)) {
-                        double S = 0.0;
-                        if (fsum) {
-#pragma unroll
-                            for (int u = 0; u < FUSE_PF; ++u)
-                                if (fa + u < fb) S = S + (-pf[u]);
-                            if (fb > fa + FUSE_PF)
-                                S = neg_flux_sum<FUSE_W>(A.fsa, A.fsa32, (size_t)i * P.n_mems, fa + FUSE_PF, fb, S);
-                        } else {
-                            S = neg_flux_sum<FUSE_W>(A.fsa, A.fsa32, (size_t)i * P.n_mems, fa, fb);
-                        }
-                        cn = cn + (S / K.env_vol) * P.dt;
-                    }
-                    A.c_env_out[e] = cn;
-                    rho = (i == 0) ? P.zF[0] * cn : rho + P.zF[i] * cn;
-                } else if (lv != 0) {
-                    A.c_mid[e] = cn;
-                } else {
-                    A.c_env_out[e] = cn;
+                if (EDGE) asm volatile("" : "+v"(div));
+                {
+                    const EnvAxis a = axis(r_own, ny);
+                    const double fL = np_flux(a.L * VC, a.L * EC, a.Llo * VC, a.Lhi * VC, a.fL, gyL);
+                    const double fR = np_flux(a.R * VC, a.R * EC, a.Rlo * VC, a.Rhi * VC, a.fR, gyR);
+                    div = div + (fL - fR) * a.fdiv;
                 }
-                if (A.obs_fx) {
-                    A.obs_fx[(size_t)i * P.n_sq + so + r * nx + cc] = still ? 0.0 : sFx[lr][lc + 1];
-                    A.obs_fy[(size_t)i * P.n_sq + so + r * nx + cc] = still ? 0.0 : sFy[lr + 1][lc];
+                cn = cn + div * P.dt;
+                if (OBS) {              // the observed step: the fluxes at the square itself
+                    const int xl = (c_own > 0) ? -1 : 0, xh = (c_own < nx - 1) ? 1 : 0;
+                    const int yl = (r_own > 0) ? -VC : 0, yh = (r_own < ny - 1) ? VC : 0;
+                    const double fx = (xl && xh) ? rd2 : rdl, fy = (yl && yh) ? rd2 : rdl;
+                    ofx = np_flux(0, 0, xl, xh, fx, vgrad(xl, xh, fx));
+                    ofy = np_flux(0, 0, yl, yh, fy, vgrad(yl, yh, fy));
                 }
             }
+            const size_t e = (size_t)i * P.n_sq + k_own;
+            unsigned lv = live_b;
+            asm volatile("" : "+v"(lv));
+            if (FUSE) {
+                // the exchange of k_env_exchange for this square and ion:
+                // a still ion's membrane fluxes are zeros, whose sum
+                // would add a signed zero
+                if (lv != 0 && !mstill) cn = cn + (s_sum[i * (TY * TX) + tid] / K->env_vol) * P.dt;
+                A.c_env_out[e] = cn;
+                rho = (i == 0) ? P.zF[0] * cn : rho + P.zF[i] * cn;
+            } else if (lv != 0) {
+                A.c_mid[e] = cn;
+            } else {
+                A.c_env_out[e] = cn;
+            }
+            if (OBS) {
+                A.obs_fx[e] = ofx;
+                A.obs_fy[e] = ofy;
+            }
         }
-    }
-    if (FUSE) {
-        const int r = r0 + tid / TX, cc = cc0 + tid % TX;
-        if (r < ny && cc < nx && live_b != 0)
-            A.u_out[so + r * nx + cc] = hm ? ((rho * K.surf_scale) / K.mean_sa) / K.kee : 0.0;
-    }
+        if (FUSE && own_in && live_b != 0)
+            A.u_out[k_own] = (live_b & SQ_HAS_MEM) ? ((rho * K->surf_scale) / K->mean_sa) / K->kee : 0.0;
+    };
+    const bool inner = r0 >= 2 && r0 + TY <= ny - 2 && cc0 >= 2 && cc0 + TX <= nx - 2;
+    if (inner) ions(std::false_type{});
+    else ions(std::true_type{});
     if (RATES) gating_rates();
 }
 
-template <bool DIFFUSE, bool RATES, bool FUSE = false>
+template <bool DIFFUSE, bool RATES, bool FUSE, bool DVAR, bool OBS>
 __global__ void __launch_bounds__(TY * TX)
 k_env_field(FieldArgs A, KParams P) {
-    __shared__ double lds[ENV_LDS];
+    // ENV_LDS doubles, and with the exchange (FUSE) n_ions for each thread
+    extern __shared__ double lds[];
     // (tile, ion group) from the XCD-chunked linear block index, tiles fastest
     const int lin = xcd_chunk(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int tile_id = lin % gridDim.x, ion_id = lin / gridDim.x;
-    env_field_tile<DIFFUSE, RATES, FUSE>(A, P, tile_id, ion_id, gridDim.y, lds,
+    env_field_tile<DIFFUSE, RATES, FUSE, DVAR, OBS>(A, P, tile_id, ion_id, gridDim.y, lds,
                                    (blockIdx.y * gridDim.x + blockIdx.x) * (TY * TX) + threadIdx.x,
                                    gridDim.x * gridDim.y * (TY * TX));
 }
@@ -2001,7 +2075,7 @@ k_step_persistent(PersistArgs PA, KParams P) {
         if (!s_stop) {
             for (int it = blockIdx.x; it < n_env_items; it += nb) {
                 const int item = (nb % N_XCD == 0) ? xcd_chunk(it, n_env_items) : it;
-                env_field_tile<true, false>(FA, P, item % PA.n_env_tiles, item / PA.n_env_tiles, PA.n_groups, lds,
+                env_field_tile<true, false, false, true, false>(FA, P, item % PA.n_env_tiles, item / PA.n_env_tiles, PA.n_groups, lds,
                                             -1, 0, false);
                 lds_barrier();
             }
@@ -2065,7 +2139,7 @@ struct bt_ctx {
     double* rates = nullptr;  // [n_chan][4][n_cells] gating rates of the current step
     double* c_env_b = nullptr;           // env state of odd steps
     int32_t* sq_live = nullptr;          // squares the exchange updates, ascending
-    uint8_t* live_flag = nullptr;        // per square: 1 if in sq_live
+    uint8_t* live_flag = nullptr;        // per square: SQ_LIVE if in sq_live, SQ_HAS_MEM
     int n_live = 0;
     unsigned* flags = nullptr; unsigned long long* bad_step = nullptr; long long* step_ctr = nullptr;
     // step graphs per stream group g: one pair of steps, and tune.graph_pairs pairs
@@ -2078,6 +2152,7 @@ struct bt_ctx {
     std::vector<int> cl_tile0, cl_env0, cl_live0;
     std::vector<int> cl_mem_lo, cl_mem_hi;   // each cluster's membrane range
     bool any_phib = false;                   // some cluster has an applied boundary voltage
+    bool denv_varies = false;                // some ion's D_env varies over some cluster
     std::vector<long long> cl_cell0;
     hipStream_t gstream[BT_MAX_STREAMS] = {};
     hipEvent_t ev_fork = nullptr;
@@ -2280,14 +2355,26 @@ static void launch_field_args(bt_ctx* c, bool diffuse, const FieldArgs& f, hipSt
     // looping over the ions; field only: one block per tile
     const int ipb = c->tune.env_ions_per_block;
     dim3 grid(ne > 0 ? ne : c->n_env_tiles, diffuse ? (c->prm.n_ions + ipb - 1) / ipb : 1);
-    if (diffuse && f.u_out)
-        hipLaunchKernelGGL((k_env_field<true, false, true>), grid, dim3(TY * TX), 0, st, f, c->kp);
-    else if (diffuse && f.rates)
-        hipLaunchKernelGGL((k_env_field<true, true>), grid, dim3(TY * TX), 0, st, f, c->kp);
-    else if (diffuse)
-        hipLaunchKernelGGL((k_env_field<true, false>), grid, dim3(TY * TX), 0, st, f, c->kp);
+    auto launch = [&](auto rates, auto fuse, auto dvar, auto obs) {
+        const size_t lds = (ENV_LDS + (fuse.value ? (size_t)c->prm.n_ions * TY * TX : 0)) * sizeof(double);
+        hipLaunchKernelGGL((k_env_field<true, rates.value, fuse.value, dvar.value, obs.value>), grid, dim3(TY * TX), lds,
+                           st, f, c->kp);
+    };
+    const std::true_type yes{};
+    const std::false_type no{};
+    if (!diffuse)
+        hipLaunchKernelGGL((k_env_field<false, false, false, false, false>), grid, dim3(TY * TX),
+                           ENV_LDS * sizeof(double), st, f, c->kp);
+    else if (f.u_out && f.obs_fx)
+        c->denv_varies ? launch(no, yes, yes, yes) : launch(no, yes, no, yes);
+    else if (f.u_out)
+        c->denv_varies ? launch(no, yes, yes, no) : launch(no, yes, no, no);
+    else if (f.obs_fx)       // (RATES without channels has no items)
+        launch(yes, no, yes, yes);
+    else if (f.rates)
+        c->denv_varies ? launch(yes, no, yes, no) : launch(yes, no, no, no);
     else
-        hipLaunchKernelGGL((k_env_field<false, false>), grid, dim3(TY * TX), 0, st, f, c->kp);
+        c->denv_varies ? launch(no, no, yes, no) : launch(no, no, no, no);
 }
 
 static void launch_field(bt_ctx* c, bool diffuse, const bt_obs* ob = nullptr, const double* vm = nullptr,
@@ -2335,7 +2422,6 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
         a.field.u = parity ? c->u_b : c->u;
         a.field.u_out = parity ? c->u : c->u_b;
         a.field.sq_ptr = B.sq_ptr;
-        a.field.has_mem = B.sq_has_mem;
         a.field.fsa = c->fsa;
         a.field.fsa32 = a.ex.fsa32;
         a.field.step_ctr = c->step_ctr;
@@ -2712,6 +2798,8 @@ static int derive_uniform(bt_ctx* c) {
     if (e != hipSuccess)
         return set_err(c, BT_EHIP, std::string("reading Dm, gjopen, D_env, Phi_b: ") + hipGetErrorString(e));
     c->any_phib = false;
+    const bool varied = c->denv_varies;
+    c->denv_varies = false;
     for (int q = 0; q < nq; ++q) {
         KCluster& K = c->kcl_host[q];
         const int lo = c->cl_mem_lo[q], hi = c->cl_mem_hi[q];
@@ -2739,6 +2827,7 @@ static int derive_uniform(bt_ctx* c) {
             bool same = true;
             for (size_t k = k0; k < k1 && same; ++k) same = (d[k] == d[k0]);
             K.denv_u[i] = same ? d[k0] : NAN;
+            c->denv_varies = c->denv_varies || !same;
         }
         K.phib = 0;
         for (size_t k = k0; k < k1 && !pb.empty() && !K.phib; ++k) K.phib = (pb[k] != 0.0);
@@ -2748,6 +2837,8 @@ static int derive_uniform(bt_ctx* c) {
                                          "supported (their gating rates are per cell)");
         c->any_phib = c->any_phib || K.phib;
     }
+    // the captured step graphs hold the env kernel of the other kind
+    if (c->denv_varies != varied) drop_graphs(c);
     return BT_OK;
 }
 
@@ -2815,7 +2906,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     for (size_t k = 0; k < NS; ++k) {
         if (sp[k + 1] > sp[k] || hm[k]) {
             sq_live.push_back((int32_t)k);
-            live_flag[k] = 1;
+            live_flag[k] = SQ_LIVE | (hm[k] ? SQ_HAS_MEM : 0);
         }
     }
 
@@ -2887,11 +2978,11 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     alloc((void**)&c->c_lag_b, ni * nc * 8);
     alloc((void**)&c->vm_b, nc * 8);
     alloc((void**)&c->c_mid, ni * ns * 8);
-    alloc((void**)&c->fsa, ni * nm * 8);
+    alloc((void**)&c->fsa, (ni * nm + FSA_PAD) * 8);
     alloc((void**)&c->fch, (p->n_chan > 0 ? (size_t)p->n_chan : 1) * nm * 8);
     alloc((void**)&c->rates, (p->n_chan > 0 ? (size_t)p->n_chan : 1) * 4 * nc * 8);
-    alloc((void**)&c->u, ns * 8);
-    alloc((void**)&c->u_b, ns * 8);
+    alloc((void**)&c->u, (ns + 1) * 8);          // (the env kernel reads u in pairs)
+    alloc((void**)&c->u_b, (ns + 1) * 8);
     alloc((void**)&c->flags, 256);
     alloc((void**)&c->bad_step, 256);
     alloc((void**)&c->step_ctr, 256);
@@ -2923,7 +3014,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     if (e == hipSuccess) e = hipMemsetAsync(c->bar, 0, 256, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->u, 0, ns * 8, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->u_b, 0, ns * 8, c->stream);    // u of squares without membranes
-    if (e == hipSuccess) e = hipMemsetAsync(c->fsa, 0, ni * nm * 8, c->stream);   // still rows stay zero
+    if (e == hipSuccess) e = hipMemsetAsync(c->fsa, 0, (ni * nm + FSA_PAD) * 8, c->stream);   // still rows stay zero
     if (e == hipSuccess)
         e = hipMemsetAsync(c->rates, 0, (p->n_chan > 0 ? (size_t)p->n_chan : 1) * 4 * nc * 8, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
