@@ -76,6 +76,8 @@ struct KParams {
     int chan_kind[BT_MAX_CHAN];
     int chan_ion[BT_MAX_CHAN];
     int ion_chan[BT_MAX_IONS];      // channel acting on each ion, -1 if none
+    unsigned ion_chan_pack;         // the same, four bits per ion, 15 if none
+    unsigned chan_ion_pack;         // chan_ion, four bits per channel
     double chan_max_dm[BT_MAX_CHAN];
     double chan_dt;
     double zplus[BT_MAX_IONS];      // z + 1e-25          (electroflux zc += nonce)
@@ -430,9 +432,29 @@ __device__ __forceinline__ void gate_rates(int kind, double V, double& mInf, dou
 // ---------------------------------------------------------------------------
 // k_mem_cell: membrane fluxes + per-cell update + Vmem
 // ---------------------------------------------------------------------------
+// What k_mem_cell reads of a tile, one scalar load: its first cell and
+// membrane, its cells and membranes, its cluster; `starts` has a bit for every
+// membrane but the tile's first that is the first of its cell, moved down by
+// one, so the number of its bits below a lane is the cell of that lane's
+// membrane within the tile; `inv_nc` = floor(2^16 / cells) + 1, whose product
+// with a t < 256 over 2^16 is t / cells (cells <= 32).
+struct TileRec {
+    int c0, m0, n_cells, n_mems, cluster, inv_nc;
+    unsigned long long starts;
+};
+static_assert(sizeof(TileRec) == 32, "one 32-byte scalar load");
+
+// What k_mem_cell reads of a membrane, one 16-byte load: its gap-junction
+// partner's cell (the sign bit set where the membrane is its own partner: no
+// gap junction), its square, its position in the square-sorted order, and its
+// partner's square (the partner's Phi_b).
+struct MemRec {
+    int nn_cell, sq, pos, nn_sq;
+};
+constexpr int MREC_BND = (int)(1u << 31);
+
 struct MemCellArgs {
-    const int32_t* mem_ptr; const int32_t* mem_cell; const int32_t* nn_mem; const int32_t* nn_cell;
-    const int32_t* mem_sq; const int32_t* mem_pos; const int32_t* tile_ptr; const int32_t* tile_cluster;
+    const TileRec* tiles; const MemRec* mrec;
     const KCluster* kcl;
     const double* mem_sa; const double* gjopen; const double* cell_vol; const double* diviterm; const double* Dm;
     const double* c_env;      // pre-diffusion env (membrane + NaK gathers, Q2)
@@ -449,16 +471,25 @@ struct MemCellArgs {
     // observed step only (NULL otherwise): raw fluxes in membrane order
     double* obs_fm; double* obs_fgj; double* obs_fch; double* obs_rate;
     const double* Phi_b = nullptr;   // applied boundary voltage per square (clusters with phib)
+    int chan_nc = 0;                 // cells of the largest tile: the row length of MemLds::chv
 };
 
-// LDS of one k_mem_cell block, shared by its wavefronts
+// LDS of one k_mem_cell tile, shared by its wavefronts. The lagged
+// concentrations and Vmem of the tile's cells (staged once, then read by their
+// membranes) take the rows their ion's fluxes go to: with one wavefront per
+// tile the lanes read them before any lane writes the row; with two, which may
+// read each other's ions (the Na/K pump), they have rows of their own.
 struct MemLds {
-    double (*mem)[TMB];       // [NI] membrane flux * mem_sa, membrane order
+    double (*mem)[TMB];       // [NI] membrane flux * mem_sa, membrane order; then the cells' new concentrations
     double (*gj)[TMB];        // [NI] -GJ flux * mem_sa
-    double (*ch)[TMB];        // [BT_MAX_CHAN] channel flux * mem_sa
-    double (*c2)[TMB];        // [NI] updated cell concentrations (WG > 1)
+    double (*ch)[TMB];        // [n_chan] channel flux * mem_sa
+    double* chv;              // [n_chan][CHV][chan_nc] per cell: gate coefficients, modulator, concentration
+    double (*lag)[TMB];       // [NI] lagged concentration per cell (WG == 1: mem)
+    double* v;                // Vmem per cell (WG == 1: gj[0])
+    int* start;               // [cells + 1] first membrane of each cell, within the tile
     int* bad;
 };
+constexpr int CHV = 6;        // a_m, b_m, a_h, b_h, modulator, cell concentration
 
 // Synchronisation of the lanes that share a tile's LDS: the block (WSYNC
 // false: the tile's one or two wavefronts are the block; an LDS-only barrier,
@@ -476,89 +507,125 @@ __device__ __forceinline__ void tile_sync() {
     }
 }
 
-// The work of wavefront W of a k_mem_cell block. W is a template argument so
+// The work of wavefront W of a k_mem_cell tile. W is a template argument so
 // that every ion index below is a compile-time constant (the per-ion kernel
 // parameters then load once, up front).
+//
+// What bounds it is the vector-memory address unit: about 16 cycles for every
+// wavefront-wide gather, whatever it hits (measured 79 % busy with 36 loads and
+// 15 stores per tile). So whatever is per cell is loaded once per cell, a lane
+// per (ion, cell) (one load for all ions of a tile of ten cells, where a load
+// per membrane and ion took NI), handed to the membranes through LDS, and the
+// cells' new state is summed and stored by the same lanes; a membrane's indices
+// are one 16-byte record, and the Na/K pump shares its ions' gathers: 23 vector
+// accesses a tile where there were 51 (five ions, no channels). 53k cells on the
+// FP32-flux path 13.8 -> 11.4 us; 23k cells with two channels, two wavefronts a
+// tile, 15.2 -> 13.5 us; 105k cells with three channels 51.4 -> 50.2 us.
 template <int NI, typename FT, int WG, int W, bool OBS, bool WSYNC = false>
 __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParams& P, int tile, const MemLds& L) {
     constexpr int NS = (NI + WG - 1) / WG;             // ion slots per wavefront
     constexpr int NQ = (BT_MAX_CHAN + WG - 1) / WG;    // channel slots per wavefront
-    const int c0 = A.tile_ptr[tile];
-    const int c1 = A.tile_ptr[tile + 1];
-    const int m0 = A.mem_ptr[c0];
-    const int m1 = A.mem_ptr[c1];
+    constexpr int NT = TMB * WG;                       // lanes of the tile
+    constexpr int NPASS = (BT_TILE_CELLS * NI + NT - 1) / NT;   // (ion, cell) items per lane, at most
+    const TileRec T = A.tiles[tile];
+    const int c0 = T.c0, m0 = T.m0, nc = T.n_cells;
     const int j = threadIdx.x % TMB;
+    const int jt = W * TMB + j;
     const int m = m0 + j;
     const int M = P.n_mems, C = P.n_cells, G2 = P.n_sq;
-    const KCluster* KC = A.kcl + A.tile_cluster[tile];
+    const KCluster* KC = A.kcl + T.cluster;
     const double nak_coef = KC->nak_coef;
     const double gjo_u = KC->gjo_u;
     const unsigned still_mem = KC->still_mem;
-    if (W == 0 && j == 0) *L.bad = 0;
+    if (W == 0 && j == 0) {
+        *L.bad = 0;
+        L.start[nc] = T.n_mems;
+    }
+    const bool own_mem = j < T.n_mems;
+    // the membrane's record first: its gathers wait for it
+    MemRec R{0, 0, 0, 0};
+    double sa = 0.0;
+    if (own_mem) {
+        R = A.mrec[m];
+        sa = A.mem_sa[m];
+    }
+    // the tile's cells: lane t takes the (ion, cell) item t, t + NT, ...
+    const int n_items = NI * nc;
+    auto item = [&](int p, int& i, int& c) {
+        const int t = jt + p * NT;
+        i = (t * T.inv_nc) >> 16;
+        c = t - i * nc;
+        return t < n_items;
+    };
+#pragma unroll
+    for (int p = 0; p < NPASS; ++p) {
+        if (p * NT >= n_items) break;
+        int i, c;
+        if (item(p, i, c)) L.lag[i][c] = A.c_lag_in[(size_t)i * C + c0 + c];
+    }
+    if (W == WG - 1 && j < nc) L.v[j] = A.vm_in[c0 + j];
+    const int n_chan = P.n_chan;
+    if (n_chan > 0) {
+        // per (channel, cell): the update coefficients of its gates (from
+        // k_env_field), its modulator and its ion's concentration
+        for (int t = jt; t < n_chan * CHV * nc; t += NT) {
+            const int r = (t * T.inv_nc) >> 16, c = t - r * nc;
+            const int ch = r / CHV, k = r - ch * CHV;
+            const double* src = (k < 4) ? A.rates + (size_t)(4 * ch + k) * C
+                              : (k == 4) ? A.chan_mod + (size_t)ch * C
+                                         : A.c_cell_in + (size_t)((P.chan_ion_pack >> (4 * ch)) & 15u) * C;
+            L.chv[r * A.chan_nc + c] = src[c0 + c];
+        }
+    }
+    tile_sync<WSYNC>();
 
-    if (m < m1) {
-        const int mc = A.mem_cell[m];
-        const int cn = A.nn_cell[m];
-        const bool bnd = (A.nn_mem[m] == m);
-        const int k = A.mem_sq[m];
-        const int pos = A.mem_pos[m];
-        const double sa = A.mem_sa[m];
+    if (own_mem) {
+        const int cn = R.nn_cell & ~MREC_BND;
+        const bool bnd = R.nn_cell < 0;
+        const int k = R.sq;
+        const int lc = __builtin_amdgcn_mbcnt_hi((unsigned)(T.starts >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)T.starts, 0));
+        if (W == 0 && (j == 0 || ((T.starts >> (j - 1)) & 1))) L.start[lc] = j;
         const double gjo = (gjo_u == gjo_u) ? gjo_u : A.gjopen[m];
         // Vmem of the membrane and of its partner: (1/cm) rho_surf of the cell
         // less Phi_b at the membrane's square (update_V, sim.py:2029)
-        double v = A.vm_in[mc];
+        double v = L.v[lc];
         double vn = A.vm_in[cn];
         if (still_mem & PHIB_BIT) {
             v = v - A.Phi_b[k];
-            vn = vn - A.Phi_b[A.mem_sq[A.nn_mem[m]]];
+            vn = vn - A.Phi_b[R.nn_sq];
+        }
+        const bool do_nak = P.i_na >= 0 && (P.i_na / NS == W || P.i_k / NS == W);
+        double nai = 0.0, nao = 0.0, ki = 0.0, ko = 0.0, cai = 0.0, cao = 0.0;
+        if (do_nak) {
+            nao = A.c_env[P.i_na * G2 + k];
+            ko = A.c_env[P.i_k * G2 + k];
+            nai = L.lag[P.i_na][lc];
+            ki = L.lag[P.i_k][lc];
+        }
+        if (P.i_ca >= 0 && P.i_ca / NS == W) {
+            cai = A.c_cell_in[P.i_ca * C + c0 + lc];
+            cao = A.c_mid[P.i_ca * G2 + k];
         }
         // the gathers of one ion slot / channel slot, issued together
-        double g_env[NS], g_lag[NS], g_lagn[NS], g_dm[NS];
+        double g_env[NS], g_lagn[NS], g_dm[NS];
         auto gather_ion = [&](int s) {
             const int i = W * NS + s;
             const double du = KC->dm_u[i];
             // the cluster's uniform Dm when it has one, else the membrane's;
             // nothing for a law with zero permeability (still ion, zero
-            // gap-junction diffusivity), which ghk_reuse does not evaluate
+            // gap-junction diffusivity), which ghk_reuse does not evaluate;
+            // the pump's ions have their env value already
             const bool still = (still_mem >> i) & 1u;
             const bool gstill = (P.dgj_surf[i] == 0.0);
-            g_env[s] = still ? 0.0 : A.c_env[i * G2 + k];
-            g_lag[s] = (still && gstill) ? 0.0 : A.c_lag_in[i * C + mc];
+            if (do_nak && i == P.i_na) g_env[s] = nao;
+            else if (do_nak && i == P.i_k) g_env[s] = ko;
+            else g_env[s] = still ? 0.0 : A.c_env[i * G2 + k];
             g_lagn[s] = gstill ? 0.0 : A.c_lag_in[i * C + cn];
             // (a wave-uniform choice: the cluster's value is already in SGPRs,
             // so a uniform Dm costs no load; a pointer chosen between the two
             // made every lane load, and measured 10% slower on the batch)
             g_dm[s] = still ? 0.0 : ((du == du) ? du : A.Dm[i * M + m]);
         };
-        double h_m[NQ], h_h[NQ], h_mod[NQ], h_out[NQ], h_in[NQ];
-        // the update coefficients a_m, b_m, a_h, b_h of each gate (per cell, from k_env_field)
-        double r_mi[NQ], r_mt[NQ], r_hi[NQ], r_ht[NQ];
-        auto gather_chan = [&](int q) {
-            const int ch = W + q * WG;
-            const int i = P.chan_ion[ch];
-            h_m[q] = A.gates[(size_t)(2 * ch) * M + m];
-            h_h[q] = A.gates[(size_t)(2 * ch + 1) * M + m];
-            h_mod[q] = A.chan_mod[(size_t)ch * C + mc];
-            h_out[q] = A.c_mid[i * G2 + k];
-            h_in[q] = A.c_cell_in[i * C + mc];
-            const double* R = A.rates + (size_t)(4 * ch) * C + mc;
-            r_mi[q] = R[0];
-            r_mt[q] = R[C];
-            r_hi[q] = R[2 * C];
-            r_ht[q] = R[3 * C];
-        };
-        const bool do_nak = P.i_na >= 0 && (P.i_na / NS == W || P.i_k / NS == W);
-        double nai = 0.0, nao = 0.0, ki = 0.0, ko = 0.0, cai = 0.0, cao = 0.0;
-        if (do_nak) {
-            nai = A.c_lag_in[P.i_na * C + mc];
-            nao = A.c_env[P.i_na * G2 + k];
-            ki = A.c_lag_in[P.i_k * C + mc];
-            ko = A.c_env[P.i_k * G2 + k];
-        }
-        if (P.i_ca >= 0 && P.i_ca / NS == W) {
-            cai = A.c_cell_in[P.i_ca * C + mc];
-            cao = A.c_mid[P.i_ca * G2 + k];
-        }
 
         // NaK-ATPase on the lagged membrane concentrations (sim.py:1196-1234, Q1)
         FT fNa = (FT)0;
@@ -580,6 +647,9 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
         for (int s = 0; s < NS; ++s) {
             const int i = W * NS + s;
             if (i >= NI) break;
+            // (convergent: every lane has read an ion's staged concentrations
+            // before any lane writes the row)
+            if (WG == 1) __builtin_amdgcn_wave_barrier();
             if (s + 1 < NS && i + 1 < NI) gather_ion(s + 1);
             if (s > 0) {
                 vmut = with_nonces(vmut, 1);
@@ -589,7 +659,7 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
             if (i == P.i_na) f = f + (double)fNa;
             if (i == P.i_k) f = f + (double)((FT)P.k_per_na * fNa);
             // GHK across the membrane and across the gap junction (sim.py:1253-1269, 2162-2206)
-            const double clag = g_lag[s];
+            const double clag = L.lag[i][lc];
             const FT fED = ghk_reuse<FT>((FT)g_env[s], (FT)clag, (FT)g_dm[s], (FT)P.zplus[i], (FT)vmut,
                                          on_path<FT>(P.f_rt, P.f_rt32), on_path<FT>(P.inv_tm, P.inv_tm32), last_m);
             f = f + (double)fED;
@@ -614,8 +684,8 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
             const double x = f * sa;
             L.mem[i][j] = x;
             if (!((still_mem >> i) & 1u)) {                  // the exchange reads no still row
-                if constexpr (sizeof(FT) == 4) static_cast<float*>(A.fsa)[(size_t)i * M + pos] = (float)x;
-                else static_cast<double*>(A.fsa)[(size_t)i * M + pos] = x;
+                if constexpr (sizeof(FT) == 4) static_cast<float*>(A.fsa)[(size_t)i * M + R.pos] = (float)x;
+                else static_cast<double*>(A.fsa)[(size_t)i * M + R.pos] = x;
             }
             L.gj[i][j] = (-fgj) * sa;
         }
@@ -629,100 +699,103 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             const int ch = W + q * WG;
-            if (ch >= P.n_chan) break;
-            gather_chan(q);
+            if (ch >= n_chan) break;
             const int i = P.chan_ion[ch];
+            const double h_m = A.gates[(size_t)(2 * ch) * M + m];
+            const double h_h = A.gates[(size_t)(2 * ch + 1) * M + m];
+            const double h_out = A.c_mid[i * G2 + k];
+            const double* cv = L.chv + ch * CHV * A.chan_nc + lc;
+            const int cs = A.chan_nc;
             const double vg = with_nonces(v, NI + ch);
             const int kind = P.chan_kind[ch];
             // update_mh as x' = a x + b with the per-cell coefficients a, b of each gate
-            const double mm = r_mi[q] * h_m[q] + r_mt[q];
-            const double hh = r_hi[q] * h_h[q] + r_ht[q];
+            const double mm = cv[0] * h_m + cv[cs];
+            const double hh = cv[2 * cs] * h_h + cv[3 * cs];
             A.gates[(size_t)(2 * ch) * M + m] = mm;
             A.gates[(size_t)(2 * ch + 1) * M + m] = hh;
             // m**p * h**q: p = 2 squares as NumPy does, p = 3 is cube()
             const double Pch = (kind == BT_CHAN_NAV1P2) ? cube(mm) * hh
                              : (kind == BT_CHAN_KV1P1) ? mm * (hh * hh) : (mm * mm) * hh;
-            const FT Dch = (FT)(Pch * P.chan_max_dm[ch] * h_mod[q]);
-            const FT fc = ghk_path<FT>((FT)h_out[q], (FT)h_in[q], Dch, (FT)P.zplus[i], (FT)(vg + FLOAT_NONCE),
+            const FT Dch = (FT)(Pch * P.chan_max_dm[ch] * cv[4 * cs]);
+            const FT fc = ghk_path<FT>((FT)h_out, (FT)cv[5 * cs], Dch, (FT)P.zplus[i], (FT)(vg + FLOAT_NONCE),
                                        P.f_rt, P.inv_tm, P.f_rt32, P.inv_tm32);
             const double x = (double)fc * sa;
             L.ch[ch][j] = x;
-            A.fch[(size_t)ch * M + pos] = x;
+            A.fch[(size_t)ch * M + R.pos] = x;
             if (OBS) A.obs_fch[(size_t)ch * M + m] = (double)fc;
         }
     }
     // per-cell inputs of the second stage, loaded once the membrane stage is
     // done: held from the start, their registers cost a wave per SIMD of
     // occupancy (measured slower on the 500k-cell batch)
-    const int c = c0 + j;
-    const bool own_cell = (c < c1);
-    int ca = 0, cb = 0;
-    double vol = 1.0, divi = 0.0;
-    double cin[NS];
-    if (own_cell) {
-        ca = A.mem_ptr[c] - m0;
-        cb = A.mem_ptr[c + 1] - m0;
-        vol = A.cell_vol[c];
-        divi = A.diviterm[c];
+    double cin[NPASS], vol[NPASS], divi = 0.0;
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-            if (W * NS + s < NI) cin[s] = A.c_cell_in[(W * NS + s) * C + c];
+    for (int p = 0; p < NPASS; ++p) {
+        if (p * NT >= n_items) break;
+        int i, c;
+        if (item(p, i, c)) {
+            cin[p] = A.c_cell_in[(size_t)i * C + c0 + c];
+            vol[p] = A.cell_vol[c0 + c];
+        }
     }
+    if (W == 0 && j < nc) divi = A.diviterm[c0 + j];
 
     tile_sync<WSYNC>();
 
     // per-cell segment sums in membrane order (np.dot(M_sum_mems, .)), then
-    // update_Co, the GJ update, no_negs, and rho_cells -> Vmem (ion order)
-    if (own_cell) {
-        bool bad = false;
-        double rho = 0.0;
-        // x / vol as the product by 1/vol (an FP64 ulp; one division per cell
-        // instead of three per ion)
-        const double rvol = 1.0 / vol;
-        auto per_vol = [&](double x) { return x * rvol; };
+    // update_Co, the GJ update, no_negs (a lane per ion and cell), and
+    // rho_cells -> Vmem (a lane per cell, in ion order)
+    bool bad = false;
+    double c2v[NPASS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const int i = W * NS + s;
-            if (i >= NI) break;
-            double base = cin[s];
-            const int ch = P.ion_chan[i];
-            if (ch >= 0) {             // immediate update_Co of the channel flux
+    for (int p = 0; p < NPASS; ++p) {
+        if (p * NT >= n_items) break;
+        int i, c;
+        if (!item(p, i, c)) continue;
+        const int ca = L.start[c], cb = L.start[c + 1];
+        // x / vol as the product by 1/vol (an FP64 ulp; one division per cell
+        // and ion instead of three)
+        const double rvol = 1.0 / vol[p];
+        auto per_vol = [&](double x) { return x * rvol; };
+        double base = cin[p];
+        if (n_chan > 0) {
+            const unsigned ch = (P.ion_chan_pack >> (4 * i)) & 15u;
+            if (ch != 15u) {           // immediate update_Co of the channel flux
                 double Sc = L.ch[ch][ca];
                 for (int q = ca + 1; q < cb; ++q) Sc = Sc + L.ch[ch][q];
                 base = base + per_vol(Sc) * P.dt;
             }
-            double S = L.mem[i][ca];
-            double Sg = L.gj[i][ca];
-            for (int q = ca + 1; q < cb; ++q) {
-                S = S + L.mem[i][q];
-                Sg = Sg + L.gj[i][q];
-            }
-            const double c1v = base + per_vol(S) * P.dt;
-            A.c_lag_out[i * C + c] = c1v;
-            double c2 = c1v + P.dt * per_vol(Sg);
-            if (c2 < 0.0) c2 = 0.0;                    // no_negs clamp (Q9)
-            if (isnan(c2)) bad = true;
-            A.c_cell_out[i * C + c] = c2;
-            if (WG > 1) L.c2[i][j] = c2;
-            else rho = (i == 0) ? P.zF[0] * c2 : rho + P.zF[i] * c2;
         }
-        if (WG == 1) {
-            const double vm = P.cm_inv * (rho * divi);
-            if (isnan(vm)) bad = true;
-            A.vm_out[c] = vm;
+        double S = L.mem[i][ca];
+        double Sg = L.gj[i][ca];
+        for (int q = ca + 1; q < cb; ++q) {
+            S = S + L.mem[i][q];
+            Sg = Sg + L.gj[i][q];
         }
-        if (bad) *L.bad = 1;
+        const double c1v = base + per_vol(S) * P.dt;
+        A.c_lag_out[(size_t)i * C + c0 + c] = c1v;
+        double c2 = c1v + P.dt * per_vol(Sg);
+        if (c2 < 0.0) c2 = 0.0;                    // no_negs clamp (Q9)
+        if (isnan(c2)) bad = true;
+        A.c_cell_out[(size_t)i * C + c0 + c] = c2;
+        c2v[p] = c2;
     }
-    if (WG > 1) {
-        tile_sync<WSYNC>();
-        if (W == 0 && own_cell) {
-            double rho = P.zF[0] * L.c2[0][j];
+    if (bad) *L.bad = 1;
+    tile_sync<WSYNC>();
 #pragma unroll
-            for (int i = 1; i < NI; ++i) rho = rho + P.zF[i] * L.c2[i][j];
-            const double vm = P.cm_inv * (rho * divi);
-            if (isnan(vm)) *L.bad = 1;
-            A.vm_out[c] = vm;
-        }
+    for (int p = 0; p < NPASS; ++p) {
+        if (p * NT >= n_items) break;
+        int i, c;
+        if (item(p, i, c)) L.mem[i][c] = c2v[p];
+    }
+    tile_sync<WSYNC>();
+    if (W == 0 && j < nc) {
+        double rho = P.zF[0] * L.mem[0][j];
+#pragma unroll
+        for (int i = 1; i < NI; ++i) rho = rho + P.zF[i] * L.mem[i][j];
+        const double vm = P.cm_inv * (rho * divi);
+        if (isnan(vm)) *L.bad = 1;
+        A.vm_out[c0 + j] = vm;
     }
     tile_sync<WSYNC>();
     if (W == 0 && j == 0 && *L.bad) {
@@ -731,27 +804,32 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     }
 }
 
+// LDS of one tile beyond the ions' flux rows: its channels' rows (fluxes, and
+// the per-cell values of chan_nc cells), in doubles
+__host__ __device__ constexpr int mem_chan_lds(int n_chan, int chan_nc) { return n_chan * (TMB + CHV * chan_nc); }
+
 // OBS: an observed step (the raw fluxes also go to the observation buffers)
 template <int NI, typename FT, int WG, bool OBS>
 __global__ void __launch_bounds__(TMB * WG)
 k_mem_cell(MemCellArgs A, KParams P) {
     static_assert(WG == 1 || WG == 2, "one or two wavefronts per tile");
     if (halted(A.flags)) return;
-    // WG wavefronts per tile; lane j of each owns membrane m0 + j and, in the
-    // per-cell stage, cell c0 + j. Wavefront w evaluates the ions
-    // [w * NS, w * NS + NS) with NS = ceil(n_ions / WG) (its ion slots; Na and
-    // K, the first two, share one pump evaluation) and the channels w, w + WG,
-    // ..., so small problems still fill the GPU. Both wavefronts pass the same
-    // barriers.
+    // WG wavefronts per tile; lane j of each owns membrane m0 + j. Wavefront w
+    // evaluates the ions [w * NS, w * NS + NS) with NS = ceil(n_ions / WG)
+    // (its ion slots; Na and K, the first two, share one pump evaluation) and
+    // the channels w, w + WG, ..., so small problems still fill the GPU. Both
+    // wavefronts pass the same barriers.
     __shared__ double s_mem[NI][TMB];
     __shared__ double s_gj[NI][TMB];
-    // channel fluxes: n_chan rows, in dynamic LDS sized at launch (none
-    // without channels, which leaves room for more blocks per CU)
+    __shared__ double s_lag[WG > 1 ? NI : 1][WG > 1 ? TMB : 1];
+    __shared__ double s_v[WG > 1 ? BT_TILE_CELLS : 1];
+    // channel rows: dynamic LDS sized at launch (none without channels, which
+    // leaves room for more blocks per CU)
     extern __shared__ double s_dyn[];
-    double (*s_ch)[TMB] = reinterpret_cast<double (*)[TMB]>(s_dyn);
-    __shared__ double s_c2[WG > 1 ? NI : 1][TMB];
+    __shared__ int s_start[BT_TILE_CELLS + 1];
     __shared__ int s_bad;
-    const MemLds L{s_mem, s_gj, s_ch, s_c2, &s_bad};
+    const MemLds L{s_mem, s_gj, reinterpret_cast<double (*)[TMB]>(s_dyn), s_dyn + P.n_chan * TMB,
+                   WG > 1 ? reinterpret_cast<double (*)[TMB]>(s_lag) : s_mem, WG > 1 ? s_v : s_gj[0], s_start, &s_bad};
     const int tile = xcd_chunk(blockIdx.x, gridDim.x);
     const int w = (WG > 1) ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / TMB)) : 0;
     if (w == 0) mem_cell_wave<NI, FT, WG, 0, OBS>(A, P, tile, L);
@@ -2006,9 +2084,11 @@ struct PersistArgs {
 };
 
 // LDS of one membrane-phase wavefront, in doubles: flux*sa and GJ flux per ion,
-// channel flux per channel, and the tile's NaN flag
-template <int NI>
-constexpr int mem_wave_lds() { return (2 * NI + BT_MAX_CHAN) * TMB + 1; }
+// the channels' rows, the cells' first membranes and the tile's NaN flag
+template <int NI, bool CHAN>
+constexpr int mem_wave_lds() {
+    return 2 * NI * TMB + (CHAN ? mem_chan_lds(BT_MAX_CHAN, BT_TILE_CELLS) : 0) + (BT_TILE_CELLS + 3) / 2;
+}
 
 // Grid barrier of a cooperative launch. Thread 0 of each block reads the
 // generation, arrives, and the last arrival resets the count and opens the next
@@ -2049,7 +2129,7 @@ __device__ __forceinline__ bool grid_sync(unsigned* bar, unsigned* flags) {
 template <int NI, typename FT, bool RATES>
 __global__ void __launch_bounds__(PB, PERSIST_WAVES_PER_SIMD)
 k_step_persistent(PersistArgs PA, KParams P) {
-    constexpr int MW = mem_wave_lds<NI>();
+    constexpr int MW = mem_wave_lds<NI, RATES>();
     constexpr int LDS = ENV_LDS > PW * MW ? ENV_LDS : PW * MW;
     __shared__ double lds[LDS];
     __shared__ int s_stop;
@@ -2060,9 +2140,10 @@ k_step_persistent(PersistArgs PA, KParams P) {
     const int n_env_items = PA.n_env_tiles * PA.n_groups;
     // this wavefront's slice of the LDS in the membrane phase
     double* wl = lds + wave * MW;
+    int* wi = reinterpret_cast<int*>(wl + MW - (BT_TILE_CELLS + 3) / 2);
     const MemLds L{reinterpret_cast<double (*)[TMB]>(wl), reinterpret_cast<double (*)[TMB]>(wl + NI * TMB),
-                   reinterpret_cast<double (*)[TMB]>(wl + 2 * NI * TMB), reinterpret_cast<double (*)[TMB]>(wl),
-                   reinterpret_cast<int*>(wl + (2 * NI + BT_MAX_CHAN) * TMB)};
+                   reinterpret_cast<double (*)[TMB]>(wl + 2 * NI * TMB), wl + (2 * NI + P.n_chan) * TMB,
+                   reinterpret_cast<double (*)[TMB]>(wl), wl + NI * TMB, wi, wi + BT_TILE_CELLS + 1};
     // one step of parity PAR (a compile-time index into the argument sets);
     // false once a grid barrier gave up
     auto step = [&](auto par_c) -> bool {
@@ -2132,7 +2213,9 @@ struct bt_ctx {
     hipStream_t stream = nullptr;
     int device = 0;
     int n_tiles = 0;
+    int tile_nc = 0;                // cells of the largest tile
     // workspace
+    TileRec* tiles = nullptr; MemRec* mrec = nullptr;   // the geometry as k_mem_cell reads it
     double* c_cell_b = nullptr; double* c_lag_b = nullptr; double* vm_b = nullptr;
     double* c_mid = nullptr; void* fsa = nullptr; double* fch = nullptr; double* u = nullptr;
     double* u_b = nullptr;    // surface charge of odd steps with the fused exchange
@@ -2210,7 +2293,9 @@ static void derive_params(const bt_params& p, KParams& k) {
         k.chan_ion[c] = p.chan_ion[c];
         k.chan_max_dm[c] = p.chan_max_dm[c];
         k.ion_chan[p.chan_ion[c]] = c;
+        k.chan_ion_pack |= (unsigned)p.chan_ion[c] << (4 * c);
     }
+    for (int i = 0; i < BT_MAX_IONS; ++i) k.ion_chan_pack |= (unsigned)(k.ion_chan[i] & 15) << (4 * i);
     k.chan_dt = p.chan_dt;
     for (int i = 0; i < p.n_ions; ++i) {
         k.zplus[i] = p.z[i] + FLOAT_NONCE;
@@ -2305,7 +2390,7 @@ static Span group_span(const bt_ctx* c, int G, int g) {
 
 template <int NI, int WG, bool OBS>
 static void launch_mem_cell_o(bt_ctx* c, const MemCellArgs& a, hipStream_t st, int nt) {
-    const size_t lds = (size_t)c->prm.n_chan * TMB * sizeof(double);     // s_ch
+    const size_t lds = (size_t)mem_chan_lds(c->prm.n_chan, c->tile_nc) * sizeof(double);
     if (c->prm.flux_mode == BT_FLUX_FP32)
         hipLaunchKernelGGL((k_mem_cell<NI, float, WG, OBS>), dim3(nt), dim3(TMB * WG), lds, st, a, c->kp);
     else
@@ -2322,7 +2407,7 @@ static void launch_mem_cell_t(bt_ctx* c, const MemCellArgs& a, hipStream_t st, i
     else launch_mem_cell_w<NI, 1>(c, a, st, nt);
 }
 
-// k_mem_cell over nt cell tiles (a.tile_ptr and a.tile_cluster start at the first)
+// k_mem_cell over nt cell tiles (a.tiles starts at the first)
 static void launch_mem_cell(bt_ctx* c, const MemCellArgs& a, hipStream_t st, int nt) {
     switch (c->prm.n_ions) {
         case 1: launch_mem_cell_t<1>(c, a, st, nt); break;
@@ -2405,13 +2490,12 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
     double* ei = parity ? c->c_env_b : B.c_env;
     double* eo = parity ? B.c_env : c->c_env_b;
     StepArgs a{field_args(c, true, ob, vi, ei, eo),
-               MemCellArgs{B.mem_ptr, B.mem_cell, B.nn_mem, B.nn_cell, B.mem_sq, B.mem_pos, B.tile_ptr,
-                           B.tile_cluster, c->kcl,
+               MemCellArgs{c->tiles, c->mrec, c->kcl,
                            B.mem_sa, B.gjopen, B.cell_vol, B.diviterm, B.Dm, ei, c->c_mid,
                            ci, li, vi, co, lo, vo, c->fsa, B.gates, B.chan_mod, c->rates, c->fch,
                            c->flags, c->bad_step, c->step_ctr,
                            ob ? ob->fluxes_mem : nullptr, ob ? ob->fluxes_gj : nullptr,
-                           ob ? ob->chan_flux : nullptr, ob ? ob->rate_NaKATP : nullptr, B.Phi_b},
+                           ob ? ob->chan_flux : nullptr, ob ? ob->rate_NaKATP : nullptr, B.Phi_b, c->tile_nc},
                ExArgs{B.sq_ptr, B.sq_has_mem, B.sq_cluster, c->kcl, c->c_mid, c->fsa, c->fch, eo, c->u,
                       c->prm.flux_mode == BT_FLUX_FP32 ? 1 : 0, c->flags,
                       c->step_ctr, count_step, (1u << BT_MAX_STREAMS) - 1u, c->sq_live, c->n_live}};
@@ -2434,8 +2518,7 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
         // that every counter holds the step count when a later split reads it)
         const Span sp = group_span(c, G, g);
         a.field.env_tiles += 3 * sp.e0;
-        a.mem.tile_ptr += sp.t0;
-        a.mem.tile_cluster += sp.t0;
+        a.mem.tiles += sp.t0;
         a.mem.step_ctr += g;
         a.ex.sq_live += sp.l0;
         a.ex.n_live = sp.nl;
@@ -2507,6 +2590,14 @@ static int persistent_grid(bt_ctx* c) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1)
         return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, PB, 0) != hipSuccess || per_cu < 1) return 0;
+    // what stays resident by LDS, counted apart with each block's LDS rounded up
+    // to 2 KB of the CU's 160 KB: the query divides the exact sizes, the
+    // hardware hands out larger granules, and one block too many never arrives
+    // at the grid barrier
+    hipFuncAttributes fa;
+    if (hipFuncGetAttributes(&fa, k) != hipSuccess) return 0;
+    per_cu = std::min(per_cu, (int)(160 * 1024 / std::max<size_t>((fa.sharedSizeBytes + 2047) / 2048 * 2048, 2048)));
+    if (per_cu < 1) return 0;
     c->pers_grid = per_cu * cus;
     return c->pers_grid;
 }
@@ -2968,12 +3059,31 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
             return set_err(nullptr, rc, msg);
         }
     }
+    // the geometry as k_mem_cell reads it
+    std::vector<TileRec> trec((size_t)b->n_tiles);
+    std::vector<MemRec> mrec(NM);
+    for (int t = 0; t < b->n_tiles; ++t) {
+        TileRec& r = trec[t];
+        r.c0 = tp[t];
+        r.m0 = mp[tp[t]];
+        r.n_cells = tp[t + 1] - tp[t];
+        r.n_mems = mp[tp[t + 1]] - r.m0;
+        r.cluster = tcl[t];
+        r.inv_nc = 65536 / r.n_cells + 1;
+        r.starts = 0;
+        for (int q = tp[t] + 1; q < tp[t + 1]; ++q) r.starts |= 1ull << (mp[q] - r.m0 - 1);
+        c->tile_nc = std::max(c->tile_nc, r.n_cells);
+    }
+    for (size_t m = 0; m < NM; ++m)
+        mrec[m] = MemRec{(nnm[m] == (int32_t)m) ? (nnc[m] | MREC_BND) : nnc[m], msq[m], mpos[m], msq[nnm[m]]};
     (void)hipGetDevice(&c->device);
     const size_t nc = p->n_cells, nm = p->n_mems, ni = p->n_ions, ns = (size_t)p->n_squares;
     hipError_t e = hipSuccess;
     auto alloc = [&](void** ptr, size_t bytes) {
         if (e == hipSuccess) e = hipMalloc(ptr, bytes < 256 ? 256 : bytes);
     };
+    alloc((void**)&c->tiles, trec.size() * sizeof(TileRec));
+    alloc((void**)&c->mrec, mrec.size() * sizeof(MemRec));
     alloc((void**)&c->c_cell_b, ni * nc * 8);
     alloc((void**)&c->c_lag_b, ni * nc * 8);
     alloc((void**)&c->vm_b, nc * 8);
@@ -3004,6 +3114,8 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     if (c->tune.exchange_form == 1 && fused_allowed(c, &c->tune)) c->tune.exchange_form = BT_EXCHANGE_FUSED;
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, sq_live.data(), sizeof(int32_t) * sq_live.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(c->mrec, mrec.data(), mrec.size() * sizeof(MemRec), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->live_flag, live_flag.data(), ns, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(c->kcl, c->kcl_host.data(), sizeof(KCluster) * (size_t)n_clusters, hipMemcpyHostToDevice);
@@ -3036,7 +3148,7 @@ int bt_destroy(bt_ctx* c) {
         if (c->ev_join[g]) (void)hipEventDestroy(c->ev_join[g]);
     }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
-    void* ptrs[] = {c->c_cell_b, c->c_lag_b, c->vm_b, c->c_mid, c->fsa, c->fch, c->u, c->u_b, c->rates, c->c_env_b,
+    void* ptrs[] = {c->tiles, c->mrec, c->c_cell_b, c->c_lag_b, c->vm_b, c->c_mid, c->fsa, c->fch, c->u, c->u_b, c->rates, c->c_env_b,
                     c->sq_live, c->live_flag, c->flags, c->bad_step, c->step_ctr, c->kcl, c->env_tiles,
                     c->vm_prev, c->net, c->bar, c->phib_stage, c->phib_prev};
     for (void* q : ptrs)
