@@ -62,12 +62,22 @@ constexpr int TMB = BT_TILE_MEMBRANES;   // membranes per k_mem_cell tile (one w
 constexpr int BLOCK = 256;               // threads per per-square kernel block
 constexpr int TY = 16, TX = 16;          // k_env_field tile
 // Default launch variants by problem size (bt_tuning; bt_autotune measures
-// them per problem): below ENV_SPLIT_TILES env tiles k_env_field splits its
-// blocks by pairs of ions (measured: pairs of ions win by 35% at 256 tiles,
-// one block per tile by 10% at 1024); below EX_SPLIT_SQUARES squares with
-// membranes k_env_exchange runs one wavefront per ion
+// them per problem). Until the caller forces a variant, and where no membrane law
+// reads the post-diffusion env, whole steps from FUSE_TILES cell tiles on have the
+// exchange in the env kernel (us per step with it and, in brackets, as a launch of
+// its own with the better of the splits below: 532 tiles 17.2 (17.6), 2,193 tiles
+// 20.2 (25.5), 5,428 30.0 (36.2), 19,239 67.6 (81.6), 50,081 187 (231)). Elsewhere,
+// below ENV_SPLIT_TILES env tiles k_env_field splits its blocks by pairs of ions
+// (measured: pairs of ions win by 35% at 256 tiles, one block per tile by 10% at
+// 1024); below EX_SPLIT_SQUARES squares with membranes k_env_exchange runs one
+// wavefront per ion
 constexpr int ENV_SPLIT_TILES = 1024;
 constexpr int EX_SPLIT_SQUARES = 1 << 19;
+constexpr int FUSE_TILES = 512;
+// Step counters and halt flags: one per group of clusters stepped apart
+// (stream groups, or groups stepped one after the other)
+constexpr int MAX_GROUPS = 16;
+static_assert(MAX_GROUPS >= BT_MAX_STREAMS, "a counter per stream group");
 constexpr double FLOAT_NONCE = 1.0e-25;  // sim_toolbox.py:50
 
 // Constants derived on the host, each in the reference's evaluation order.
@@ -804,6 +814,16 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     }
 }
 
+// the membranes' records, once per context
+__global__ void __launch_bounds__(BLOCK)
+k_mem_records(const int32_t* nn_mem, const int32_t* nn_cell, const int32_t* mem_sq, const int32_t* mem_pos, MemRec* out,
+              int n) {
+    const int m = blockIdx.x * BLOCK + threadIdx.x;
+    if (m >= n) return;
+    const int nm = nn_mem[m];
+    out[m] = MemRec{nm == m ? (nn_cell[m] | MREC_BND) : nn_cell[m], mem_sq[m], mem_pos[m], mem_sq[nm]};
+}
+
 // LDS of one tile beyond the ions' flux rows: its channels' rows (fluxes, and
 // the per-cell values of chan_nc cells), in doubles
 __host__ __device__ constexpr int mem_chan_lds(int n_chan, int chan_nc) { return n_chan * (TMB + CHV * chan_nc); }
@@ -1241,7 +1261,7 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // a halted run writes nothing (every thread read the same flag)
     if (stop) return;
     if (FUSE && A.count_step && tile_id == 0 && ion_id == 0 && tid == 0)
-        for (int g = 0; g < BT_MAX_STREAMS; ++g)
+        for (int g = 0; g < MAX_GROUPS; ++g)
             if (A.ctr_mask & (1u << g)) A.step_ctr[g] = A.step_ctr[g] + 1;
     const int o = (lr + 2) * VC + lc + 2;                       // own square in sV and the staged ions
     // grad(screen * v_env) along one axis (E = -grad, one-sided at the world
@@ -1412,7 +1432,7 @@ constexpr int EXQ = 64;
 
 __device__ __forceinline__ void advance_step(const ExArgs& A) {
 #pragma unroll
-    for (int g = 0; g < BT_MAX_STREAMS; ++g)
+    for (int g = 0; g < MAX_GROUPS; ++g)
         if (A.ctr_mask & (1u << g)) A.step_ctr[g] = A.step_ctr[g] + 1;
 }
 
@@ -2039,6 +2059,12 @@ k_gemm_grouped(const GemmProb* probs, const int32_t* block_prob) {
     gemm_tile(P.A, P.B, P.C, P.S, P.n, P.k, (int)blockIdx.x - P.tile0, part);
 }
 
+// a halt of any of the G groups becomes a halt of all
+__global__ void __launch_bounds__(64) k_spread_halt(unsigned* flags, int G) {
+    const unsigned f = (threadIdx.x < G) ? flags[threadIdx.x] : 0u;
+    if (__ballot(f != 0u) && threadIdx.x < MAX_GROUPS) flags[threadIdx.x] = f | 1u;
+}
+
 // per-cluster max over cells and ions of |c - c_prev| / |c| (init residual)
 __global__ void __launch_bounds__(BLOCK)
 k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, unsigned long long* rmax,
@@ -2225,9 +2251,10 @@ struct bt_ctx {
     uint8_t* live_flag = nullptr;        // per square: SQ_LIVE if in sq_live, SQ_HAS_MEM
     int n_live = 0;
     unsigned* flags = nullptr; unsigned long long* bad_step = nullptr; long long* step_ctr = nullptr;
-    // step graphs per stream group g: one pair of steps, and tune.graph_pairs pairs
-    hipGraph_t graph[BT_MAX_STREAMS] = {}; hipGraphExec_t gexec[BT_MAX_STREAMS] = {};
-    hipGraph_t graph_n[BT_MAX_STREAMS] = {}; hipGraphExec_t gexec_n[BT_MAX_STREAMS] = {};
+    // step graphs per group g of clusters: one pair of steps, and tune.graph_pairs pairs
+    hipGraph_t graph[MAX_GROUPS] = {}; hipGraphExec_t gexec[MAX_GROUPS] = {};
+    hipGraph_t graph_n[MAX_GROUPS] = {}; hipGraphExec_t gexec_n[MAX_GROUPS] = {};
+    int serial_groups = 1;               // groups of clusters whose replayed steps run one after the other
     // stream groups (tune.streams > 1): per cluster q, the first of its cell
     // tiles, env tiles and live squares and of its cells (n_clusters + 1
     // entries each; empty where the clusters' work lists are not in cluster
@@ -2241,6 +2268,9 @@ struct bt_ctx {
     hipEvent_t ev_fork = nullptr;
     hipEvent_t ev_join[BT_MAX_STREAMS] = {};
     bt_tuning tune{};                  // launch variants of the step kernels
+    // until bt_set_tuning or bt_autotune says which, whole steps fuse the
+    // exchange into the env kernel wherever that is allowed
+    bool auto_pick = false;
     bool autotuned = false;
     unsigned* bar = nullptr;           // grid barrier of the persistent step kernel
     int pers_grid = -1;                // its cooperative grid (-1 not yet known, 0 unavailable)
@@ -2356,8 +2386,9 @@ static KCluster derive_cluster(const bt_params& p, const bt_cluster& b) {
 
 // Default wavefronts per tile of k_mem_cell: two (ions split between them)
 // while one wavefront per tile would leave the SIMDs with few waves to switch
-// between; pairs of steps per replayed graph (fewer graph launches).
-constexpr int BT_MEM_WG_TILES = 4096;
+// between (step us with two and one: 2,193 tiles 20.2 and 20.5, 3,849 tiles 27.3
+// and 24.7); pairs of steps per replayed graph (fewer graph launches).
+constexpr int BT_MEM_WG_TILES = 3000;
 constexpr int BT_GRAPH_PAIRS = 8;
 constexpr int BT_MAX_GRAPH_PAIRS = 64;
 constexpr int BT_PERSIST_STEPS = 512;   // steps per cooperative launch of the persistent kernel (even)
@@ -2375,7 +2406,7 @@ static Span group_span(const bt_ctx* c, int G, int g) {
     const int nq = (int)c->clusters.size();      // at least G (streams_allowed)
     // b[gg]: the first cluster of group gg, strictly increasing, with room
     // for one cluster in each later group
-    int b[BT_MAX_STREAMS + 1];
+    int b[MAX_GROUPS + 1];
     b[0] = 0;
     for (int gg = 1; gg < G; ++gg) {
         const long long target = c->cl_cell0[nq] * gg / G;
@@ -2438,7 +2469,7 @@ static void launch_field_args(bt_ctx* c, bool diffuse, const FieldArgs& f, hipSt
     // diffusion: one block per (tile, env_ions_per_block ions): few ions per
     // block while tiles alone would leave CUs idle, else one block per tile
     // looping over the ions; field only: one block per tile
-    const int ipb = c->tune.env_ions_per_block;
+    const int ipb = f.u_out ? c->prm.n_ions : c->tune.env_ions_per_block;
     dim3 grid(ne > 0 ? ne : c->n_env_tiles, diffuse ? (c->prm.n_ions + ipb - 1) / ipb : 1);
     auto launch = [&](auto rates, auto fuse, auto dvar, auto obs) {
         const size_t lds = (ENV_LDS + (fuse.value ? (size_t)c->prm.n_ions * TY * TX : 0)) * sizeof(double);
@@ -2498,7 +2529,7 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
                            ob ? ob->chan_flux : nullptr, ob ? ob->rate_NaKATP : nullptr, B.Phi_b, c->tile_nc},
                ExArgs{B.sq_ptr, B.sq_has_mem, B.sq_cluster, c->kcl, c->c_mid, c->fsa, c->fch, eo, c->u,
                       c->prm.flux_mode == BT_FLUX_FP32 ? 1 : 0, c->flags,
-                      c->step_ctr, count_step, (1u << BT_MAX_STREAMS) - 1u, c->sq_live, c->n_live}};
+                      c->step_ctr, count_step, (1u << MAX_GROUPS) - 1u, c->sq_live, c->n_live}};
     if (fused) {
         // the env kernel does the exchange: the surface charge ping-pongs
         // with the env state (the kernel reads u on a halo while it writes its
@@ -2522,20 +2553,48 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
         a.mem.step_ctr += g;
         a.ex.sq_live += sp.l0;
         a.ex.n_live = sp.nl;
-        a.ex.ctr_mask = (g == 0) ? (((1u << BT_MAX_STREAMS) - 1u) & ~((1u << G) - 2u)) : (1u << g);
+        a.ex.ctr_mask = (g == 0) ? (((1u << MAX_GROUPS) - 1u) & ~((1u << G) - 2u)) : (1u << g);
         a.field.ctr_mask = a.ex.ctr_mask;
+        if (c->tune.streams <= 1) {
+            // groups one after the other halt each by its own flag, so that the
+            // earliest unstable step is found whichever group it is in
+            // (k_spread_halt then stops all)
+            a.field.flags += g;
+            a.mem.flags += g;
+            a.ex.flags += g;
+        }
     }
     return a;
+}
+
+// the exchange fused into the env kernel: no membrane law may read the
+// post-diffusion env (Ca pump, channels), and one block must hold every ion
+// of a square (its charge)
+static bool fused_allowed(const bt_ctx* c, const bt_tuning* t) {
+    return c->prm.n_chan == 0 && c->prm.i_ca < 0 && t->env_ions_per_block == c->prm.n_ions;
+}
+
+// whether whole steps run with the exchange fused into the env kernel
+static bool steps_fused(const bt_ctx* c) {
+    if (!c->auto_pick || c->n_tiles < FUSE_TILES) return c->tune.exchange_form == BT_EXCHANGE_FUSED;
+    bt_tuning t = c->tune;
+    t.env_ions_per_block = c->prm.n_ions;
+    return fused_allowed(c, &t);
+}
+
+// the stream of group g of G: the caller's, or with stream groups its own
+static hipStream_t group_stream(bt_ctx* c, int G, int g) {
+    return (G > 1 && c->tune.streams > 1) ? c->gstream[g] : c->stream;
 }
 
 // One step on the stream.
 // which: -1 all, 0 membrane/cell, 1 env field+diffusion, 2 exchange, 3 field only
 static void enqueue_step(bt_ctx* c, int parity, int which = -1, int G = 1, int g = 0) {
     const bt_obs* ob = c->capture;
-    const bool fused = c->tune.exchange_form == BT_EXCHANGE_FUSED;
+    const bool fused = (which < 0) ? steps_fused(c) : c->tune.exchange_form == BT_EXCHANGE_FUSED;
     const StepArgs a = step_args(c, parity, ob, which < 0 ? 1 : 0, G, g, fused);
     const Span sp = group_span(c, G, g);
-    hipStream_t st = (G > 1) ? c->gstream[g] : c->stream;
+    hipStream_t st = group_stream(c, G, g);
     if (fused) {
         // membranes first (they read the pre-diffusion env only), then the
         // env kernel with the exchange
@@ -2647,7 +2706,7 @@ static int launch_persistent(bt_ctx* c, int n_steps) {
 }
 
 static void drop_graphs(bt_ctx* c) {
-    for (int g = 0; g < BT_MAX_STREAMS; ++g) {
+    for (int g = 0; g < MAX_GROUPS; ++g) {
         if (c->gexec[g]) { (void)hipGraphExecDestroy(c->gexec[g]); c->gexec[g] = nullptr; }
         if (c->graph[g]) { (void)hipGraphDestroy(c->graph[g]); c->graph[g] = nullptr; }
         if (c->gexec_n[g]) { (void)hipGraphExecDestroy(c->gexec_n[g]); c->gexec_n[g] = nullptr; }
@@ -2655,21 +2714,44 @@ static void drop_graphs(bt_ctx* c) {
     }
 }
 
+// whether the clusters can be split into G groups stepped apart
+static bool groups_allowed(const bt_ctx* c, int G) {
+    return G >= 1 && G <= MAX_GROUPS && (G == 1 || ((int)c->clusters.size() >= G && !c->cl_tile0.empty() &&
+                                                   c->prm.n_chan == 0 && !(c->net && c->c_net)));
+}
+
 // whether the problem can be stepped in G stream groups
-static bool streams_allowed(const bt_ctx* c, int G) {
-    return G >= 1 && G <= BT_MAX_STREAMS && (G == 1 || ((int)c->clusters.size() >= G && !c->cl_tile0.empty() &&
-                                                        c->prm.n_chan == 0 && !(c->net && c->c_net)));
+static bool streams_allowed(const bt_ctx* c, int G) { return G <= BT_MAX_STREAMS && groups_allowed(c, G); }
+
+// Groups of clusters whose replayed steps run one after the other, each group's
+// through a whole bt_step call: clusters do not interact within a step, and the
+// next step of a group whose data fits the 256 MB Infinity Cache finds it there,
+// where a step over a larger batch has pushed it out to HBM by the time it comes
+// back. The bytes are those a step moves: the state twice (ping-pong), the
+// membranes' records, areas and fluxes, the squares' flags. Measured, FP64, us per
+// step with one group and with two: 276 MB (304k cells) 114.0 and 115.8, 340 MB
+// 143.5 and 132.1, 400 MB 170.5 and 161.8, 468 MB (500k cells) 200.4 and 186.3
+// (three: 185.5): smaller groups also fill the GPU less well, so the second one
+// starts at 1.2 times the cache.
+constexpr double GROUP_BYTES = 256.0 * (1 << 20);
+static int pick_serial_groups(const bt_ctx* c) {
+    const long long ni = c->prm.n_ions;
+    const long long moving = ni - (c->kcl_host.empty() ? 0 : __builtin_popcount(c->kcl_host[0].still_mem & 0xffu));
+    const long long fb = c->prm.flux_mode == BT_FLUX_FP32 ? 4 : 8;
+    const long long bytes = (long long)c->prm.n_cells * (32 * ni + 40) +
+                            (long long)c->prm.n_mems * (long long)(sizeof(MemRec) + 8 + fb * moving) +
+                            (long long)c->prm.n_squares * (16 * ni + 21);
+    int G = (int)std::min(ceil((double)bytes / GROUP_BYTES - 0.2), (double)MAX_GROUPS);
+    while (G > 1 && !groups_allowed(c, G)) --G;
+    return std::max(G, 1);
 }
 
-// the exchange fused into the env kernel: no membrane law may read the
-// post-diffusion env (Ca pump, channels), and one block must hold every ion
-// of a square (its charge)
-static bool fused_allowed(const bt_ctx* c, const bt_tuning* t) {
-    return c->prm.n_chan == 0 && c->prm.i_ca < 0 && t->env_ions_per_block == c->prm.n_ions;
+// the groups of the current tuning: stream groups, or those stepped one after
+// the other (1: the whole problem at once)
+static int n_step_groups(const bt_ctx* c) {
+    if (c->tune.persistent) return 1;
+    return c->tune.streams > 1 ? (int)c->tune.streams : c->serial_groups;
 }
-
-// the stream groups of the current tuning (1: the whole problem on the caller's stream)
-static int n_stream_groups(const bt_ctx* c) { return c->tune.persistent ? 1 : std::max(1, (int)c->tune.streams); }
 
 // the groups' streams and the fork/join events, created on first use
 static int ensure_group_streams(bt_ctx* c, int G) {
@@ -2686,11 +2768,11 @@ static int ensure_group_streams(bt_ctx* c, int G) {
 // pairs when that is more than one) of every stream group, each on its
 // group's stream, if they do not exist yet.
 static int capture_graphs(bt_ctx* c) {
-    const int G = n_stream_groups(c);
-    int rc = ensure_group_streams(c, G);
+    const int G = n_step_groups(c);
+    int rc = ensure_group_streams(c, c->tune.streams > 1 ? G : 1);
     if (rc != BT_OK) return rc;
     auto capture = [&](int g, int npairs, hipGraph_t* gr, hipGraphExec_t* x) -> int {
-        hipStream_t st = (G > 1) ? c->gstream[g] : c->stream;
+        hipStream_t st = group_stream(c, G, g);
         HIP_TRY(c, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         for (int q = 0; q < npairs; ++q) {
             enqueue_step(c, 0, -1, G, g);
@@ -2715,29 +2797,35 @@ static int capture_graphs(bt_ctx* c) {
     return BT_OK;
 }
 
-// Replay the step graphs for `pairs` pairs of steps: tune.graph_pairs pairs
-// per launch of the long graph, single pairs for the rest. With stream groups
+// Replay the step graphs for `pairs` pairs of steps, group by group:
+// tune.graph_pairs pairs per launch of the long graph, single pairs for the rest. With stream groups
 // the other groups' streams first wait for the caller's stream, and the
 // caller's stream then waits for all of them.
 static int launch_graphs(bt_ctx* c, int pairs) {
-    const int G = n_stream_groups(c);
-    if (G > 1) {
+    const int G = n_step_groups(c);
+    const bool streams = c->tune.streams > 1;
+    if (streams) {
         HIP_TRY(c, hipEventRecord(c->ev_fork, c->stream));
         for (int g = 1; g < G; ++g) HIP_TRY(c, hipStreamWaitEvent(c->gstream[g], c->ev_fork, 0));
+    } else if (G > 1) {
+        // (a step over the whole problem flags group 0's word only)
+        hipLaunchKernelGGL(k_spread_halt, dim3(1), dim3(64), 0, c->stream, c->flags, G);
     }
     const int gp = c->tune.graph_pairs;
     for (int g = 0; g < G; ++g) {
-        hipStream_t st = (G > 1) ? c->gstream[g] : c->stream;
+        hipStream_t st = group_stream(c, G, g);
         int done = 0;
         if (c->gexec_n[g])
             for (; done + gp <= pairs; done += gp) HIP_TRY(c, hipGraphLaunch(c->gexec_n[g], st));
         for (; done < pairs; ++done) HIP_TRY(c, hipGraphLaunch(c->gexec[g], st));
     }
-    if (G > 1)
+    if (streams)
         for (int g = 1; g < G; ++g) {
             HIP_TRY(c, hipEventRecord(c->ev_join[g], c->gstream[g]));
             HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_join[g], 0));
         }
+    else if (G > 1)
+        hipLaunchKernelGGL(k_spread_halt, dim3(1), dim3(64), 0, c->stream, c->flags, G);
     return BT_OK;
 }
 
@@ -2749,7 +2837,7 @@ static int copy_back(bt_ctx* c) {
     HIP_TRY(c, hipMemcpyAsync(c->buf.vm_cell, c->vm_b, nc * 8, hipMemcpyDeviceToDevice, c->stream));
     HIP_TRY(c, hipMemcpyAsync(c->buf.c_env, c->c_env_b, ni * (size_t)c->kp.n_sq * 8, hipMemcpyDeviceToDevice,
                               c->stream));
-    if (c->tune.exchange_form == BT_EXCHANGE_FUSED)
+    if (steps_fused(c))
         HIP_TRY(c, hipMemcpyAsync(c->u, c->u_b, (size_t)c->kp.n_sq * 8, hipMemcpyDeviceToDevice, c->stream));
     return BT_OK;
 }
@@ -3061,7 +3149,6 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     }
     // the geometry as k_mem_cell reads it
     std::vector<TileRec> trec((size_t)b->n_tiles);
-    std::vector<MemRec> mrec(NM);
     for (int t = 0; t < b->n_tiles; ++t) {
         TileRec& r = trec[t];
         r.c0 = tp[t];
@@ -3074,8 +3161,6 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
         for (int q = tp[t] + 1; q < tp[t + 1]; ++q) r.starts |= 1ull << (mp[q] - r.m0 - 1);
         c->tile_nc = std::max(c->tile_nc, r.n_cells);
     }
-    for (size_t m = 0; m < NM; ++m)
-        mrec[m] = MemRec{(nnm[m] == (int32_t)m) ? (nnc[m] | MREC_BND) : nnc[m], msq[m], mpos[m], msq[nnm[m]]};
     (void)hipGetDevice(&c->device);
     const size_t nc = p->n_cells, nm = p->n_mems, ni = p->n_ions, ns = (size_t)p->n_squares;
     hipError_t e = hipSuccess;
@@ -3083,7 +3168,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
         if (e == hipSuccess) e = hipMalloc(ptr, bytes < 256 ? 256 : bytes);
     };
     alloc((void**)&c->tiles, trec.size() * sizeof(TileRec));
-    alloc((void**)&c->mrec, mrec.size() * sizeof(MemRec));
+    alloc((void**)&c->mrec, nm * sizeof(MemRec));
     alloc((void**)&c->c_cell_b, ni * nc * 8);
     alloc((void**)&c->c_lag_b, ni * nc * 8);
     alloc((void**)&c->vm_b, nc * 8);
@@ -3106,16 +3191,20 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     c->tune.mem_waves = (c->n_tiles < BT_MEM_WG_TILES) ? 2 : 1;
     c->tune.env_ions_per_block = (c->n_env_tiles < ENV_SPLIT_TILES) ? std::min(2, p->n_ions) : p->n_ions;
     c->tune.exchange_form = (c->n_live < EX_SPLIT_SQUARES) ? 0 : 1;
+    if (c->tune.exchange_form == 1 && fused_allowed(c, &c->tune)) c->tune.exchange_form = BT_EXCHANGE_FUSED;
+    c->auto_pick = true;
     c->tune.graph_pairs = BT_GRAPH_PAIRS;
     c->tune.persistent = 0;
     c->tune.streams = 1;
-    // large problems whose membrane laws read the pre-diffusion env only:
-    // the exchange in the env kernel (measured faster on the 500k-cell batch)
-    if (c->tune.exchange_form == 1 && fused_allowed(c, &c->tune)) c->tune.exchange_form = BT_EXCHANGE_FUSED;
+    c->serial_groups = pick_serial_groups(c);
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, sq_live.data(), sizeof(int32_t) * sq_live.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(c->mrec, mrec.data(), mrec.size() * sizeof(MemRec), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_mem_records, dim3(grid_blocks(p->n_mems)), dim3(BLOCK), 0, c->stream, b->nn_mem, b->nn_cell,
+                           b->mem_sq, b->mem_pos, c->mrec, p->n_mems);
+        e = hipGetLastError();
+    }
     if (e == hipSuccess) e = hipMemcpy(c->live_flag, live_flag.data(), ns, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(c->kcl, c->kcl_host.data(), sizeof(KCluster) * (size_t)n_clusters, hipMemcpyHostToDevice);
@@ -3277,6 +3366,7 @@ int bt_set_tuning(bt_ctx* c, const bt_tuning* t) {
     for (int g = 1; g < BT_MAX_STREAMS; ++g)
         if (c->gstream[g]) HIP_TRY(c, hipStreamSynchronize(c->gstream[g]));
     c->tune = *t;
+    c->auto_pick = false;
     drop_graphs(c);
     return BT_OK;
 }
@@ -3331,7 +3421,7 @@ static hipError_t state_copy(bt_ctx* c, const std::vector<std::pair<void*, size_
 int bt_capture_graphs(bt_ctx* c) {
     if (!c) return BT_EINVAL;
     bool fresh = false;
-    for (int g = 0; g < n_stream_groups(c); ++g)
+    for (int g = 0; g < n_step_groups(c); ++g)
         fresh = fresh || !c->gexec[g] || (c->tune.graph_pairs > 1 && !c->gexec_n[g]);
     int rc = capture_graphs(c);
     if (rc != BT_OK || !fresh) return rc;
@@ -3372,6 +3462,8 @@ int bt_autotune(bt_ctx* c, int32_t n_launches, bt_tuning* chosen, double* trial_
     HIP_TRY(c, hipMalloc((void**)&save, sbytes));
     hipError_t e = state_copy(c, regions, save, false);
     const bt_tuning prev = c->tune;
+    const bool prev_auto = c->auto_pick;
+    c->auto_pick = false;
     // the per-kernel trials run the three-kernel step (the fused exchange is
     // timed as whole steps below)
     bt_tuning split = prev;
@@ -3470,6 +3562,10 @@ int bt_autotune(bt_ctx* c, int32_t n_launches, bt_tuning* chosen, double* trial_
         c->tune = prev;
     }
     (void)hipFree(save);
+    if (rc != BT_OK || e != hipSuccess) {
+        c->auto_pick = prev_auto;
+        drop_graphs(c);
+    }
     if (rc != BT_OK) return rc;
     if (e != hipSuccess) return set_err(c, BT_EHIP, std::string("autotune state copy: ") + hipGetErrorString(e));
     c->tune = best;
@@ -3577,6 +3673,7 @@ int bt_set_network(bt_ctx* c, const bt_network* net, double* c_net) {
     for (int g = 1; g < BT_MAX_STREAMS; ++g)
         if (c->gstream[g]) HIP_TRY(c, hipStreamSynchronize(c->gstream[g]));
     drop_graphs(c);
+    c->serial_groups = pick_serial_groups(c);
     c->pers_grid = -1;
     if (c->tune.persistent && persistent_grid(c) < 1) c->tune.persistent = 0;
     if (!streams_allowed(c, c->tune.streams)) c->tune.streams = 1;
