@@ -93,6 +93,7 @@ struct KParams {
     double zplus[BT_MAX_IONS];      // z + 1e-25          (electroflux zc += nonce)
     double zF[BT_MAX_IONS];         // zs * p.F           (get_current)
     double zq[BT_MAX_IONS];         // z (for alpha = (D*z*q)/(kb*T))
+    double zq_kt[BT_MAX_IONS];      // (z*q)/(kb*T)
     double dgj_surf[BT_MAX_IONS];   // D_gj[i] * p.gj_surface
     double c_bound[BT_MAX_IONS];
     double dt, tm, gj_len, F, RT, RT_gj, q, kbT, cm_inv;
@@ -117,6 +118,8 @@ struct KParams {
 struct KCluster {
     int ny, nx, sq_off, pad;
     double delta, two_delta;
+    double rdl, rd2;                // 1/delta, 1/(2 delta)
+    double r_vol, r_sa, r_kee;      // 1/env_vol, 1/mean_sa, 1/kee (dv_const)
     double env_vol;                 // cell_height*delta**2
     double surf_scale;              // cell_height*delta**2 (rho_env_surf factor)
     double mean_sa, kee, screen;    // kee = ko_env*eo*er
@@ -153,6 +156,23 @@ __device__ __forceinline__ int xcd_chunk(int b, int n) {
     const int q = n / N_XCD, r = n % N_XCD;
     const int x = b % N_XCD, k = b / N_XCD;
     return (x < r) ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
+}
+
+// A value of one of the step's arrays. SC1: with agent scope, past the CU's own L1
+// (the team kernel, whose blocks read what others have written in the same launch).
+template <bool SC1, typename T>
+__device__ __forceinline__ T ld(const T* p) {
+    if constexpr (SC1) return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
+}
+
+// Tables that no kernel writes, by wave-uniform index: scalar loads also where the
+// compiler cannot see that nothing in the kernel overwrites them.
+template <typename T>
+using table = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ table<T> as_table(const T* p) {
+    return (table<T>)(uintptr_t)p;
 }
 
 __device__ __forceinline__ bool halted(const unsigned* flags) {
@@ -195,6 +215,16 @@ __device__ __forceinline__ float dv(float a, float b) {
     const float r = __builtin_amdgcn_rcpf(b);
     const float q = a * r;
     return fmaf(fmaf(-b, q, a), r, q);
+}
+
+// a / b for a constant b > 0 with r = 1/b correctly rounded on the host: the
+// product corrected once, which is the IEEE quotient (Markstein) unless the
+// quotient or the residual leaves the normal range; where the residual is no
+// number (an infinite or NaN a) the product is the quotient.
+__device__ __forceinline__ double dv_const(double a, double b, double r) {
+    const double q = a * r;
+    const double e = fma(-b, q, a);
+    return (e == e) ? fma(e, r, q) : q;
 }
 
 // exp(x) on the FP32-flux path, for |x| < 80 (the laws' exponents stay far
@@ -356,10 +386,12 @@ __device__ __forceinline__ FT dvc(FT x, double inv64, float inv32) {
     else return x * inv64;
 }
 
+// (KP, and the argument structs' types further down: a kernel's own arguments, or
+// the team kernel's in the constant address space)
+//
 // pumpNaKATP (sim_toolbox.py:71-122): returns f_Na; f_K = -(2/3)*f_Na.
-template <typename FT>
-__device__ __forceinline__ FT pump_nak(FT cNai, FT cNao, FT cKi, FT cKo, FT Vm, double nak_coef,
-                                      const KParams& P) {
+template <typename FT, typename KP>
+__device__ __forceinline__ FT pump_nak(FT cNai, FT cNao, FT cKi, FT cKo, FT Vm, double nak_coef, KP& P) {
     FT a = cNao * (FT)1e-3;
     FT b = cKi * (FT)1e-3;
     FT Qnumo = (FT)P.qn_scal * cube(a) * (b * b);
@@ -379,8 +411,8 @@ __device__ __forceinline__ FT pump_nak(FT cNai, FT cNao, FT cKi, FT cKo, FT Vm, 
 }
 
 // pumpCaATP (sim_toolbox.py:124-182) after no_negs on both concentrations.
-template <typename FT>
-__device__ __forceinline__ FT pump_ca(FT cCai, FT cCao, FT Vm, const KParams& P) {
+template <typename FT, typename KP>
+__device__ __forceinline__ FT pump_ca(FT cCai, FT cCao, FT Vm, KP& P) {
     FT Qnumo = (FT)P.qca_num * cCao;
     FT Qdenomo = (FT)P.cATP * cCai;
     if (Qdenomo == (FT)0) Qdenomo = (FT)1.0e-16;
@@ -466,7 +498,7 @@ constexpr int MREC_BND = (int)(1u << 31);
 struct MemCellArgs {
     const TileRec* tiles; const MemRec* mrec;
     const KCluster* kcl;
-    const double* mem_sa; const double* gjopen; const double* cell_vol; const double* diviterm; const double* Dm;
+    const double* mem_sa; const double* gjopen; const double* rvol; const double* diviterm; const double* Dm;
     const double* c_env;      // pre-diffusion env (membrane + NaK gathers, Q2)
     const double* c_mid;      // post-diffusion env (Ca pump and channel gathers)
     const double* c_cell_in; const double* c_lag_in; const double* vm_in;
@@ -498,6 +530,8 @@ struct MemLds {
     double* v;                // Vmem per cell (WG == 1: gj[0])
     int* start;               // [cells + 1] first membrane of each cell, within the tile
     int* bad;
+    unsigned* flags;          // where a NaN sets flag_bit
+    unsigned flag_bit;
 };
 constexpr int CHV = 6;        // a_m, b_m, a_h, b_h, modulator, cell concentration
 
@@ -517,9 +551,10 @@ __device__ __forceinline__ void tile_sync() {
     }
 }
 
-// The work of wavefront W of a k_mem_cell tile. W is a template argument so
-// that every ion index below is a compile-time constant (the per-ion kernel
-// parameters then load once, up front).
+// The work of wavefront W of a k_mem_cell tile. WT >= 0 is W at compile time, so
+// that every ion index below is a constant (the per-ion kernel parameters then
+// load once, up front); WT = -1 takes it from w (the team kernel, where one code
+// for both wavefronts is worth more).
 //
 // What bounds it is the vector-memory address unit: about 16 cycles for every
 // wavefront-wide gather, whatever it hits (measured 79 % busy with 36 loads and
@@ -531,27 +566,29 @@ __device__ __forceinline__ void tile_sync() {
 // accesses a tile where there were 51 (five ions, no channels). 53k cells on the
 // FP32-flux path 13.8 -> 11.4 us; 23k cells with two channels, two wavefronts a
 // tile, 15.2 -> 13.5 us; 105k cells with three channels 51.4 -> 50.2 us.
-template <int NI, typename FT, int WG, int W, bool OBS, bool WSYNC = false>
-__device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParams& P, int tile, const MemLds& L) {
+template <int NI, typename FT, int WG, int WT, bool OBS, bool WSYNC = false, bool SC1 = false, typename MA, typename KP>
+__device__ __forceinline__ void mem_cell_wave(MA& A, KP& P, int tile, const MemLds& L, int w = 0) {
+    const int W = WT >= 0 ? WT : w;
     constexpr int NS = (NI + WG - 1) / WG;             // ion slots per wavefront
     constexpr int NQ = (BT_MAX_CHAN + WG - 1) / WG;    // channel slots per wavefront
     constexpr int NT = TMB * WG;                       // lanes of the tile
     constexpr int NPASS = (BT_TILE_CELLS * NI + NT - 1) / NT;   // (ion, cell) items per lane, at most
-    const TileRec T = A.tiles[tile];
-    const int c0 = T.c0, m0 = T.m0, nc = T.n_cells;
+    const table<int> T = as_table(reinterpret_cast<const int*>(A.tiles + tile));    // a TileRec
+    const int c0 = T[0], m0 = T[1], nc = T[2], n_mem = T[3], inv_nc = T[5];
+    const unsigned long long starts = (unsigned)T[6] | (unsigned long long)(unsigned)T[7] << 32;
     const int j = threadIdx.x % TMB;
     const int jt = W * TMB + j;
     const int m = m0 + j;
     const int M = P.n_mems, C = P.n_cells, G2 = P.n_sq;
-    const KCluster* KC = A.kcl + T.cluster;
+    const table<KCluster> KC = as_table(A.kcl + T[4]);
     const double nak_coef = KC->nak_coef;
     const double gjo_u = KC->gjo_u;
     const unsigned still_mem = KC->still_mem;
     if (W == 0 && j == 0) {
         *L.bad = 0;
-        L.start[nc] = T.n_mems;
+        L.start[nc] = n_mem;
     }
-    const bool own_mem = j < T.n_mems;
+    const bool own_mem = j < n_mem;
     // the membrane's record first: its gathers wait for it
     MemRec R{0, 0, 0, 0};
     double sa = 0.0;
@@ -563,7 +600,7 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     const int n_items = NI * nc;
     auto item = [&](int p, int& i, int& c) {
         const int t = jt + p * NT;
-        i = (t * T.inv_nc) >> 16;
+        i = (t * inv_nc) >> 16;
         c = t - i * nc;
         return t < n_items;
     };
@@ -571,20 +608,20 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     for (int p = 0; p < NPASS; ++p) {
         if (p * NT >= n_items) break;
         int i, c;
-        if (item(p, i, c)) L.lag[i][c] = A.c_lag_in[(size_t)i * C + c0 + c];
+        if (item(p, i, c)) L.lag[i][c] = ld<SC1>(A.c_lag_in + (size_t)i * C + c0 + c);
     }
-    if (W == WG - 1 && j < nc) L.v[j] = A.vm_in[c0 + j];
+    if (W == WG - 1 && j < nc) L.v[j] = ld<SC1>(A.vm_in + c0 + j);
     const int n_chan = P.n_chan;
     if (n_chan > 0) {
         // per (channel, cell): the update coefficients of its gates (from
         // k_env_field), its modulator and its ion's concentration
         for (int t = jt; t < n_chan * CHV * nc; t += NT) {
-            const int r = (t * T.inv_nc) >> 16, c = t - r * nc;
+            const int r = (t * inv_nc) >> 16, c = t - r * nc;
             const int ch = r / CHV, k = r - ch * CHV;
             const double* src = (k < 4) ? A.rates + (size_t)(4 * ch + k) * C
                               : (k == 4) ? A.chan_mod + (size_t)ch * C
                                          : A.c_cell_in + (size_t)((P.chan_ion_pack >> (4 * ch)) & 15u) * C;
-            L.chv[r * A.chan_nc + c] = src[c0 + c];
+            L.chv[r * A.chan_nc + c] = ld<SC1>(src + c0 + c);
         }
     }
     tile_sync<WSYNC>();
@@ -593,13 +630,13 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
         const int cn = R.nn_cell & ~MREC_BND;
         const bool bnd = R.nn_cell < 0;
         const int k = R.sq;
-        const int lc = __builtin_amdgcn_mbcnt_hi((unsigned)(T.starts >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)T.starts, 0));
-        if (W == 0 && (j == 0 || ((T.starts >> (j - 1)) & 1))) L.start[lc] = j;
+        const int lc = __builtin_amdgcn_mbcnt_hi((unsigned)(starts >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)starts, 0));
+        if (W == 0 && (j == 0 || ((starts >> (j - 1)) & 1))) L.start[lc] = j;
         const double gjo = (gjo_u == gjo_u) ? gjo_u : A.gjopen[m];
         // Vmem of the membrane and of its partner: (1/cm) rho_surf of the cell
         // less Phi_b at the membrane's square (update_V, sim.py:2029)
         double v = L.v[lc];
-        double vn = A.vm_in[cn];
+        double vn = ld<SC1>(A.vm_in + cn);
         if (still_mem & PHIB_BIT) {
             v = v - A.Phi_b[k];
             vn = vn - A.Phi_b[R.nn_sq];
@@ -607,14 +644,14 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
         const bool do_nak = P.i_na >= 0 && (P.i_na / NS == W || P.i_k / NS == W);
         double nai = 0.0, nao = 0.0, ki = 0.0, ko = 0.0, cai = 0.0, cao = 0.0;
         if (do_nak) {
-            nao = A.c_env[P.i_na * G2 + k];
-            ko = A.c_env[P.i_k * G2 + k];
+            nao = ld<SC1>(A.c_env + P.i_na * G2 + k);
+            ko = ld<SC1>(A.c_env + P.i_k * G2 + k);
             nai = L.lag[P.i_na][lc];
             ki = L.lag[P.i_k][lc];
         }
         if (P.i_ca >= 0 && P.i_ca / NS == W) {
-            cai = A.c_cell_in[P.i_ca * C + c0 + lc];
-            cao = A.c_mid[P.i_ca * G2 + k];
+            cai = ld<SC1>(A.c_cell_in + P.i_ca * C + c0 + lc);
+            cao = ld<SC1>(A.c_mid + P.i_ca * G2 + k);
         }
         // the gathers of one ion slot / channel slot, issued together
         double g_env[NS], g_lagn[NS], g_dm[NS];
@@ -629,8 +666,8 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
             const bool gstill = (P.dgj_surf[i] == 0.0);
             if (do_nak && i == P.i_na) g_env[s] = nao;
             else if (do_nak && i == P.i_k) g_env[s] = ko;
-            else g_env[s] = still ? 0.0 : A.c_env[i * G2 + k];
-            g_lagn[s] = gstill ? 0.0 : A.c_lag_in[i * C + cn];
+            else g_env[s] = still ? 0.0 : ld<SC1>(A.c_env + i * G2 + k);
+            g_lagn[s] = gstill ? 0.0 : ld<SC1>(A.c_lag_in + i * C + cn);
             // (a wave-uniform choice: the cluster's value is already in SGPRs,
             // so a uniform Dm costs no load; a pointer chosen between the two
             // made every lane load, and measured 10% slower on the batch)
@@ -711,9 +748,9 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
             const int ch = W + q * WG;
             if (ch >= n_chan) break;
             const int i = P.chan_ion[ch];
-            const double h_m = A.gates[(size_t)(2 * ch) * M + m];
-            const double h_h = A.gates[(size_t)(2 * ch + 1) * M + m];
-            const double h_out = A.c_mid[i * G2 + k];
+            const double h_m = ld<SC1>(A.gates + (size_t)(2 * ch) * M + m);
+            const double h_h = ld<SC1>(A.gates + (size_t)(2 * ch + 1) * M + m);
+            const double h_out = ld<SC1>(A.c_mid + i * G2 + k);
             const double* cv = L.chv + ch * CHV * A.chan_nc + lc;
             const int cs = A.chan_nc;
             const double vg = with_nonces(v, NI + ch);
@@ -738,14 +775,14 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     // per-cell inputs of the second stage, loaded once the membrane stage is
     // done: held from the start, their registers cost a wave per SIMD of
     // occupancy (measured slower on the 500k-cell batch)
-    double cin[NPASS], vol[NPASS], divi = 0.0;
+    double cin[NPASS], rv[NPASS], divi = 0.0;
 #pragma unroll
     for (int p = 0; p < NPASS; ++p) {
         if (p * NT >= n_items) break;
         int i, c;
         if (item(p, i, c)) {
-            cin[p] = A.c_cell_in[(size_t)i * C + c0 + c];
-            vol[p] = A.cell_vol[c0 + c];
+            cin[p] = ld<SC1>(A.c_cell_in + (size_t)i * C + c0 + c);
+            rv[p] = A.rvol[c0 + c];
         }
     }
     if (W == 0 && j < nc) divi = A.diviterm[c0 + j];
@@ -763,9 +800,8 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
         int i, c;
         if (!item(p, i, c)) continue;
         const int ca = L.start[c], cb = L.start[c + 1];
-        // x / vol as the product by 1/vol (an FP64 ulp; one division per cell
-        // and ion instead of three)
-        const double rvol = 1.0 / vol[p];
+        // x / vol as the product by 1/vol (an FP64 ulp)
+        const double rvol = rv[p];
         auto per_vol = [&](double x) { return x * rvol; };
         double base = cin[p];
         if (n_chan > 0) {
@@ -809,8 +845,12 @@ __device__ __forceinline__ void mem_cell_wave(const MemCellArgs& A, const KParam
     }
     tile_sync<WSYNC>();
     if (W == 0 && j == 0 && *L.bad) {
-        atomicOr(A.flags, 1u);
-        atomicMin(A.bad_step, (unsigned long long)(*A.step_ctr));
+        if constexpr (SC1) {       // the team's barrier word; the team records the step itself
+            __hip_atomic_fetch_or(L.flags, L.flag_bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+            atomicOr(L.flags, L.flag_bit);
+            atomicMin(A.bad_step, (unsigned long long)(*A.step_ctr));
+        }
     }
 }
 
@@ -823,6 +863,14 @@ k_mem_records(const int32_t* nn_mem, const int32_t* nn_cell, const int32_t* mem_
     const int nm = nn_mem[m];
     out[m] = MemRec{nm == m ? (nn_cell[m] | MREC_BND) : nn_cell[m], mem_sq[m], mem_pos[m], mem_sq[nm]};
 }
+
+__global__ void __launch_bounds__(BLOCK) k_reciprocal(const double* x, double* out, int n) {
+    const int c = blockIdx.x * BLOCK + threadIdx.x;
+    if (c < n) out[c] = 1.0 / x[c];
+}
+
+// the barriers (tile_sync) of mem_cell_wave
+constexpr int MEM_SYNCS = 5;
 
 // LDS of one tile beyond the ions' flux rows: its channels' rows (fluxes, and
 // the per-cell values of chan_nc cells), in doubles
@@ -849,7 +897,8 @@ k_mem_cell(MemCellArgs A, KParams P) {
     __shared__ int s_start[BT_TILE_CELLS + 1];
     __shared__ int s_bad;
     const MemLds L{s_mem, s_gj, reinterpret_cast<double (*)[TMB]>(s_dyn), s_dyn + P.n_chan * TMB,
-                   WG > 1 ? reinterpret_cast<double (*)[TMB]>(s_lag) : s_mem, WG > 1 ? s_v : s_gj[0], s_start, &s_bad};
+                   WG > 1 ? reinterpret_cast<double (*)[TMB]>(s_lag) : s_mem, WG > 1 ? s_v : s_gj[0], s_start, &s_bad,
+                   A.flags, 1u};
     const int tile = xcd_chunk(blockIdx.x, gridDim.x);
     const int w = (WG > 1) ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / TMB)) : 0;
     if (w == 0) mem_cell_wave<NI, FT, WG, 0, OBS>(A, P, tile, L);
@@ -894,14 +943,14 @@ struct FieldArgs {
 // RATES: also the gating rates (diffuse mode with channels). Divisions by the
 // grid spacing and by kT are products by their FP64 reciprocals (an FP64 ulp
 // each).
-// the gate-update coefficients of item t_it = ch * n_cells + cell from the
+// the gate-update coefficients of channel ch in a cell from the
 // cell's Vmem vmc: the channel's rates at Vmem carrying the n_ions + ch
 // nonces of the membrane stage, and update_mh (channelsabc.py:54-58),
 // x' = (tau x + dt inf)/(tau + dt), as x' = a x + b with a = tau/(tau+dt),
 // b = dt*inf/(tau+dt) (FP64, an ulp from the quotient form)
-__device__ __forceinline__ void gate_coef_item(const FieldArgs& A, const KParams& P, int t_it, double vmc) {
+template <typename FA, typename KP>
+__device__ __forceinline__ void gate_coef_item(FA& A, KP& P, int ch, int cell, double vmc) {
     const int nc = P.n_cells;
-    const int ch = t_it / nc, cell = t_it - ch * nc;
     const double V = with_nonces(vmc, P.n_ions + ch) * 1000.0 + 0.0;
     double mInf, mTau, hInf, hTau;
     gate_rates(P.chan_kind[ch], V, mInf, mTau, hInf, hTau);
@@ -917,12 +966,12 @@ __device__ __forceinline__ void gate_coef_item(const FieldArgs& A, const KParams
 // sum of -x[q] over q in [a, b), added in order from a; the loads are issued
 // eight at a time (clamped to b - 1, past-the-end values unused) so one
 // square's membranes cost one memory latency instead of one each
-template <typename T, int W = 8>
+template <typename T, int W = 8, bool SC1 = false>
 __device__ __forceinline__ double neg_seg_sum(const T* x, int a, int b, double S = 0.0) {
     for (int q0 = a; q0 < b; q0 += W) {
         T t[W];
 #pragma unroll
-        for (int u = 0; u < W; ++u) t[u] = x[min(q0 + u, b - 1)];
+        for (int u = 0; u < W; ++u) t[u] = ld<SC1>(x + min(q0 + u, b - 1));
 #pragma unroll
         for (int u = 0; u < W; ++u)
             if (q0 + u < b) S = S + (-(double)t[u]);
@@ -931,12 +980,11 @@ __device__ __forceinline__ double neg_seg_sum(const T* x, int a, int b, double S
 }
 
 // row i of the membrane fluxes (FP64 or FP32), summed negated over [a, b) in
-// FP64, continuing the sum S
-template <int W = 8>
-__device__ __forceinline__ double neg_flux_sum(const void* fsa, int fsa32, size_t row, int a, int b,
-                                               double S = 0.0) {
-    return fsa32 ? neg_seg_sum<float, W>(static_cast<const float*>(fsa) + row, a, b, S)
-                 : neg_seg_sum<double, W>(static_cast<const double*>(fsa) + row, a, b, S);
+// FP64
+template <bool SC1 = false>
+__device__ __forceinline__ double neg_flux_sum(const void* fsa, int fsa32, size_t row, int a, int b) {
+    return fsa32 ? neg_seg_sum<float, 8, SC1>(static_cast<const float*>(fsa) + row, a, b)
+                 : neg_seg_sum<double, 8, SC1>(static_cast<const double*>(fsa) + row, a, b);
 }
 
 // FUSE: the membrane fluxes of FUSE_I ions of a square are summed together,
@@ -1007,6 +1055,18 @@ constexpr int ENV_A1 = (TY + 2 * ENV_UH) * (TX + 2 * ENV_UH) + ENV_VR * (TX + 2 
 constexpr int ENV_A2 = 2 * ENV_VR * ENV_VC + 2 * ENV_ER * ENV_EC;
 constexpr int ENV_POOL = ENV_A1 > ENV_A2 ? ENV_A1 : ENV_A2;
 constexpr int ENV_LDS = ENV_POOL + ENV_VR * ENV_VC + BT_MAX_IONS;
+// the same for a team block, whose four quarters each have an ion's buffers
+constexpr int TSUB = 4;
+constexpr int ENV_TEAM_POOL = TSUB * ENV_A2 > ENV_A1 ? TSUB * ENV_A2 : ENV_A1;
+constexpr int ENV_TEAM_LDS = ENV_TEAM_POOL + ENV_VR * ENV_VC + BT_MAX_IONS;
+
+// two neighbours of a row, at the alignment of one
+typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+template <bool SC1>
+__device__ __forceinline__ d2 ld_pair(const double* p) {
+    if constexpr (SC1) return d2{ld<true>(p), ld<true>(p + 1)};
+    else return *reinterpret_cast<const d2*>(p);
+}
 
 // Where a square's difference stencils read along one axis, as offsets in
 // squares from it: its neighbours L and R (itself at the world's edge) and the
@@ -1036,9 +1096,9 @@ __device__ __forceinline__ EnvAxis env_axis_inner(double rd2) {
     return EnvAxis{-1, 1, -2, 0, 0, 2, rd2, rd2, rd2};
 }
 
-// One env tile's work for the ion group ion_id of n_groups (the ions
-// [ion_id * ipb, ion_id * ipb + ipb), ipb = ceil(n_ions / n_groups)), with
-// the block's LDS at lds (ENV_LDS doubles). With RATES the block's threads also
+// One env tile's work for the ions [i_lo, i_lo + ipb) (those there are), for
+// which its tile's field is rebuilt, by thread tid of 256, with the block's LDS at
+// lds (ENV_LDS doubles). With RATES the block's threads also
 // evaluate the gating-rate items rate_first, rate_first + rate_stride, ...
 //
 // A thread owns one square. The divergence at a square needs the fluxes of its
@@ -1054,11 +1114,15 @@ __device__ __forceinline__ EnvAxis env_axis_inner(double rd2) {
 //
 // DVAR: some cluster's D_env varies over its squares (its values are staged
 // too; 20 VGPRs that a uniform D_env does without); OBS: an observed step.
-template <bool DIFFUSE, bool RATES, bool FUSE, bool DVAR, bool OBS>
-__device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams& P, int tile_id, int ion_id,
-                                               int n_groups, double* lds, int rate_first, int rate_stride,
+//
+// TEAM: a block of TSUB times 256 threads (tid over all of them): they share the
+// tile's field, then each 256 take every TSUB-th ion.
+template <bool DIFFUSE, bool RATES, bool FUSE, bool DVAR, bool OBS, bool TEAM = false, typename FA, typename KP>
+__device__ __forceinline__ void env_field_tile(FA& A, KP& P, int tile_id, int i_lo, int ipb,
+                                               int tid, double* lds, int rate_first, int rate_stride,
                                                bool check_halt = true) {
     static_assert(!FUSE || (DIFFUSE && !RATES), "the fused exchange is a diffusion step without channels");
+    static_assert(!TEAM || !FUSE, "a team's exchange is a phase of its own");
     // the halt flag is read first and tested before the first store, so its
     // latency overlaps the block's first loads (a caller that has already
     // decided for the whole block passes check_halt = false)
@@ -1066,23 +1130,21 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     constexpr int UH = ENV_UH, UR = TY + 2 * UH, UC = TX + 2 * UH;   // u on tile +- 6
     constexpr int VR = ENV_VR, VC = ENV_VC;                     // v and concentrations on tile +- 2
     constexpr int ER = ENV_ER, EC = ENV_EC;                     // D_env on tile +- 1
+    constexpr int NSUB = TEAM ? TSUB : 1, NTH = NSUB * TY * TX;
+    const int sub = TEAM ? __builtin_amdgcn_readfirstlane(tid / (TY * TX)) : 0;
+    const int st = TEAM ? tid % (TY * TX) : tid;                // thread of the 256 on its square
     double* sU = lds;                                           // [UR][UC]
     double* sT = lds + UR * UC;                                 // [VR][UC]
-    double* sV = lds + ENV_POOL;                                // [VR][VC]
+    double* sV = lds + (TEAM ? ENV_TEAM_POOL : ENV_POOL);       // [VR][VC]
     double* s_du = sV + VR * VC;
-    const int* et = A.env_tiles + 3 * tile_id;
-    const KCluster* K = A.kcl + et[0];
+    const table<int> et = as_table(A.env_tiles + 3 * tile_id);
+    const table<KCluster> K = as_table(A.kcl + et[0]);
     const int ny = K->ny, nx = K->nx, so = K->sq_off;
     const int r0 = et[1], cc0 = et[2];
-    const int tid = threadIdx.x;
-    const double rdl = 1.0 / K->delta, rd2 = 1.0 / K->two_delta;
+    const double rdl = K->rdl, rd2 = K->rd2;
     const double screen = K->screen;
     const unsigned still_mem = K->still_mem;
 
-    // ion group ion_id takes the ions [ion_id * ipb, ion_id * ipb + ipb), with
-    // ipb = ceil(n_ions / n_groups), and rebuilds its tile's field for them
-    const int ipb = (P.n_ions + n_groups - 1) / n_groups;
-    const int i_lo = ion_id * ipb;
     const int i_hi = min(i_lo + ipb, P.n_ions);
 
     // Every load the block needs first is issued here before any of them is
@@ -1093,12 +1155,12 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     const int nc = P.n_cells;
     const int items = RATES ? P.n_chan * nc : 0;
     double vm_first = 0.0;
-    if (RATES && rate_first >= 0 && rate_first < items) vm_first = A.vm[rate_first % nc];
+    if (RATES && rate_first >= 0 && rate_first < items) vm_first = ld<TEAM>(A.vm + rate_first % nc);
     double du_mine = 0.0;
     if (DIFFUSE && tid < P.n_ions) du_mine = K->denv_u[tid];
 
     static_assert(TY == 16 && TX == 16, "a thread per square of a 16 x 16 tile");
-    const int lr = tid / TX, lc = tid % TX;                // own square in the tile
+    const int lr = st / TX, lc = st % TX;                  // own square in the tile
     const int r_own = r0 + lr, c_own = cc0 + lc;
     const bool own_in = r_own < ny && c_own < nx;
     const int k_own = so + r_own * nx + c_own;
@@ -1146,10 +1208,10 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     auto on_edge = [&](int r, int cc) { return r == 0 || r == ny - 1 || cc == 0 || cc == nx - 1; };
     const int off_own = clampi(r_own, ny) * nx + clampi(c_own, nx);
     int drs, dcs;                                          // ring square of the D_env block
-    ring(min(tid, RD - 1), 1, drs, dcs);
+    ring(min(st, RD - 1), 1, drs, dcs);
     const int rd_r = r0 - 1 + drs, rd_c = cc0 - 1 + dcs;
     const int off_dring = clampi(rd_r, ny) * nx + clampi(rd_c, nx);
-    const int pt = min(tid, NP - 1);
+    const int pt = min(st, NP - 1);
     const int prow = pt / (VC / 2), pcol = 2 * (pt % (VC / 2));
     const int p_r = r0 - 2 + prow, p_c = cc0 - 2 + pcol;   // the pair's first square
     const bool pe0 = on_edge(p_r, p_c), pe1 = on_edge(p_r, p_c + 1);
@@ -1161,32 +1223,31 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // in-grid addresses (du: the cluster's D_env of the ion when it is one
     // value, no loads; NaN when it varies). What lies outside the world is
     // staged from the clamped square and never read.
-    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
     d2 tc = {0.0, 0.0};
     double td_own = 0.0, td_ring = 0.0;
     auto load_ion = [&](int i, double du) {
         const double* cenv = A.c_env + (size_t)i * P.n_sq + so;
         const double* D = A.D_env + (size_t)i * P.n_sq + so;
-        if (tid < NP) tc = *reinterpret_cast<const d2*>(cenv + off_pair);
+        if (st < NP) tc = ld_pair<TEAM>(cenv + off_pair);
         if (DVAR && !(du == du)) {
             td_own = D[off_own];
             td_ring = D[off_dring];
         }
     };
-    if (DIFFUSE && i_lo < i_hi) load_ion(i_lo, K->denv_u[i_lo]);
+    if (DIFFUSE && i_lo + sub < i_hi) load_ion(i_lo + sub, K->denv_u[i_lo + sub]);
     // u last: its loads are the only unconditional ones, so the waits for
     // them count the same on every path. Pairs of a row (cc0 - UH is even, so
     // a pair that starts left of the world lies outside it; one that ends past
     // the batch's last square reads the buffer's padding).
     static_assert(UC % 2 == 0 && UH % 2 == 0 && TX % 2 == 0, "u is staged in pairs");
     constexpr int NU = UR * UC / 2;
-    constexpr int NIT = (NU + TY * TX - 1) / (TY * TX);
+    constexpr int NIT = (NU + NTH - 1) / NTH;
     d2 t[NIT];
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int e = 2 * min(tid + it * TY * TX, NU - 1);
+        const int e = 2 * min(tid + it * NTH, NU - 1);
         const int rr = r0 - UH + e / UC, cc = cc0 - UH + e % UC;
-        t[it] = *reinterpret_cast<const d2*>(A.u + so + clampi(rr, ny) * nx + clampi(cc, nx));
+        t[it] = ld_pair<TEAM>(A.u + so + clampi(rr, ny) * nx + clampi(cc, nx));
     }
 
     // FUSE: the square's membrane-flux sums of every moving ion, taken here, all
@@ -1206,14 +1267,14 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // live beside the prefetched loads and cost occupancy.
     auto gating_rates = [&]() {
         for (int t_it = rate_first; t_it >= 0 && t_it < items; t_it += rate_stride)
-            gate_coef_item(A, P, t_it, (t_it == rate_first) ? vm_first : A.vm[t_it % nc]);
+            gate_coef_item(A, P, t_it / nc, t_it % nc, (t_it == rate_first) ? vm_first : ld<TEAM>(A.vm + t_it % nc));
     };
     if (DIFFUSE && tid < P.n_ions) s_du[tid] = du_mine;
 
     // u with zero padding outside the grid (gaussian_filter mode='constant')
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int e = 2 * (tid + it * TY * TX);
+        const int e = 2 * (tid + it * NTH);
         if (e < UR * UC) {
             const int rr = r0 - UH + e / UC, cc = cc0 - UH + e % UC;
             const bool in = rr >= 0 && rr < ny && cc >= 0;
@@ -1224,7 +1285,7 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     lds_barrier();
     // axis-0 pass (scipy correlate1d: centre tap, then pairs outermost first),
     // two rows a thread: ten LDS reads for two squares instead of nine for one
-    for (int e = tid; e < (VR / 2) * UC; e += TY * TX) {
+    for (int e = tid; e < (VR / 2) * UC; e += NTH) {
         const double* x = sU + 2 * (e / UC) * UC + e % UC;      // row -4 of the first square
         double w[10];
 #pragma unroll
@@ -1260,7 +1321,7 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     lds_barrier();
     // a halted run writes nothing (every thread read the same flag)
     if (stop) return;
-    if (FUSE && A.count_step && tile_id == 0 && ion_id == 0 && tid == 0)
+    if (FUSE && A.count_step && tile_id == 0 && i_lo == 0 && tid == 0)
         for (int g = 0; g < MAX_GROUPS; ++g)
             if (A.ctr_mask & (1u << g)) A.step_ctr[g] = A.step_ctr[g] + 1;
     const int o = (lr + 2) * VC + lc + 2;                       // own square in sV and the staged ions
@@ -1268,7 +1329,7 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
     // edges), between the squares lo and hi (LDS offsets) with the factor f
     auto vgrad = [&](int lo, int hi, double f) { return (screen * sV[o + hi] - screen * sV[o + lo]) * f; };
     if (!DIFFUSE) {
-        if (own_in) {
+        if (own_in && sub == 0) {
             const int xl = (c_own > 0) ? -1 : 0, xh = (c_own < nx - 1) ? 1 : 0;
             const int yl = (r_own > 0) ? -VC : 0, yh = (r_own < ny - 1) ? VC : 0;
             A.v_env[k_own] = sV[o];
@@ -1307,17 +1368,21 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
             gyR = vgrad(a.Rlo * VC, a.Rhi * VC, a.fR);
         }
         double rho = 0.0;               // FUSE: the square's charge over the ions, in ion order
-        for (int i = i_lo; i < i_hi; ++i) {
+        for (int r = 0; r < (TEAM ? (ipb + NSUB - 1) / NSUB : i_hi - i_lo); ++r) {
+            const int i = i_lo + r * NSUB + sub;
+            if (TEAM && i >= i_hi) {
+                lds_barrier();
+                continue;
+            }
             const double cb = P.c_bound[i];
-            const double zi = P.zq[i];
-            const double zq_kt = (zi * P.q) / P.kbT;        // alpha = D * zq_kt
-            double* sC = lds + ((i - i_lo) & 1) * (VR * VC);
-            double* sD = lds + 2 * VR * VC + ((i - i_lo) & 1) * (ER * EC);
+            const double zq_kt = P.zq_kt[i];                // alpha = D * zq_kt
+            double* sC = lds + sub * ENV_A2 + (r & 1) * (VR * VC);
+            double* sD = lds + sub * ENV_A2 + 2 * VR * VC + (r & 1) * (ER * EC);
             // concentrations of ion i (loaded one ion ahead) with the world
             // boundary reset to c_env_bound (Q3)
-            if (tid < NP) {
-                sC[2 * tid] = pe0 ? cb : (p_last ? tc.y : tc.x);
-                sC[2 * tid + 1] = pe1 ? cb : tc.y;
+            if (st < NP) {
+                sC[2 * st] = pe0 ? cb : (p_last ? tc.y : tc.x);
+                sC[2 * st + 1] = pe1 ? cb : tc.y;
             }
             // D_env zero over the cluster (block-uniform): the Nernst-Planck flux
             // is a signed zero everywhere and the update keeps the
@@ -1331,10 +1396,10 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
             const int od = (lr + 1) * EC + lc + 1;
             if (!still && !duni) {
                 sD[od] = td_own;
-                if (tid < RD) sD[drs * EC + dcs] = td_ring;
+                if (st < RD) sD[drs * EC + dcs] = td_ring;
             }
             // the next ion's loads, in flight through this ion's flux stages
-            if (i + 1 < i_hi) load_ion(i + 1, s_du[i + 1]);
+            if (i + NSUB < i_hi) load_ion(i + NSUB, s_du[i + NSUB]);
             lds_barrier();
             if (!own_in) continue;
             double cn = sC[o], ofx = 0.0, ofy = 0.0;
@@ -1377,7 +1442,7 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
                 // the exchange of k_env_exchange for this square and ion:
                 // a still ion's membrane fluxes are zeros, whose sum
                 // would add a signed zero
-                if (lv != 0 && !mstill) cn = cn + (s_sum[i * (TY * TX) + tid] / K->env_vol) * P.dt;
+                if (lv != 0 && !mstill) cn = cn + dv_const(s_sum[i * (TY * TX) + tid], K->env_vol, K->r_vol) * P.dt;
                 A.c_env_out[e] = cn;
                 rho = (i == 0) ? P.zF[0] * cn : rho + P.zF[i] * cn;
             } else if (lv != 0) {
@@ -1391,7 +1456,8 @@ __device__ __forceinline__ void env_field_tile(const FieldArgs& A, const KParams
             }
         }
         if (FUSE && own_in && live_b != 0)
-            A.u_out[k_own] = (live_b & SQ_HAS_MEM) ? ((rho * K->surf_scale) / K->mean_sa) / K->kee : 0.0;
+            A.u_out[k_own] = (live_b & SQ_HAS_MEM) ? dv_const(dv_const(rho * K->surf_scale, K->mean_sa, K->r_sa), K->kee, K->r_kee)
+                                               : 0.0;
     };
     const bool inner = r0 >= 2 && r0 + TY <= ny - 2 && cc0 >= 2 && cc0 + TX <= nx - 2;
     if (inner) ions(std::false_type{});
@@ -1407,7 +1473,9 @@ k_env_field(FieldArgs A, KParams P) {
     // (tile, ion group) from the XCD-chunked linear block index, tiles fastest
     const int lin = xcd_chunk(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int tile_id = lin % gridDim.x, ion_id = lin / gridDim.x;
-    env_field_tile<DIFFUSE, RATES, FUSE, DVAR, OBS>(A, P, tile_id, ion_id, gridDim.y, lds,
+    // ion group ion_id takes the ions [ion_id * ipb, ion_id * ipb + ipb), ipb = ceil(n_ions / gridDim.y)
+    const int ipb = (P.n_ions + gridDim.y - 1) / gridDim.y;
+    env_field_tile<DIFFUSE, RATES, FUSE, DVAR, OBS>(A, P, tile_id, ion_id * ipb, ipb, threadIdx.x, lds,
                                    (blockIdx.y * gridDim.x + blockIdx.x) * (TY * TX) + threadIdx.x,
                                    gridDim.x * gridDim.y * (TY * TX));
 }
@@ -1415,8 +1483,16 @@ k_env_field(FieldArgs A, KParams P) {
 // ---------------------------------------------------------------------------
 // k_env_exchange: membrane -> env exchange, rho_env -> surface charge
 // ---------------------------------------------------------------------------
+// A square the exchange updates, one 16-byte load: its index, its membranes'
+// range in the square-sorted order, its cluster (the sign bit set where it has no
+// surface charge).
+struct LiveRec {
+    int k, a, b, cluster;
+};
+constexpr int LIVE_NO_CHARGE = (int)(1u << 31);
+
 struct ExArgs {
-    const int32_t* sq_ptr; const uint8_t* has_mem; const int32_t* sq_cluster; const KCluster* kcl;
+    const KCluster* kcl;
     const double* c_mid; const void* fsa; const double* fch; double* c_env; double* u;
     int fsa32;                // fsa holds FP32 values (the FP32-flux path)
     // step counters: block 0 of a counted step advances step_ctr[g] for each
@@ -1425,7 +1501,7 @@ struct ExArgs {
     const unsigned* flags; long long* step_ctr; int count_step; unsigned ctr_mask;
     // the squares the exchange updates (membranes or a surface charge), ascending;
     // the others keep u = 0 and take their env state from k_env_field
-    const int32_t* sq_live; int n_live;
+    const LiveRec* sq_live; int n_live;
 };
 
 constexpr int EXQ = 64;
@@ -1439,36 +1515,28 @@ __device__ __forceinline__ void advance_step(const ExArgs& A) {
 // One wavefront per ion over EXQ squares; the charge of each square is then
 // summed over the ions in ion order from LDS.
 
-__global__ void __launch_bounds__(BT_MAX_IONS * EXQ)
-k_env_exchange(ExArgs A, KParams P) {
-    if (halted(A.flags)) return;
-    __shared__ double s_cn[BT_MAX_IONS][EXQ];
-    const int i = threadIdx.x / EXQ, j = threadIdx.x % EXQ;
-    const int q = blockIdx.x * EXQ + j;
-    if (A.count_step && blockIdx.x == 0 && threadIdx.x == 0) advance_step(A);
-    const bool live = (q < A.n_live);
-    const int k = live ? A.sq_live[q] : 0;
-    double surf_scale = 0.0, mean_sa = 1.0, kee = 1.0;
-    bool hm = false;
+template <bool SC1, typename XA, typename KP>
+__device__ __forceinline__ void exchange_chunk(XA& A, KP& P, int i, int q, bool in, int j,
+                                               double (*s_cn)[EXQ]) {
+    const bool live = in && (q < A.n_live);
+    const KCluster* K = A.kcl;
+    LiveRec R{0, 0, 0, 0};
+    if (live) R = A.sq_live[q];
+    const int k = R.k;
+    const bool hm = R.cluster >= 0;
     if (live) {
-        const int a = A.sq_ptr[k], b = A.sq_ptr[k + 1];
-        const KCluster* K = A.kcl + A.sq_cluster[k];
-        const double env_vol = K->env_vol;
-        if (i == 0) {          // the surface charge's inputs, fetched with the rest
-            surf_scale = K->surf_scale;
-            mean_sa = K->mean_sa;
-            kee = K->kee;
-            hm = A.has_mem[k] != 0;
-        }
-        double cn = A.c_mid[(size_t)i * P.n_sq + k];
+        const int a = R.a, b = R.b;
+        K += R.cluster & ~LIVE_NO_CHARGE;
+        const double env_vol = K->env_vol, r_vol = K->r_vol;
+        double cn = ld<SC1>(A.c_mid + (size_t)i * P.n_sq + k);
         const int ch = P.ion_chan[i];
         if (ch >= 0) {
-            const double Sc = neg_seg_sum(A.fch + (size_t)ch * P.n_mems, a, b);
-            cn = cn + (Sc / env_vol) * P.dt;
+            const double Sc = neg_seg_sum<double, 8, SC1>(A.fch + (size_t)ch * P.n_mems, a, b);
+            cn = cn + dv_const(Sc, env_vol, r_vol) * P.dt;
         }
         if (!((K->still_mem >> i) & 1u)) {         // a still ion's fluxes are zeros
-            const double S = neg_flux_sum(A.fsa, A.fsa32, (size_t)i * P.n_mems, a, b);
-            cn = cn + (S / env_vol) * P.dt;
+            const double S = neg_flux_sum<SC1>(A.fsa, A.fsa32, (size_t)i * P.n_mems, a, b);
+            cn = cn + dv_const(S, env_vol, r_vol) * P.dt;
         }
         A.c_env[(size_t)i * P.n_sq + k] = cn;
         s_cn[i][j] = cn;
@@ -1478,35 +1546,44 @@ k_env_exchange(ExArgs A, KParams P) {
         double rho = P.zF[0] * s_cn[0][j];
         for (int ii = 1; ii < P.n_ions; ++ii) rho = rho + P.zF[ii] * s_cn[ii][j];
         double uu = 0.0;
-        if (hm) uu = ((rho * surf_scale) / mean_sa) / kee;
+        if (hm) uu = dv_const(dv_const(rho * K->surf_scale, K->mean_sa, K->r_sa), K->kee, K->r_kee);
         A.u[k] = uu;
     }
 }
 
+__global__ void __launch_bounds__(BT_MAX_IONS * EXQ)
+k_env_exchange(ExArgs A, KParams P) {
+    if (halted(A.flags)) return;
+    __shared__ double s_cn[BT_MAX_IONS][EXQ];
+    const int i = threadIdx.x / EXQ, j = threadIdx.x % EXQ;
+    if (A.count_step && blockIdx.x == 0 && threadIdx.x == 0) advance_step(A);
+    exchange_chunk<false>(A, P, i, blockIdx.x * EXQ + j, true, j, s_cn);
+}
+
 // the exchange of the q-th square with membranes, over all ions
 __device__ __forceinline__ void exchange_square(const ExArgs& A, const KParams& P, int q) {
-    const int k = A.sq_live[q];
-    const int a = A.sq_ptr[k], b = A.sq_ptr[k + 1];
-    const KCluster& K = A.kcl[A.sq_cluster[k]];
+    const LiveRec R = A.sq_live[q];
+    const int k = R.k, a = R.a, b = R.b;
+    const KCluster& K = A.kcl[R.cluster & ~LIVE_NO_CHARGE];
     double rho = 0.0;
     for (int i = 0; i < P.n_ions; ++i) {
         double cn = A.c_mid[(size_t)i * P.n_sq + k];
         const int ch = P.ion_chan[i];
         if (ch >= 0) {
             const double Sc = neg_seg_sum(A.fch + (size_t)ch * P.n_mems, a, b);
-            cn = cn + (Sc / K.env_vol) * P.dt;
+            cn = cn + dv_const(Sc, K.env_vol, K.r_vol) * P.dt;
         }
         // a still ion's membrane fluxes are zeros: their sum would add a
         // signed zero, which leaves cn as it is
         if (!((K.still_mem >> i) & 1u)) {
             const double S = neg_flux_sum(A.fsa, A.fsa32, (size_t)i * P.n_mems, a, b);
-            cn = cn + (S / K.env_vol) * P.dt;
+            cn = cn + dv_const(S, K.env_vol, K.r_vol) * P.dt;
         }
         A.c_env[(size_t)i * P.n_sq + k] = cn;
         rho = (i == 0) ? P.zF[0] * cn : rho + P.zF[i] * cn;
     }
     double uu = 0.0;
-    if (A.has_mem[k]) uu = ((rho * K.surf_scale) / K.mean_sa) / K.kee;
+    if (R.cluster >= 0) uu = dv_const(dv_const(rho * K.surf_scale, K.mean_sa, K.r_sa), K.kee, K.r_kee);
     A.u[k] = uu;
 }
 
@@ -2083,142 +2160,314 @@ k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, u
 }
 
 // ---------------------------------------------------------------------------
-// k_step_persistent: many steps in one cooperative launch
+// k_step_team: many steps in one launch, a team of blocks per XCD
 // ---------------------------------------------------------------------------
-// Each step's three dependent phases (env field + diffusion, membranes and
-// cells, exchange) run in one launch whose blocks all stay resident
-// (hipLaunchCooperativeKernel) and meet at a grid barrier between phases: the
-// per-launch drain and ramp of the three-kernel step are gone, and a launch
-// runs any even number of steps. Work is dealt out in grid-stride order: env
-// (tile, ion group) items per block, cell tiles per wavefront (each wavefront
-// owns one tile at a time, with the membrane kernel's single-wavefront form),
-// squares with membranes per thread.
-constexpr int PB = 256;                      // threads per persistent block
-constexpr int PW = PB / TMB;                 // wavefronts per persistent block
-#ifndef PERSIST_WAVES_PER_SIMD
-#define PERSIST_WAVES_PER_SIMD 4             // occupancy the register budget is held to
-#endif
-constexpr unsigned BT_FLAG_BARRIER = 2u;     // flags bit: a grid barrier gave up waiting
-constexpr unsigned BARRIER_SPINS = 1u << 24; // about a second of s_sleep before it gives up
+// A small problem's step is three launches each of which lasts one wavefront's
+// latency chain plus 2-3 us of launch and drain, with every value a kernel
+// reads last written on another XCD, past its L2. Here a slot of clusters (all
+// of a single cluster; at most eight slots of a batch, about equal) is stepped by
+// the blocks of ONE XCD, whose 32 CUs share an L2: a barrier between phases is
+// then an L2 atomic and takes about 1 us for 32 blocks, and the state stays in
+// that L2 from step to step. (A barrier over all XCDs took 2.8 us at best, 5-80
+// us with the fences that write L2 back.)
+//
+// Coherence: stores write through to the XCD's L2; what other blocks of the team
+// have written in this launch is loaded with agent scope (ld<true>), which
+// passes by the CU's own L1. Geometry and constants are plain loads.
+//
+// Teams form at run time, so nothing depends on where blocks are placed or on
+// all of them being resident: a block registers with its XCD (read from the
+// hardware); the first to do so claims a slot and, once the expected number has
+// registered or 30 us have passed, closes the team; later blocks leave. Only
+// blocks of a closed team ever wait for each other, all of them running. With
+// its slot done a team claims the next. A wait of about a second sets
+// BT_FLAG_BARRIER and the block leaves.
+//
+// One block is one CU's 16 wavefronts. Phases of a step: environment (a block per
+// env tile and ion group, its quarters sharing the ions) and membranes (one or two
+// wavefronts per cell tile), side by side where no membrane law reads the
+// post-diffusion env, else one after the other; then the exchange (a wavefront
+// per ion over 64 squares).
+constexpr int TB = 1024;                     // threads per block
+constexpr int TW = TB / TMB;                 // wavefronts per block
+static_assert(TB == TSUB * TY * TX, "a block's quarters are env tiles' threads");
+constexpr int TEAM_BLOCKS = 32;              // blocks of a full team: the CUs of an XCD
+constexpr unsigned BT_FLAG_BARRIER = 2u;     // flags bit: a team barrier gave up waiting
+constexpr unsigned TEAM_STOP = 1u << 31;     // barrier word's bit: a NaN in the slot
+constexpr unsigned TEAM_CLOSED = 1u << 31;   // registration word's bit
+constexpr unsigned TEAM_NONE = ~0u;          // team size word: no slot left, leave
+constexpr unsigned TEAM_SPINS = 1u << 22;    // polls (over a second) before a wait gives up
+constexpr int TEAM_STEPS = 1 << 12;          // steps per launch: even, and a team that formed short of blocks is soon re-formed
 
-struct PersistArgs {
-    FieldArgs field[2];                      // by step parity
-    MemCellArgs mem[2];
-    ExArgs ex[2];
-    unsigned* bar;                           // [0] arrivals, [1] generation
-    int n_env_tiles, n_groups, n_tiles, n_steps;
+struct TeamCtl {
+    unsigned reg, size, slot, pad0[29];      // registered blocks; blocks of the closed team; its slot
+    unsigned bar, pad1[31];                  // barrier arrivals since the launch, and TEAM_STOP
+};
+struct TeamCtls {
+    TeamCtl team[16];                        // by XCD
+    unsigned next_slot, pad[31];
 };
 
-// LDS of one membrane-phase wavefront, in doubles: flux*sa and GJ flux per ion,
-// the channels' rows, the cells' first membranes and the tile's NaN flag
-template <int NI, bool CHAN>
-constexpr int mem_wave_lds() {
-    return 2 * NI * TMB + (CHAN ? mem_chan_lds(BT_MAX_CHAN, BT_TILE_CELLS) : 0) + (BT_TILE_CELLS + 3) / 2;
+// A slot's share of the work lists, its cells and its squares.
+struct TeamSlot {
+    int t0, nt, e0, ne, l0, nl, c0, c1, k0, k1;
+};
+
+struct TeamArgs {
+    FieldArgs field[2];                      // by step parity: from the caller's buffers to the workspace, and back
+    MemCellArgs mem[2];
+    ExArgs ex[2];
+    const TeamSlot* slots; int n_slots;
+    TeamCtls* ctl; TeamCtls* ctl_next;       // this launch's words (zero); the next launch's, zeroed here
+    int n_groups;                            // ion groups of the env phase
+    int n_blocks;                            // blocks expected per XCD
+    int split;                               // two wavefronts per cell tile, else one
+    int mem_slots;                           // cell tiles of a block at a time
+    int env_blocks;                          // of a full team, where the phases run side by side
+    int n_steps;
+    long long step0;                         // index of the first step
+    int ordered;                             // the membrane laws read the post-diffusion env
+    KParams P;
+};
+
+__device__ __forceinline__ unsigned agent_load(const unsigned* p) {
+    return __hip_atomic_load(const_cast<unsigned*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Grid barrier of a cooperative launch. Thread 0 of each block reads the
-// generation, arrives, and the last arrival resets the count and opens the next
-// generation; the others wait for it. The agent-scope fences make every block's
-// global writes before the barrier visible to every block after it (across the
-// XCDs' L2 caches). A wait that exceeds BARRIER_SPINS sets BT_FLAG_BARRIER and
-// the block goes on, so every wave reaches the end of the kernel whatever
-// happens. Returns false once the flag is set.
-__device__ __forceinline__ bool grid_sync(unsigned* bar, unsigned* flags) {
-    __shared__ int s_ok;
+// LDS of the team kernel, in doubles: the env sub-blocks', the membrane
+// wavefronts' (flux rows, channel rows, the cells' first membranes and the NaN
+// flag) or the exchange's, whichever is largest
+__host__ __device__ constexpr int team_wave_lds(int ni, int n_chan, int chan_nc, bool split) {
+    return 2 * ni * TMB + mem_chan_lds(n_chan, chan_nc) + (split ? ni * TMB + BT_TILE_CELLS : 0) + (BT_TILE_CELLS + 3) / 2;
+}
+__host__ __device__ constexpr int team_lds(int ni, int n_chan, int chan_nc, int mem_slots, bool split) {
+    int n = ENV_TEAM_LDS;
+    const int m = mem_slots * team_wave_lds(ni, n_chan, chan_nc, split);
+    if (m > n) n = m;
+    if (TW * EXQ > n) n = TW * EXQ;
+    return n;
+}
+
+// Barrier of a team of n blocks (target: arrivals that complete it, counted from
+// the launch): this block's stores are in L2 when it arrives. Returns the
+// barrier word, or 0 after a wait that gave up.
+__device__ __forceinline__ unsigned team_sync(TeamCtl* T, unsigned target, unsigned* flags, unsigned* s_word) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
-        int ok = 1;
-        __threadfence();
-        const unsigned gen = __hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (atomicAdd(&bar[0], 1u) == gridDim.x - 1) {
-            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __threadfence();
-            atomicAdd(&bar[1], 1u);
-        } else {
-            unsigned spins = 0;
-            while (__hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-                __builtin_amdgcn_s_sleep(2);
-                if (++spins > BARRIER_SPINS) {
-                    atomicOr(flags, BT_FLAG_BARRIER);
-                    break;
-                }
+        // (workgroup scope: carried out in the XCD's L2, where the whole team sees
+        // it; with agent scope it goes to memory, 1.7 us a barrier instead of 0.9)
+        __hip_atomic_fetch_add(&T->bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        unsigned w = 0, spins = 0;
+        for (;;) {
+            w = agent_load(&T->bar);
+            if ((w & ~TEAM_STOP) >= target) break;
+            if (++spins > TEAM_SPINS) {
+                atomicOr(flags, BT_FLAG_BARRIER);
+                w = 0;
+                break;
             }
         }
-        __threadfence();
-        if (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & BT_FLAG_BARRIER) ok = 0;
-        s_ok = ok;
+        *s_word = w;
     }
     __syncthreads();
-    return s_ok != 0;
+    return *s_word;
 }
 
-template <int NI, typename FT, bool RATES>
-__global__ void __launch_bounds__(PB, PERSIST_WAVES_PER_SIMD)
-k_step_persistent(PersistArgs PA, KParams P) {
-    constexpr int MW = mem_wave_lds<NI, RATES>();
-    constexpr int LDS = ENV_LDS > PW * MW ? ENV_LDS : PW * MW;
-    __shared__ double lds[LDS];
-    __shared__ int s_stop;
-    const int nb = gridDim.x;
-    const int wave = threadIdx.x / TMB;
-    const int gtid = blockIdx.x * PB + threadIdx.x;
-    const int nthr = nb * PB;
-    const int n_env_items = PA.n_env_tiles * PA.n_groups;
-    // this wavefront's slice of the LDS in the membrane phase
-    double* wl = lds + wave * MW;
-    int* wi = reinterpret_cast<int*>(wl + MW - (BT_TILE_CELLS + 3) / 2);
-    const MemLds L{reinterpret_cast<double (*)[TMB]>(wl), reinterpret_cast<double (*)[TMB]>(wl + NI * TMB),
-                   reinterpret_cast<double (*)[TMB]>(wl + 2 * NI * TMB), wl + (2 * NI + P.n_chan) * TMB,
-                   reinterpret_cast<double (*)[TMB]>(wl), wl + NI * TMB, wi, wi + BT_TILE_CELLS + 1};
-    // one step of parity PAR (a compile-time index into the argument sets);
-    // false once a grid barrier gave up
-    auto step = [&](auto par_c) -> bool {
-        constexpr int par = decltype(par_c)::value;
-        const FieldArgs& FA = PA.field[par];
-        // phase A: env field and diffusion (and the gating coefficients). The
-        // flags change only in the membrane phase, so one read decides for the block.
-        if (threadIdx.x == 0) s_stop = halted(FA.flags) ? 1 : 0;
-        lds_barrier();
-        if (!s_stop) {
-            for (int it = blockIdx.x; it < n_env_items; it += nb) {
-                const int item = (nb % N_XCD == 0) ? xcd_chunk(it, n_env_items) : it;
-                env_field_tile<true, false, false, true, false>(FA, P, item % PA.n_env_tiles, item / PA.n_env_tiles, PA.n_groups, lds,
-                                            -1, 0, false);
-                lds_barrier();
-            }
-            if (RATES) {
-                const int items = P.n_chan * P.n_cells;
-                for (int t_it = gtid; t_it < items; t_it += nthr) gate_coef_item(FA, P, t_it, FA.vm[t_it % P.n_cells]);
+// The arguments stay in the kernel-argument segment and each phase reads what it
+// uses there, through a pointer the compiler cannot see through: held in
+// registers over the step loop they spilled 700 SGPRs to vector lanes, and each
+// phase moved them back one by one.
+template <int NI, typename FT, bool CHAN>
+__global__ void __launch_bounds__(TB)
+k_step_team(TeamArgs) {
+    extern __shared__ double lds[];
+    __shared__ unsigned s_word;
+    __shared__ int s_rank, s_size, s_slot;
+    auto args = [] {
+        table<TeamArgs> p = (table<TeamArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    const int tid = threadIdx.x;
+    // HW_REG_XCC_ID (register 20), 4 bits
+    const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | 20);
+    TeamCtl* const T = args()->ctl->team + xcd;
+    unsigned* const flags = args()->mem[0].flags;
+    const int n_slots = args()->n_slots, n_blocks = args()->n_blocks;
+    if (blockIdx.x == 0)
+        for (int i = tid; i < (int)(sizeof(TeamCtls) / sizeof(unsigned)); i += TB)
+            reinterpret_cast<unsigned*>(args()->ctl_next)[i] = 0u;
+    if (tid == 0) {
+        int size = 0;
+        const unsigned t = atomicAdd(&T->reg, 1u);
+        if (!(t & TEAM_CLOSED)) {
+            if (t == 0) {
+                const unsigned slot = halted(flags) ? TEAM_NONE : atomicAdd(&args()->ctl->next_slot, 1u);
+                if (slot >= (unsigned)n_slots) {
+                    atomicOr(&T->reg, TEAM_CLOSED);
+                    __hip_atomic_store(&T->size, TEAM_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    const unsigned long long t0 = wall_clock64();      // 100 MHz
+                    while (agent_load(&T->reg) < (unsigned)n_blocks && wall_clock64() - t0 < 3000ull) {}
+                    size = (int)atomicOr(&T->reg, TEAM_CLOSED);
+                    __hip_atomic_store(&T->slot, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    __hip_atomic_store(&T->size, (unsigned)size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            } else {
+                unsigned m = 0, spins = 0;
+                while ((m = agent_load(&T->size)) == 0 && ++spins < TEAM_SPINS) {}
+                if (m == 0) atomicOr(flags, BT_FLAG_BARRIER);
+                size = (m == 0 || m == TEAM_NONE) ? 0 : (int)m;
             }
         }
-        if (!grid_sync(PA.bar, PA.mem[par].flags)) return false;
-        // phase B: membranes and cells, one tile per wavefront at a time; the
-        // halt check is uniform over the wavefront
-        {
-            const MemCellArgs& MA = PA.mem[par];
-            const bool stop = __builtin_amdgcn_readfirstlane(halted(MA.flags) ? 1 : 0) != 0;
-            if (!stop) {
-                const int nw = nb * PW;
-                for (int w = blockIdx.x * PW + wave; w < PA.n_tiles; w += nw) {
-                    mem_cell_wave<NI, FT, 1, 0, false, true>(MA, P, w, L);
+        s_rank = (int)(t & ~TEAM_CLOSED);
+        s_size = size;
+        s_slot = size ? (int)agent_load(&T->slot) : -1;
+    }
+    __syncthreads();
+    const int rank = __builtin_amdgcn_readfirstlane(s_rank), nb = __builtin_amdgcn_readfirstlane(s_size);
+    if (nb == 0) return;
+    int slot = __builtin_amdgcn_readfirstlane(s_slot);
+    unsigned target = 0;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TMB), lane = tid % TMB;
+
+    while (slot >= 0 && slot < n_slots) {
+        const table<TeamSlot> S = as_table(args()->slots + slot);
+        const int n_steps = args()->n_steps;
+        // side by side, the env phase takes the team's first blocks and the
+        // membrane phase the others
+        const bool ordered = args()->ordered != 0, side = !ordered && nb > 1;
+        const int eb = side ? min(max(nb * args()->env_blocks / n_blocks, 1), nb - 1) : nb;
+        const int mb = side ? nb - eb : nb;
+        auto env_phase = [&](int par) {
+            const table<TeamArgs> TA = args();
+            const int e0 = S->e0, ne = S->ne, n_env = ne * TA->n_groups;
+            const int ipb = (TA->P.n_ions + TA->n_groups - 1) / TA->n_groups;
+            if (rank < eb)
+                for (int it = rank; it < n_env; it += eb) {
+                    env_field_tile<true, false, false, true, false, true>(TA->field[par], TA->P, e0 + it % ne, (it / ne) * ipb,
+                                                                          ipb, tid, lds, -1, 0, false);
+                    lds_barrier();
+                }
+            if (CHAN) {
+                // the gating coefficients of the slot's cells
+                const int c0 = S->c0, cells = S->c1 - c0, items = TA->P.n_chan * cells;
+                for (int t = rank * TB + tid; t < items; t += nb * TB) {
+                    const int ch = t / cells, c = c0 + (t - ch * cells);
+                    gate_coef_item(TA->field[par], TA->P, ch, c, ld<true>(TA->field[par].vm + c));
+                }
+            }
+        };
+        auto mem_phase = [&](int par) {
+            const int b = nb - 1 - rank;
+            if (b >= mb) return;
+            const table<TeamArgs> TA = args();
+            // the LDS of a cell tile: a slice for each wavefront, or for each two (split)
+            constexpr int MR = NI * TMB;
+            const bool split = TA->split != 0;
+            const int n_chan = TA->P.n_chan, chan_nc = TA->mem[0].chan_nc, mem_slots = TA->mem_slots;
+            const int t0 = S->t0, nt = S->nt;
+            const int mslot = split ? wave / 2 : wave, mhalf = wave & 1;
+            double* const wl = lds + mslot * team_wave_lds(NI, n_chan, chan_nc, split);
+            double* const wc = wl + 2 * MR;                            // channel rows
+            double* const wv = wc + mem_chan_lds(n_chan, chan_nc);     // split: lagged rows, Vmem
+            int* const wi = reinterpret_cast<int*>(wv + (split ? MR + BT_TILE_CELLS : 0));
+            const MemLds L{reinterpret_cast<double (*)[TMB]>(wl), reinterpret_cast<double (*)[TMB]>(wl + MR),
+                           reinterpret_cast<double (*)[TMB]>(wc), wc + n_chan * TMB,
+                           reinterpret_cast<double (*)[TMB]>(split ? wv : wl), split ? wv + MR : wl + MR, wi,
+                           wi + BT_TILE_CELLS + 1, &T->bar, TEAM_STOP};
+            if (split) {
+                // every wavefront of the block passes every barrier of a round
+                for (int q0 = b; q0 < nt; q0 += mb * mem_slots) {
+                    const int t = q0 + mslot * mb;
+                    if (mslot < mem_slots && t < nt)
+                        mem_cell_wave<NI, FT, 2, -1, false, false, true>(TA->mem[par], TA->P, t0 + t, L, mhalf);
+                    else
+                        for (int q = 0; q < MEM_SYNCS; ++q) lds_barrier();
+                    lds_barrier();
+                }
+            } else if (mslot < mem_slots) {
+                for (int t = b + mslot * mb; t < nt; t += mb * mem_slots) {
+                    mem_cell_wave<NI, FT, 1, 0, false, true, true>(TA->mem[par], TA->P, t0 + t, L);
                     tile_sync<true>();
                 }
             }
-        }
-        if (!grid_sync(PA.bar, PA.mem[par].flags)) return false;
-        // phase C: the exchange of the squares with membranes; the step counter
-        {
-            const ExArgs& XA = PA.ex[par];
-            if (!halted(XA.flags)) {
-                if (gtid == 0) advance_step(XA);
-                for (int q = gtid; q < XA.n_live; q += nthr) exchange_square(XA, P, q);
+        };
+        auto exchange_phase = [&](int par) {
+            const table<TeamArgs> TA = args();
+            constexpr int per_block = TW / NI;
+            const int l0 = S->l0, nl = S->nl, n_chunks = (nl + EXQ - 1) / EXQ;
+            const int q = wave / NI, i = wave - q * NI;
+            for (int c0 = rank; c0 < n_chunks; c0 += nb * per_block) {
+                const int k = (c0 + q * nb) * EXQ + lane;
+                exchange_chunk<true>(TA->ex[par], TA->P, i, l0 + k, q < per_block && k < nl, lane,
+                                     reinterpret_cast<double (*)[EXQ]>(lds + (q < per_block ? q : 0) * NI * EXQ));
+                lds_barrier();
             }
+        };
+        unsigned word = 1;
+        int s = 0;
+        for (; s < n_steps; ++s) {
+            const int par = s & 1;
+            env_phase(par);
+            if (ordered) {
+                word = team_sync(T, target += nb, flags, &s_word);
+                if (word == 0) return;
+            } else if (!side) {
+                lds_barrier();
+            }
+            mem_phase(par);
+            word = team_sync(T, target += nb, flags, &s_word);
+            if (word == 0) return;
+            if (word & TEAM_STOP) break;
+            exchange_phase(par);
+            word = team_sync(T, target += nb, flags, &s_word);
+            if (word == 0) return;
         }
-        return grid_sync(PA.bar, PA.mem[par].flags);
-    };
-    for (int s = 0; s < PA.n_steps; s += 2) {
-        if (!step(std::integral_constant<int, 0>{})) break;
-        if (!step(std::integral_constant<int, 1>{})) break;
+        const table<TeamArgs> TA = args();
+        if (word & TEAM_STOP) {
+            if (rank == 0 && tid == 0) {
+                atomicOr(flags, 1u);
+                atomicMin(TA->mem[0].bad_step, (unsigned long long)(TA->step0 + s));
+            }
+        } else {
+            // v_env and E of the state
+            const int ne = S->ne;
+            for (int it = rank; it < ne; it += nb) {
+                env_field_tile<false, false, false, false, false, true>(TA->field[0], TA->P, S->e0 + it, 0, 0, tid, lds, -1, 0,
+                                                                        false);
+                lds_barrier();
+            }
+            if (slot == 0 && rank == 0 && tid < MAX_GROUPS)
+                const_cast<long long*>(TA->mem[0].step_ctr)[tid] = TA->step0 + n_steps;
+        }
+        if (n_steps & 1) {
+            // the state from the workspace to the caller's buffers (halted or not,
+            // as after replayed steps)
+            auto back = [&](double* dst, const double* src, int lo, int hi) {
+                for (int k = lo + rank * TB + tid; k < hi; k += nb * TB) dst[k] = ld<true>(src + k);
+            };
+            const int c0 = S->c0, c1 = S->c1, k0 = S->k0, k1 = S->k1;
+            for (int i = 0; i < TA->P.n_ions; ++i) {
+                const size_t ro = (size_t)i * TA->P.n_cells, rs = (size_t)i * TA->P.n_sq;
+                back(TA->mem[1].c_cell_out + ro, TA->mem[1].c_cell_in + ro, c0, c1);
+                back(TA->mem[1].c_lag_out + ro, TA->mem[1].c_lag_in + ro, c0, c1);
+                back(TA->field[1].c_env_out + rs, TA->field[1].c_env + rs, k0, k1);
+            }
+            back(TA->mem[1].vm_out, TA->mem[1].vm_in, c0, c1);
+        }
+        // the next slot, claimed by the team's first block
+        if (rank == 0 && tid == 0) {
+            const unsigned next = atomicAdd(&TA->ctl->next_slot, 1u);
+            __hip_atomic_store(&T->slot, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        word = team_sync(T, target += nb, flags, &s_word);
+        if (word == 0 || (word & TEAM_STOP)) return;
+        if (tid == 0) s_slot = (int)min(agent_load(&T->slot), 0x7fffffffu);
+        __syncthreads();
+        slot = __builtin_amdgcn_readfirstlane(s_slot);
     }
 }
 
@@ -2242,12 +2491,13 @@ struct bt_ctx {
     int tile_nc = 0;                // cells of the largest tile
     // workspace
     TileRec* tiles = nullptr; MemRec* mrec = nullptr;   // the geometry as k_mem_cell reads it
+    double* rvol = nullptr;         // 1 / cell_vol
     double* c_cell_b = nullptr; double* c_lag_b = nullptr; double* vm_b = nullptr;
     double* c_mid = nullptr; void* fsa = nullptr; double* fch = nullptr; double* u = nullptr;
     double* u_b = nullptr;    // surface charge of odd steps with the fused exchange
     double* rates = nullptr;  // [n_chan][4][n_cells] gating rates of the current step
     double* c_env_b = nullptr;           // env state of odd steps
-    int32_t* sq_live = nullptr;          // squares the exchange updates, ascending
+    LiveRec* sq_live = nullptr;          // squares the exchange updates, ascending
     uint8_t* live_flag = nullptr;        // per square: SQ_LIVE if in sq_live, SQ_HAS_MEM
     int n_live = 0;
     unsigned* flags = nullptr; unsigned long long* bad_step = nullptr; long long* step_ctr = nullptr;
@@ -2272,8 +2522,11 @@ struct bt_ctx {
     // exchange into the env kernel wherever that is allowed
     bool auto_pick = false;
     bool autotuned = false;
-    unsigned* bar = nullptr;           // grid barrier of the persistent step kernel
-    int pers_grid = -1;                // its cooperative grid (-1 not yet known, 0 unavailable)
+    // team kernel: the slots of clusters, and two sets of control words, one for
+    // a launch and one that it leaves zeroed for the next
+    std::vector<TeamSlot> slots_host;
+    TeamSlot* slots = nullptr; TeamCtls* ctl = nullptr; int ctl_at = 0;
+    bool team_fits = false;            // small enough for the team kernel to be the faster one
     long long steps_done = 0;
     const bt_obs* capture = nullptr;   // set while enqueueing an observed step
     // observables workspace (allocated on first use)
@@ -2331,6 +2584,7 @@ static void derive_params(const bt_params& p, KParams& k) {
         k.zplus[i] = p.z[i] + FLOAT_NONCE;
         k.zF[i] = p.z[i] * p.F;
         k.zq[i] = p.z[i];
+        k.zq_kt[i] = (p.z[i] * p.q) / (p.kb * p.T);
         k.dgj_surf[i] = p.d_gj[i] * p.gj_surface;
         k.c_bound[i] = p.c_bound[i];
     }
@@ -2377,6 +2631,8 @@ static KCluster derive_cluster(const bt_params& p, const bt_cluster& b) {
     k.surf_scale = p.cell_height * (b.delta * b.delta);
     k.mean_sa = b.mean_sa;
     k.kee = (b.ko_env * p.eo) * p.er;
+    k.rdl = 1.0 / k.delta; k.rd2 = 1.0 / k.two_delta;
+    k.r_vol = 1.0 / k.env_vol; k.r_sa = 1.0 / k.mean_sa; k.r_kee = 1.0 / k.kee;
     k.screen = (2.0 / (b.ko_env * b.delta)) * (p.cell_radius / p.true_cell_size);
     k.nak_coef = -3.0 * p.NaK_block * b.alpha_NaK;
     for (int i = 0; i < BT_MAX_IONS; ++i) k.dm_u[i] = k.denv_u[i] = NAN;
@@ -2391,7 +2647,6 @@ static KCluster derive_cluster(const bt_params& p, const bt_cluster& b) {
 constexpr int BT_MEM_WG_TILES = 3000;
 constexpr int BT_GRAPH_PAIRS = 8;
 constexpr int BT_MAX_GRAPH_PAIRS = 64;
-constexpr int BT_PERSIST_STEPS = 512;   // steps per cooperative launch of the persistent kernel (even)
 constexpr int BT_AUTOTUNE_TRIALS = 13;
 
 // A stream group's share of the step's work lists: its cell tiles [t0, t0 +
@@ -2522,12 +2777,12 @@ static StepArgs step_args(bt_ctx* c, int parity, const bt_obs* ob, int count_ste
     double* eo = parity ? B.c_env : c->c_env_b;
     StepArgs a{field_args(c, true, ob, vi, ei, eo),
                MemCellArgs{c->tiles, c->mrec, c->kcl,
-                           B.mem_sa, B.gjopen, B.cell_vol, B.diviterm, B.Dm, ei, c->c_mid,
+                           B.mem_sa, B.gjopen, c->rvol, B.diviterm, B.Dm, ei, c->c_mid,
                            ci, li, vi, co, lo, vo, c->fsa, B.gates, B.chan_mod, c->rates, c->fch,
                            c->flags, c->bad_step, c->step_ctr,
                            ob ? ob->fluxes_mem : nullptr, ob ? ob->fluxes_gj : nullptr,
                            ob ? ob->chan_flux : nullptr, ob ? ob->rate_NaKATP : nullptr, B.Phi_b, c->tile_nc},
-               ExArgs{B.sq_ptr, B.sq_has_mem, B.sq_cluster, c->kcl, c->c_mid, c->fsa, c->fch, eo, c->u,
+               ExArgs{c->kcl, c->c_mid, c->fsa, c->fch, eo, c->u,
                       c->prm.flux_mode == BT_FLUX_FP32 ? 1 : 0, c->flags,
                       c->step_ctr, count_step, (1u << MAX_GROUPS) - 1u, c->sq_live, c->n_live}};
     if (fused) {
@@ -2618,91 +2873,84 @@ static void enqueue_step(bt_ctx* c, int parity, int which = -1, int G = 1, int g
                            c->bad_step, (const long long*)c->step_ctr, which < 0 ? 1 : 0);
 }
 
-// The persistent step kernel of this problem, or nullptr where it has no
-// instantiation: five or six ions, no reaction network (the network keeps its
-// own kernel).
-static const void* persistent_kernel(bt_ctx* c) {
+// The team kernel of this problem, or nullptr where it has no instantiation: five
+// or six ions, no reaction network (the network keeps its own kernel).
+static const void* team_kernel(const bt_ctx* c) {
     if (c->net && c->c_net) return nullptr;
     const bool f32 = c->prm.flux_mode == BT_FLUX_FP32;
-    const bool rates = c->prm.n_chan > 0;
+    const bool chan = c->prm.n_chan > 0;
     switch (c->prm.n_ions) {
         case 5:
-            if (f32) return rates ? (const void*)&k_step_persistent<5, float, true> : (const void*)&k_step_persistent<5, float, false>;
-            return rates ? (const void*)&k_step_persistent<5, double, true> : (const void*)&k_step_persistent<5, double, false>;
+            if (f32) return chan ? (const void*)&k_step_team<5, float, true> : (const void*)&k_step_team<5, float, false>;
+            return chan ? (const void*)&k_step_team<5, double, true> : (const void*)&k_step_team<5, double, false>;
         case 6:
-            if (f32) return rates ? (const void*)&k_step_persistent<6, float, true> : (const void*)&k_step_persistent<6, float, false>;
-            return rates ? (const void*)&k_step_persistent<6, double, true> : (const void*)&k_step_persistent<6, double, false>;
+            if (f32) return chan ? (const void*)&k_step_team<6, float, true> : (const void*)&k_step_team<6, float, false>;
+            return chan ? (const void*)&k_step_team<6, double, true> : (const void*)&k_step_team<6, double, false>;
         default:
             return nullptr;
     }
 }
 
-// blocks of a cooperative launch of the persistent kernel: as many as stay
-// resident together (0 where the kernel or cooperative launches are unavailable)
-static int persistent_grid(bt_ctx* c) {
-    if (c->pers_grid >= 0) return c->pers_grid;
-    c->pers_grid = 0;
-    const void* k = persistent_kernel(c);
-    int coop = 0, cus = 0, per_cu = 0;
-    if (!k || hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
-        return 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus < 1)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, PB, 0) != hipSuccess || per_cu < 1) return 0;
-    // what stays resident by LDS, counted apart with each block's LDS rounded up
-    // to 2 KB of the CU's 160 KB: the query divides the exact sizes, the
-    // hardware hands out larger granules, and one block too many never arrives
-    // at the grid barrier
-    hipFuncAttributes fa;
-    if (hipFuncGetAttributes(&fa, k) != hipSuccess) return 0;
-    per_cu = std::min(per_cu, (int)(160 * 1024 / std::max<size_t>((fa.sharedSizeBytes + 2047) / 2048 * 2048, 2048)));
-    if (per_cu < 1) return 0;
-    c->pers_grid = per_cu * cus;
-    return c->pers_grid;
-}
-
-// The blocks a persistent launch uses: as many as the largest phase has work
-// items for (env (tile, ion group) items, cell tiles at PW per block, squares
-// with membranes and (channel, cell) gating items at PB per block), rounded up
-// to a multiple of the XCD count, and at most what stays resident. Every block
-// arrives at each grid barrier, so a small problem waits on few arrivals.
-static int persistent_launch_grid(bt_ctx* c) {
-    const int cap = persistent_grid(c);
-    if (cap < 1) return cap;
-    const long long groups = (c->prm.n_ions + c->tune.env_ions_per_block - 1) / c->tune.env_ions_per_block;
-    long long need = (long long)c->n_env_tiles * groups;
-    need = std::max(need, (long long)(c->n_tiles + PW - 1) / PW);
-    need = std::max(need, (long long)(c->n_live + PB - 1) / PB);
-    need = std::max(need, ((long long)c->prm.n_chan * c->prm.n_cells + PB - 1) / PB);
-    need = ((std::max(need, 1LL) + N_XCD - 1) / N_XCD) * N_XCD;
-    return (int)std::min<long long>(need, cap);
-}
-
-// n_steps (even) steps in cooperative launches of the persistent kernel
-static int launch_persistent(bt_ctx* c, int n_steps) {
-    const void* k = persistent_kernel(c);
-    const int grid = persistent_launch_grid(c);
-    if (!k || grid < 1) return set_err(c, BT_EINVAL, "no persistent step kernel for this problem");
-    PersistArgs pa;
+// n_steps steps, v_env and E of the last, and the state in the caller's buffers,
+// in launches of the team kernel
+static int launch_team(bt_ctx* c, int n_steps) {
+    const void* k = team_kernel(c);
+    if (!k) return set_err(c, BT_EINVAL, "no persistent step kernel for this problem");
+    TeamArgs ta;
     for (int par = 0; par < 2; ++par) {
-        const StepArgs a = step_args(c, par, nullptr, 1);
-        pa.field[par] = a.field;
-        pa.mem[par] = a.mem;
-        pa.ex[par] = a.ex;
+        const StepArgs a = step_args(c, par, nullptr, 0);
+        ta.field[par] = a.field;
+        ta.mem[par] = a.mem;
+        ta.ex[par] = a.ex;
     }
-    pa.bar = c->bar;
-    pa.n_env_tiles = c->n_env_tiles;
-    pa.n_groups = (c->prm.n_ions + c->tune.env_ions_per_block - 1) / c->tune.env_ions_per_block;
-    pa.n_tiles = c->n_tiles;
-    for (int done = 0; done < n_steps;) {
-        // at most BT_PERSIST_STEPS steps per launch
-        pa.n_steps = std::min(n_steps - done, BT_PERSIST_STEPS);
-        HIP_TRY(c, hipMemsetAsync(c->bar, 0, 2 * sizeof(unsigned), c->stream));
-        void* args[] = {(void*)&pa, (void*)&c->kp};
-        HIP_TRY(c, hipLaunchCooperativeKernel(k, dim3(grid), dim3(PB), args, 0, c->stream));
-        done += pa.n_steps;
+    ta.P = c->kp;
+    ta.slots = c->slots;
+    ta.n_slots = (int)c->slots_host.size();
+    ta.ordered = (c->prm.n_chan > 0 || c->kp.i_ca >= 0) ? 1 : 0;
+    int ne = 1, nt = 1;
+    for (const TeamSlot& q : c->slots_host) {
+        ne = std::max(ne, q.ne);
+        nt = std::max(nt, q.nt);
+    }
+    const int ni = c->prm.n_ions;
+    // Blocks by the largest slot's work: an env (tile, ion group) item each, and
+    // cell tiles two to a block while there are blocks for that (a CU's 16
+    // wavefronts share four SIMDs: fewer of them finish sooner).
+    const int avail = ta.ordered ? TEAM_BLOCKS : TEAM_BLOCKS / 2;
+    ta.n_groups = std::max(1, std::min(ni, avail / ne));
+    const int want_env = ne * ta.n_groups, want_mem = (nt + 1) / 2;
+    if (ta.ordered) {
+        ta.n_blocks = std::min(TEAM_BLOCKS, std::max(2, std::max(want_env, want_mem)));
+        ta.env_blocks = ta.n_blocks;
+    } else {
+        ta.n_blocks = std::min(TEAM_BLOCKS, std::max(2, want_env + want_mem));
+        ta.env_blocks = want_env <= TEAM_BLOCKS / 2
+                            ? want_env
+                            : std::max(1, std::min(ta.n_blocks - 1, (int)((long long)ta.n_blocks * 5 * ne / (5 * ne + nt))));
+    }
+    const int mem_blocks = ta.ordered ? ta.n_blocks : ta.n_blocks - ta.env_blocks;
+    // two wavefronts per tile while the tiles fit at once
+    ta.split = (nt <= mem_blocks * (TW / 2)) ? 1 : 0;
+    const size_t per = (size_t)team_wave_lds(ni, c->prm.n_chan, c->tile_nc, ta.split != 0) * sizeof(double);
+    ta.mem_slots = (int)std::min<size_t>(ta.split ? TW / 2 : TW, (159 * 1024) / per);
+    const size_t lds = (size_t)team_lds(ni, c->prm.n_chan, c->tile_nc, ta.mem_slots, ta.split != 0) * sizeof(double);
+    HIP_TRY(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    for (int done = 0; done < n_steps; done += ta.n_steps) {
+        ta.n_steps = std::min(n_steps - done, TEAM_STEPS);
+        ta.step0 = c->steps_done + done;
+        ta.ctl = c->ctl + c->ctl_at;
+        c->ctl_at ^= 1;
+        ta.ctl_next = c->ctl + c->ctl_at;
+        void* args[] = {(void*)&ta};
+        HIP_TRY(c, hipLaunchKernel(k, dim3(N_XCD * ta.n_blocks), dim3(TB), args, lds, c->stream));
     }
     return BT_OK;
+}
+
+// whether bt_step runs its steps in the team kernel
+static bool use_team(const bt_ctx* c) {
+    if (!c->auto_pick) return c->tune.persistent != 0;
+    return c->team_fits && team_kernel(c) != nullptr;
 }
 
 static void drop_graphs(bt_ctx* c) {
@@ -3133,6 +3381,56 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
         }
     }
     {
+        // the team kernel's slots: contiguous clusters, at most one slot per XCD,
+        // the largest slot as small as that allows (all in one slot where the work
+        // lists are not in cluster order)
+        const int nq = n_clusters;
+        if (c->cl_tile0.empty()) {
+            c->slots_host.push_back(TeamSlot{0, b->n_tiles, 0, c->n_env_tiles, 0, (int)sq_live.size(), 0, p->n_cells, 0,
+                                             p->n_squares});
+        } else {
+            // a cluster's cost: its cell tiles and env tiles (about equal times)
+            auto cost = [&](int q) {
+                return c->cl_tile0[q + 1] - c->cl_tile0[q] + 4 * (c->cl_env0[q + 1] - c->cl_env0[q]);
+            };
+            auto slots_at = [&](long long cap, std::vector<int>* ends) {
+                int n = 1;
+                long long sum = 0;
+                for (int q = 0; q < nq; ++q) {
+                    if (sum > 0 && sum + cost(q) > cap) {
+                        ++n;
+                        sum = 0;
+                        if (ends) ends->push_back(q);
+                    }
+                    sum += cost(q);
+                }
+                if (ends) ends->push_back(nq);
+                return n;
+            };
+            long long lo = 0, hi = 0;
+            for (int q = 0; q < nq; ++q) {
+                lo = std::max<long long>(lo, cost(q));
+                hi += cost(q);
+            }
+            while (lo < hi) {
+                const long long mid = (lo + hi) / 2;
+                if (slots_at(mid, nullptr) <= N_XCD) hi = mid;
+                else lo = mid + 1;
+            }
+            std::vector<int> ends;
+            slots_at(lo, &ends);
+            int qa = 0;
+            for (int qz : ends) {
+                const int k1 = cl[qz - 1].sq_off + cl[qz - 1].grid_ny * cl[qz - 1].grid_nx;
+                c->slots_host.push_back(TeamSlot{c->cl_tile0[qa], c->cl_tile0[qz] - c->cl_tile0[qa], c->cl_env0[qa],
+                                                 c->cl_env0[qz] - c->cl_env0[qa], c->cl_live0[qa],
+                                                 c->cl_live0[qz] - c->cl_live0[qa], (int)c->cl_cell0[qa],
+                                                 (int)c->cl_cell0[qz], cl[qa].sq_off, k1});
+                qa = qz;
+            }
+        }
+    }
+    {
         // each cluster's membrane range, for the per-cluster constants
         c->cl_mem_lo.assign(n_clusters, p->n_mems);
         c->cl_mem_hi.assign(n_clusters, 0);
@@ -3147,7 +3445,10 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
             return set_err(nullptr, rc, msg);
         }
     }
-    // the geometry as k_mem_cell reads it
+    // the geometry as the exchange and k_mem_cell read it
+    std::vector<LiveRec> lrec;
+    lrec.reserve(sq_live.size());
+    for (const int32_t k : sq_live) lrec.push_back(LiveRec{k, sp[k], sp[k + 1], sqc[k] | (hm[k] ? 0 : LIVE_NO_CHARGE)});
     std::vector<TileRec> trec((size_t)b->n_tiles);
     for (int t = 0; t < b->n_tiles; ++t) {
         TileRec& r = trec[t];
@@ -3169,6 +3470,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     };
     alloc((void**)&c->tiles, trec.size() * sizeof(TileRec));
     alloc((void**)&c->mrec, nm * sizeof(MemRec));
+    alloc((void**)&c->rvol, nc * 8);
     alloc((void**)&c->c_cell_b, ni * nc * 8);
     alloc((void**)&c->c_lag_b, ni * nc * 8);
     alloc((void**)&c->vm_b, nc * 8);
@@ -3181,11 +3483,12 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     alloc((void**)&c->flags, 256);
     alloc((void**)&c->bad_step, 256);
     alloc((void**)&c->step_ctr, 256);
-    alloc((void**)&c->bar, 256);
+    alloc((void**)&c->ctl, 2 * sizeof(TeamCtls));
+    alloc((void**)&c->slots, c->slots_host.size() * sizeof(TeamSlot));
     alloc((void**)&c->kcl, sizeof(KCluster) * (size_t)n_clusters);
     alloc((void**)&c->env_tiles, sizeof(int) * tiles.size());
     alloc((void**)&c->c_env_b, ni * ns * 8);
-    alloc((void**)&c->sq_live, sizeof(int32_t) * (sq_live.empty() ? 1 : sq_live.size()));
+    alloc((void**)&c->sq_live, sizeof(LiveRec) * (lrec.empty() ? 1 : lrec.size()));
     alloc((void**)&c->live_flag, ns);
     c->n_live = (int)sq_live.size();
     c->tune.mem_waves = (c->n_tiles < BT_MEM_WG_TILES) ? 2 : 1;
@@ -3198,11 +3501,13 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     c->tune.streams = 1;
     c->serial_groups = pick_serial_groups(c);
     if (e == hipSuccess && !sq_live.empty())
-        e = hipMemcpy(c->sq_live, sq_live.data(), sizeof(int32_t) * sq_live.size(), hipMemcpyHostToDevice);
+        e = hipMemcpy(c->sq_live, lrec.data(), sizeof(LiveRec) * lrec.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_mem_records, dim3(grid_blocks(p->n_mems)), dim3(BLOCK), 0, c->stream, b->nn_mem, b->nn_cell,
                            b->mem_sq, b->mem_pos, c->mrec, p->n_mems);
+        hipLaunchKernelGGL(k_reciprocal, dim3(grid_blocks(p->n_cells)), dim3(BLOCK), 0, c->stream, b->cell_vol, c->rvol,
+                           p->n_cells);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(c->live_flag, live_flag.data(), ns, hipMemcpyHostToDevice);
@@ -3212,7 +3517,9 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     if (e == hipSuccess) e = hipMemsetAsync(c->flags, 0, 256, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->bad_step, 0xff, 256, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->step_ctr, 0, 256, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(c->bar, 0, 256, c->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->ctl, 0, 2 * sizeof(TeamCtls), c->stream);
+    if (e == hipSuccess)
+        e = hipMemcpy(c->slots, c->slots_host.data(), c->slots_host.size() * sizeof(TeamSlot), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemsetAsync(c->u, 0, ns * 8, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->u_b, 0, ns * 8, c->stream);    // u of squares without membranes
     if (e == hipSuccess) e = hipMemsetAsync(c->fsa, 0, (ni * nm + FSA_PAD) * 8, c->stream);   // still rows stay zero
@@ -3237,9 +3544,9 @@ int bt_destroy(bt_ctx* c) {
         if (c->ev_join[g]) (void)hipEventDestroy(c->ev_join[g]);
     }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
-    void* ptrs[] = {c->tiles, c->mrec, c->c_cell_b, c->c_lag_b, c->vm_b, c->c_mid, c->fsa, c->fch, c->u, c->u_b, c->rates, c->c_env_b,
+    void* ptrs[] = {c->tiles, c->mrec, c->rvol, c->c_cell_b, c->c_lag_b, c->vm_b, c->c_mid, c->fsa, c->fch, c->u, c->u_b, c->rates, c->c_env_b,
                     c->sq_live, c->live_flag, c->flags, c->bad_step, c->step_ctr, c->kcl, c->env_tiles,
-                    c->vm_prev, c->net, c->bar, c->phib_stage, c->phib_prev};
+                    c->vm_prev, c->net, c->ctl, c->slots, c->phib_stage, c->phib_prev};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (void* q : c->obs_alloc) (void)hipFree(q);
@@ -3305,12 +3612,14 @@ int bt_step(bt_ctx* c, int32_t n_steps, int32_t use_graph) {
         }
         return bt_step(c, n_steps - 1, use_graph);
     }
-    int pairs = n_steps / 2;
-    if (c->tune.persistent && pairs > 0) {
-        // every pair of steps in cooperative launches of the persistent kernel
-        int rc = launch_persistent(c, 2 * pairs);
+    if (use_team(c)) {
+        int rc = launch_team(c, n_steps);
         if (rc != BT_OK) return rc;
-    } else if (use_graph && pairs > 0) {
+        c->steps_done += n_steps;
+        return BT_OK;
+    }
+    int pairs = n_steps / 2;
+    if (use_graph && pairs > 0) {
         // a graph of tune.graph_pairs pairs of steps for the bulk, one of a
         // single pair for the rest; both are captured and instantiated on the
         // first call that replays graphs, so later calls only launch them
@@ -3355,9 +3664,9 @@ int bt_set_tuning(bt_ctx* c, const bt_tuning* t) {
     if (t->graph_pairs < 1 || t->graph_pairs > BT_MAX_GRAPH_PAIRS)
         return set_err(c, BT_EINVAL, "graph_pairs must be in 1..64");
     if (t->persistent != 0 && t->persistent != 1) return set_err(c, BT_EINVAL, "persistent must be 0 or 1");
-    if (t->persistent && persistent_grid(c) < 1)
-        return set_err(c, BT_EINVAL, "no persistent step kernel for this problem (it needs 5 or 6 ions, no "
-                                     "reaction network, and cooperative launches)");
+    if (t->persistent && !team_kernel(c))
+        return set_err(c, BT_EINVAL, "no persistent step kernel for this problem (it needs 5 or 6 ions and no "
+                                     "reaction network)");
     if (t->streams < 1 || t->streams > BT_MAX_STREAMS) return set_err(c, BT_EINVAL, "streams must be in 1..4");
     if (t->streams > 1 && !streams_allowed(c, t->streams))
         return set_err(c, BT_EINVAL, "stream groups need at least that many clusters, work lists in cluster order, "
@@ -3519,7 +3828,7 @@ int bt_autotune(bt_ctx* c, int32_t n_launches, bt_tuning* chosen, double* trial_
             fused_t.env_ions_per_block = c->prm.n_ions;
             for (const Whole& w : cands) {
                 if (rc != BT_OK || e != hipSuccess) break;
-                if (w.persistent && persistent_grid(c) < 1) continue;
+                if (w.persistent && !team_kernel(c)) continue;
                 if (!streams_allowed(c, w.streams)) continue;
                 if (w.fused && !fused_allowed(c, &fused_t)) continue;
                 c->tune = w.fused ? fused_t : best;
@@ -3674,8 +3983,7 @@ int bt_set_network(bt_ctx* c, const bt_network* net, double* c_net) {
         if (c->gstream[g]) HIP_TRY(c, hipStreamSynchronize(c->gstream[g]));
     drop_graphs(c);
     c->serial_groups = pick_serial_groups(c);
-    c->pers_grid = -1;
-    if (c->tune.persistent && persistent_grid(c) < 1) c->tune.persistent = 0;
+    if (c->tune.persistent && !team_kernel(c)) c->tune.persistent = 0;
     if (!streams_allowed(c, c->tune.streams)) c->tune.streams = 1;
     return BT_OK;
 }

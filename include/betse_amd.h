@@ -236,9 +236,10 @@ typedef struct {
                                    adds each square's membrane fluxes to its diffused value (needs no channels, no
                                    Ca pump and env_ions_per_block = n_ions) */
     int32_t graph_pairs;        /* pairs of steps per replayed step graph, 1..64 */
-    int32_t persistent;         /* 1: bt_step runs its pairs of steps in cooperative launches of one persistent
-                                   kernel (grid barriers between a step's phases; 5 or 6 ions, no reaction
-                                   network); 0: replayed step graphs */
+    int32_t persistent;         /* 1: bt_step runs its steps in launches of one persistent kernel, in which the
+                                   blocks of each XCD form a team that steps a share of the clusters (barriers
+                                   between a step's phases within the XCD; 5 or 6 ions, no reaction network);
+                                   0: replayed step graphs */
     int32_t streams;            /* 1..BT_MAX_STREAMS: with replayed graphs, the clusters of a batch are split
                                    into this many groups of about equal cells, each stepped by its own graphs
                                    on its own stream, so that one group's kernels run in the ramps and tails of
