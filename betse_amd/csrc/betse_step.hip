@@ -33,6 +33,9 @@
 //                   in each of four wavefronts that split the rates:
 //                   the substances' explicit Euler update (networks.py:2805-2982)
 //
+// Small problems run whole calls of steps in one launch (k_step_team): the blocks of
+// each XCD step a share of the clusters, with barriers within the XCD.
+//
 // The env state ping-pongs between the caller's c_env and a workspace copy, like
 // the cell state, since k_env_field reads neighbours that other blocks update.
 //
@@ -2197,6 +2200,17 @@ constexpr unsigned TEAM_STOP = 1u << 31;     // barrier word's bit: a NaN in the
 constexpr unsigned TEAM_CLOSED = 1u << 31;   // registration word's bit
 constexpr unsigned TEAM_NONE = ~0u;          // team size word: no slot left, leave
 constexpr unsigned TEAM_SPINS = 1u << 22;    // polls (over a second) before a wait gives up
+// The work of a slot, in cell tiles (an env tile costs about four), up to which the
+// team kernel is the default. us per step, team against replayed graphs (FP64):
+//   plain     4 cell + 1 env tiles   9.1 / 15.8     145 + 16  12.3 / 16.2
+//             61 + 16               10.9 / 15.9     226 + 25  17.7 / 16.1
+//             8 clusters of 200-400 cells 10.8 / 16.1, 32 of 60-200 13.7 / 17.9,
+//             64 of 60-200 18.5 / 16.6
+//   ordered   4 + 1                 15.1 / 19.6     61 + 9    19.4 / 20.3
+//   (channels or a Ca pump)         37 + 16 18.8 / 19.5   61 + 16 20.6 / 19.9
+// Beyond, one XCD's 32 CUs have more to do than eight times as many save.
+constexpr int TEAM_TILES = 220;
+constexpr int TEAM_TILES_ORDERED = 100;
 constexpr int TEAM_STEPS = 1 << 12;          // steps per launch: even, and a team that formed short of blocks is soon re-formed
 
 struct TeamCtl {
@@ -2527,6 +2541,7 @@ struct bt_ctx {
     std::vector<TeamSlot> slots_host;
     TeamSlot* slots = nullptr; TeamCtls* ctl = nullptr; int ctl_at = 0;
     bool team_fits = false;            // small enough for the team kernel to be the faster one
+    bool team_warm = false;            // it has been launched
     long long steps_done = 0;
     const bt_obs* capture = nullptr;   // set while enqueueing an observed step
     // observables workspace (allocated on first use)
@@ -3429,6 +3444,10 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
                 qa = qz;
             }
         }
+        const bool ordered = p->n_chan > 0 || p->i_ca >= 0;
+        c->team_fits = true;
+        for (const TeamSlot& q : c->slots_host)
+            c->team_fits = c->team_fits && q.nt + 4 * q.ne <= (ordered ? TEAM_TILES_ORDERED : TEAM_TILES);
     }
     {
         // each cluster's membrane range, for the per-cluster constants
@@ -3613,10 +3632,17 @@ int bt_step(bt_ctx* c, int32_t n_steps, int32_t use_graph) {
         return bt_step(c, n_steps - 1, use_graph);
     }
     if (use_team(c)) {
-        int rc = launch_team(c, n_steps);
-        if (rc != BT_OK) return rc;
-        c->steps_done += n_steps;
-        return BT_OK;
+        // (a captured launch would be replayed on control words that are not its
+        // own: under the caller's capture the steps are separate launches)
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(c, hipStreamIsCapturing(c->stream, &cap));
+        if (cap == hipStreamCaptureStatusNone) {
+            int rc = launch_team(c, n_steps);
+            if (rc != BT_OK) return rc;
+            c->steps_done += n_steps;
+            return BT_OK;
+        }
+        use_graph = 0;
     }
     int pairs = n_steps / 2;
     if (use_graph && pairs > 0) {
@@ -3729,10 +3755,12 @@ static hipError_t state_copy(bt_ctx* c, const std::vector<std::pair<void*, size_
 
 int bt_capture_graphs(bt_ctx* c) {
     if (!c) return BT_EINVAL;
-    bool fresh = false;
-    for (int g = 0; g < n_step_groups(c); ++g)
+    // (steps that run in the team kernel replay no graphs: it is launched once)
+    const bool team = use_team(c);
+    bool fresh = team && !c->team_warm;
+    for (int g = 0; g < n_step_groups(c) && !team; ++g)
         fresh = fresh || !c->gexec[g] || (c->tune.graph_pairs > 1 && !c->gexec_n[g]);
-    int rc = capture_graphs(c);
+    int rc = team ? BT_OK : capture_graphs(c);
     if (rc != BT_OK || !fresh) return rc;
     // replay each graph once from a saved copy of the state and put the state
     // back: the first launch of an instantiated graph carries one-time costs
@@ -3745,7 +3773,8 @@ int bt_capture_graphs(bt_ctx* c) {
     HIP_TRY(c, hipMalloc((void**)&save, sbytes));
     hipError_t e = state_copy(c, regions, save, false);
     if (e == hipSuccess) {
-        rc = launch_graphs(c, c->tune.graph_pairs > 1 ? c->tune.graph_pairs + 1 : 1);
+        rc = team ? launch_team(c, 2) : launch_graphs(c, c->tune.graph_pairs > 1 ? c->tune.graph_pairs + 1 : 1);
+        c->team_warm = c->team_warm || (team && rc == BT_OK);
         if (rc == BT_OK) e = state_copy(c, regions, save, true);
     }
     (void)hipFree(save);

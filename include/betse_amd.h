@@ -239,7 +239,8 @@ typedef struct {
     int32_t persistent;         /* 1: bt_step runs its steps in launches of one persistent kernel, in which the
                                    blocks of each XCD form a team that steps a share of the clusters (barriers
                                    between a step's phases within the XCD; 5 or 6 ions, no reaction network);
-                                   0: replayed step graphs */
+                                   0: replayed step graphs, or the persistent kernel where a context's tuning has
+                                   been left alone and the clusters are small */
     int32_t streams;            /* 1..BT_MAX_STREAMS: with replayed graphs, the clusters of a batch are split
                                    into this many groups of about equal cells, each stepped by its own graphs
                                    on its own stream, so that one group's kernels run in the ramps and tails of
@@ -278,6 +279,7 @@ int bt_stage_boundary(bt_ctx* ctx, const double* Phi_b_next);
 
 /* Capture and instantiate the step graphs now (bt_step otherwise does it on
  * its first call that replays graphs), so that no later bt_step pays for it.
+ * Where bt_step runs in the persistent kernel, that is launched once instead.
  * Newly captured graphs are also replayed once from a saved copy of the state,
  * which is then put back (bit for bit), so that their first launch's one-time
  * costs fall here too. Allocates the copy for the duration of the call. */
