@@ -187,6 +187,16 @@ SIGNATURES = {
     "bt_gnn_mse": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int64, ctypes.c_float, _vp, _vp, ctypes.c_int32, _vp]),
     "bt_gnn_adam": (ctypes.c_int, [_vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_float, ctypes.c_float,
                                    ctypes.c_float, ctypes.c_float, ctypes.c_int32, _vp]),
+    "bt_gnn_adam_all": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, ctypes.c_int32, ctypes.c_float, ctypes.c_float,
+                                       ctypes.c_float, ctypes.c_float, ctypes.c_int32, _vp]),
+    "bt_gnn_layered": (ctypes.c_int, [ctypes.c_int32] * 4),
+    "bt_gnn_cache_len": (ctypes.c_int64, [ctypes.c_int32] * 4),
+    "bt_gnn_backward_len": (ctypes.c_int64, [ctypes.c_int32] * 5),
+    "bt_gnn_forward": (ctypes.c_int, [_vp] + [ctypes.c_int32] * 4 + [_vp, _vp, _vp, ctypes.c_int32, _vp,
+                                                                     ctypes.c_int32, _vp, _vp]),
+    "bt_gnn_backward": (ctypes.c_int, [_vp] + [ctypes.c_int32] * 4 + [_vp, _vp, _vp, ctypes.c_int32, _vp,
+                                                                      ctypes.c_int32, _vp, _vp, _vp, ctypes.c_int64,
+                                                                      _vp]),
 }
 
 _lib: Optional[ctypes.CDLL] = None

@@ -63,6 +63,11 @@ class WarmStartGNN:
             self.v = {k: torch.zeros_like(v) for k, v in self.params.items()}
         self.t = 0
         self._ws = None
+        # parameter names in the order of the whole-pass entry points
+        self._names = (["W_in", "b_in"] + [f"{k}{l}" for l in range(n_layers) for k in "Wb"] + ["W_out", "b_out"])
+        # a kernel per layer where there is one for these sizes, else products
+        # and elementwise calls
+        self._layered = bool(self.lib.bt_gnn_layered(f_in, f_out, hidden, n_layers))
 
     # ------------------------------------------------------------------
     def _s(self):
@@ -76,6 +81,9 @@ class WarmStartGNN:
         torch = self.torch
         with torch.cuda.device(self.device), torch.cuda.stream(self.stream):
             return torch.empty(shape, dtype=torch.float32, device=self.device)
+
+    def _pointers(self, tensors):
+        return (_vp * len(tensors))(*[t.data_ptr() for t in tensors])
 
     def _workspace(self, n: int):
         need = max(n * max(self.H, self.f_out), 64 * 2 * self.H * self.H, 1 << 16)
@@ -104,6 +112,15 @@ class WarmStartGNN:
         """X: (n, f_in) float32; ptr/idx: int32 CSR of the symmetric neighbour graph."""
         n, H = X.shape[0], self.H
         P = self.params
+        if self._layered and n * H < 1 << 30:
+            cache = self._empty(self.lib.bt_gnn_cache_len(H, self.L, n, int(keep)))
+            y = self._empty(n, self.f_out)
+            self._chk(self.lib.bt_gnn_forward(self._pointers([P[k] for k in self._names]), self.f_in, self.f_out, H,
+                                              self.L, _p(X), _p(ptr), _p(idx), n, _p(cache), int(keep), _p(y),
+                                              self._s()), "forward")
+            if keep:
+                self._cache = {"X": X, "n": n, "layers": cache}
+            return y
         z0 = self._empty(n, H)
         h = self._empty(n, H)
         self.gemm(X, self.f_in, 1, P["W_in"], H, 1, z0, H, n, H, self.f_in)
@@ -142,6 +159,15 @@ class WarmStartGNN:
         c = self._cache
         n, H, fo = dY.shape[0], self.H, self.f_out
         P = self.params
+        if "layers" in c:
+            sizes = [P[k].numel() for k in P]
+            g = {k: t.view(P[k].shape) for k, t in zip(P, self._empty(sum(sizes)).split(sizes))}
+            ws = self._empty(self.lib.bt_gnn_backward_len(self.f_in, fo, H, self.L, n))
+            self._chk(self.lib.bt_gnn_backward(self._pointers([P[k] for k in self._names]), self.f_in, fo, H, self.L,
+                                               _p(c["X"]), _p(ptr), _p(idx), n, _p(c["layers"]), c["n"], _p(dY),
+                                               self._pointers([g[k] for k in self._names]), _p(ws), ws.numel(),
+                                               self._s()), "backward")
+            return g
         g = {k: self._empty(*v.shape) for k, v in P.items()}
         hL = c[f"h{self.L}"]
         self.gemm(hL, 1, H, dY, fo, 1, g["W_out"], fo, H, fo, n)            # h_L^T dY
@@ -168,10 +194,11 @@ class WarmStartGNN:
 
     def adam(self, grads, lr: float = 1e-3, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8) -> None:
         self.t += 1
-        for k, p in self.params.items():
-            self._chk(self.lib.bt_gnn_adam(_p(p), _p(grads[k]), _p(self.m[k]), _p(self.v[k]), p.numel(),
-                                           ctypes.c_float(lr), ctypes.c_float(b1), ctypes.c_float(b2),
-                                           ctypes.c_float(eps), self.t, self._s()), "adam")
+        names = list(self.params)
+        ptrs = [self._pointers([d[k] for k in names]) for d in (self.params, grads, self.m, self.v)]
+        counts = (ctypes.c_int64 * len(names))(*[self.params[k].numel() for k in names])
+        self._chk(self.lib.bt_gnn_adam_all(*ptrs, counts, len(names), ctypes.c_float(lr), ctypes.c_float(b1),
+                                           ctypes.c_float(b2), ctypes.c_float(eps), self.t, self._s()), "adam")
 
     def params_np(self) -> Dict[str, np.ndarray]:
         self.stream.synchronize()

@@ -432,6 +432,29 @@ int bt_gnn_mse(const float* Y, const float* T, const float* mask, int64_t count,
 int bt_gnn_adam(float* p, const float* g, float* m, float* v, int64_t count, float lr, float b1, float b2,
                 float eps, int32_t t, void* stream);
 
+/* bt_gnn_adam on several tensors (counts[q] elements each). */
+int bt_gnn_adam_all(float* const* p, const float* const* g, float* const* m, float* const* v, const int64_t* counts,
+                    int32_t n_tensors, float lr, float b1, float b2, float eps, int32_t t, void* stream);
+/* Whole passes of the network, a kernel per layer: bit for bit the results of
+ * the calls above composed layer by layer. bt_gnn_layered: 1 where they exist
+ * (hidden 16, 32 or 64, f_out <= 16, f_in <= 128, n_layers 1..15), else 0 and
+ * the passes return BT_EINVAL, as they do for n * hidden >= 2^30. params and grads (host arrays of device
+ * pointers): W_in, b_in, then W and b of each layer, then W_out, b_out.
+ * ptr/idx: neighbour CSR (symmetric for the backward pass).
+ * bt_gnn_forward leaves in cache (bt_gnn_cache_len floats, 16-byte aligned),
+ * with keep, what the backward pass reads; n nodes of f_in features in, n of
+ * f_out in y. bt_gnn_backward reads the first n of the cache's cache_n nodes
+ * and writes every gradient; ws: bt_gnn_backward_len floats, 16-byte aligned. */
+int bt_gnn_layered(int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers);
+int64_t bt_gnn_cache_len(int32_t hidden, int32_t n_layers, int32_t n, int32_t keep);
+int64_t bt_gnn_backward_len(int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers, int32_t n);
+int bt_gnn_forward(const float* const* params, int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers,
+                   const float* X, const int32_t* ptr, const int32_t* idx, int32_t n, float* cache, int32_t keep,
+                   float* y, void* stream);
+int bt_gnn_backward(const float* const* params, int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers,
+                    const float* X, const int32_t* ptr, const int32_t* idx, int32_t n, const float* cache,
+                    int32_t cache_n, const float* dY, float* const* grads, float* ws, int64_t ws_len, void* stream);
+
 /* Wait for the stream; return BT_OK or BT_UNSTABLE (a NaN was produced; the
  * state is frozen at the step that produced it and *bad_step receives its
  * 0-based index counted from context creation, or -1). With streams > 1
