@@ -2145,12 +2145,15 @@ __global__ void __launch_bounds__(64) k_spread_halt(unsigned* flags, int G) {
     if (__ballot(f != 0u) && threadIdx.x < MAX_GROUPS) flags[threadIdx.x] = f | 1u;
 }
 
-// per-cluster max over cells and ions of |c - c_prev| / |c| (init residual)
+// Per-cluster max over cells and ions of |c - c_prev| / |c| (init residual). A
+// wavefront whose cells are one cluster's reduces them before its atomic: with one
+// per cell a cluster's cells queued on its word, 169 us for 60k cells of 48 clusters,
+// now 15 us.
 __global__ void __launch_bounds__(BLOCK)
 k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, unsigned long long* rmax,
            int n_cells, int n_ions) {
-    const int cidx = blockIdx.x * BLOCK + threadIdx.x;
-    if (cidx >= n_cells) return;
+    // (lanes past the end take the last cell again: the maximum is the same)
+    const int cidx = min(blockIdx.x * BLOCK + (int)threadIdx.x, n_cells - 1);
     double r = 0.0;
     for (int i = 0; i < n_ions; ++i) {
         const double x = c[(size_t)i * n_cells + cidx];
@@ -2159,7 +2162,17 @@ k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, u
         if (q > r || isnan(q)) r = isnan(q) ? INFINITY : q;
     }
     // non-negative doubles order like their bit patterns
-    atomicMax(&rmax[cell_cluster[cidx]], (unsigned long long)__double_as_longlong(r));
+    unsigned long long v = (unsigned long long)__double_as_longlong(r);
+    const int q = cell_cluster[cidx], q0 = __builtin_amdgcn_readfirstlane(q);
+    if (__all(q == q0)) {
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long w = __shfl_xor(v, o);
+            v = w > v ? w : v;
+        }
+        if (threadIdx.x % 64 == 0) atomicMax(&rmax[q0], v);
+    } else {
+        atomicMax(&rmax[q], v);
+    }
 }
 
 // ---------------------------------------------------------------------------
