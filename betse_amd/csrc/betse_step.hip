@@ -2200,13 +2200,17 @@ k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, u
 // BT_FLAG_BARRIER and the block leaves.
 //
 // One block is one CU's 16 wavefronts. Phases of a step: environment (a block per
-// env tile and ion group, its quarters sharing the ions) and membranes (one or two
+// env tile and ion group, its quarters sharing the ions) and membranes (one or three
 // wavefronts per cell tile), side by side where no membrane law reads the
 // post-diffusion env, else one after the other; then the exchange (a wavefront
 // per ion over 64 squares).
 constexpr int TB = 1024;                     // threads per block
 constexpr int TW = TB / TMB;                 // wavefronts per block
 static_assert(TB == TSUB * TY * TX, "a block's quarters are env tiles' threads");
+// Wavefronts that share a tile's five or six ions. The membrane phase is a chain of
+// double-precision arithmetic on few wavefronts: us per step with two / three, 362
+// cells 10.7 / 10.2, 37 tiles on 32x32 9.2 / 8.5, 145 tiles 13.0 / 12.3.
+constexpr int TSPLIT = 3;
 constexpr int TEAM_BLOCKS = 32;              // blocks of a full team: the CUs of an XCD
 constexpr unsigned BT_FLAG_BARRIER = 2u;     // flags bit: a team barrier gave up waiting
 constexpr unsigned TEAM_STOP = 1u << 31;     // barrier word's bit: a NaN in the slot
@@ -2248,7 +2252,7 @@ struct TeamArgs {
     TeamCtls* ctl; TeamCtls* ctl_next;       // this launch's words (zero); the next launch's, zeroed here
     int n_groups;                            // ion groups of the env phase
     int n_blocks;                            // blocks expected per XCD
-    int split;                               // two wavefronts per cell tile, else one
+    int split;                               // TSPLIT wavefronts per cell tile, else one
     int mem_slots;                           // cell tiles of a block at a time
     int env_blocks;                          // of a full team, where the phases run side by side
     int n_steps;
@@ -2391,12 +2395,12 @@ k_step_team(TeamArgs) {
             const int b = nb - 1 - rank;
             if (b >= mb) return;
             const table<TeamArgs> TA = args();
-            // the LDS of a cell tile: a slice for each wavefront, or for each two (split)
+            // the LDS of a cell tile: a slice for each wavefront, or for each TSPLIT (split)
             constexpr int MR = NI * TMB;
             const bool split = TA->split != 0;
             const int n_chan = TA->P.n_chan, chan_nc = TA->mem[0].chan_nc, mem_slots = TA->mem_slots;
             const int t0 = S->t0, nt = S->nt;
-            const int mslot = split ? wave / 2 : wave, mhalf = wave & 1;
+            const int mslot = split ? wave / TSPLIT : wave, mpart = wave % TSPLIT;
             double* const wl = lds + mslot * team_wave_lds(NI, n_chan, chan_nc, split);
             double* const wc = wl + 2 * MR;                            // channel rows
             double* const wv = wc + mem_chan_lds(n_chan, chan_nc);     // split: lagged rows, Vmem
@@ -2410,7 +2414,7 @@ k_step_team(TeamArgs) {
                 for (int q0 = b; q0 < nt; q0 += mb * mem_slots) {
                     const int t = q0 + mslot * mb;
                     if (mslot < mem_slots && t < nt)
-                        mem_cell_wave<NI, FT, 2, -1, false, false, true>(TA->mem[par], TA->P, t0 + t, L, mhalf);
+                        mem_cell_wave<NI, FT, TSPLIT, -1, false, false, true>(TA->mem[par], TA->P, t0 + t, L, mpart);
                     else
                         for (int q = 0; q < MEM_SYNCS; ++q) lds_barrier();
                     lds_barrier();
@@ -2957,10 +2961,10 @@ static int launch_team(bt_ctx* c, int n_steps) {
                             : std::max(1, std::min(ta.n_blocks - 1, (int)((long long)ta.n_blocks * 5 * ne / (5 * ne + nt))));
     }
     const int mem_blocks = ta.ordered ? ta.n_blocks : ta.n_blocks - ta.env_blocks;
-    // two wavefronts per tile while the tiles fit at once
-    ta.split = (nt <= mem_blocks * (TW / 2)) ? 1 : 0;
+    // a tile's ions over TSPLIT wavefronts while the tiles fit at once
+    ta.split = (nt <= mem_blocks * (TW / TSPLIT)) ? 1 : 0;
     const size_t per = (size_t)team_wave_lds(ni, c->prm.n_chan, c->tile_nc, ta.split != 0) * sizeof(double);
-    ta.mem_slots = (int)std::min<size_t>(ta.split ? TW / 2 : TW, (159 * 1024) / per);
+    ta.mem_slots = (int)std::min<size_t>(ta.split ? TW / TSPLIT : TW, (159 * 1024) / per);
     const size_t lds = (size_t)team_lds(ni, c->prm.n_chan, c->tile_nc, ta.mem_slots, ta.split != 0) * sizeof(double);
     HIP_TRY(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     for (int done = 0; done < n_steps; done += ta.n_steps) {
