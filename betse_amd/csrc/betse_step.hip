@@ -2145,6 +2145,45 @@ __global__ void __launch_bounds__(64) k_spread_halt(unsigned* flags, int G) {
     if (__ballot(f != 0u) && threadIdx.x < MAX_GROUPS) flags[threadIdx.x] = f | 1u;
 }
 
+// The step's status to the host: two words in pinned memory, read after the stream
+// has been waited for (two blocking copies took 20 us more per call).
+struct Status {
+    unsigned flags;
+    unsigned long long bad_step;
+};
+__global__ void __launch_bounds__(64)
+k_status(const unsigned* flags, const unsigned long long* bad_step, Status* out) {
+    if (threadIdx.x == 0) {
+        out->flags = *flags;
+        out->bad_step = *bad_step;
+    }
+}
+
+// The state from the workspace to the caller's buffers, a segment per blockIdx.y, and
+// first what dst held to keep (may be NULL): one launch for what were five copies.
+struct BackSeg {
+    double* dst; const double* src; double* keep; long long n;
+};
+struct BackArgs {
+    BackSeg s[5];
+};
+__global__ void __launch_bounds__(BLOCK)
+k_copy_back(BackArgs a) {
+    const BackSeg S = a.s[blockIdx.y];
+    const long long stride = (long long)gridDim.x * BLOCK;
+    long long e = (long long)blockIdx.x * BLOCK + threadIdx.x;
+    if ((((size_t)S.dst | (size_t)S.src) & 15) == 0 && !S.keep) {
+        typedef double v2d __attribute__((ext_vector_type(2)));
+        for (; e < S.n / 2; e += stride) reinterpret_cast<v2d*>(S.dst)[e] = reinterpret_cast<const v2d*>(S.src)[e];
+        if ((S.n & 1) && blockIdx.x == 0 && threadIdx.x == 0) S.dst[S.n - 1] = S.src[S.n - 1];
+        return;
+    }
+    for (; e < S.n; e += stride) {
+        if (S.keep) S.keep[e] = S.dst[e];
+        S.dst[e] = S.src[e];
+    }
+}
+
 // Per-cluster max over cells and ions of |c - c_prev| / |c| (init residual). A
 // wavefront whose cells are one cluster's reduces them before its atomic: with one
 // per cell a cluster's cells queued on its word, 169 us for 60k cells of 48 clusters,
@@ -2532,6 +2571,7 @@ struct bt_ctx {
     uint8_t* live_flag = nullptr;        // per square: SQ_LIVE if in sq_live, SQ_HAS_MEM
     int n_live = 0;
     unsigned* flags = nullptr; unsigned long long* bad_step = nullptr; long long* step_ctr = nullptr;
+    Status* status = nullptr;            // pinned
     // step graphs per group g of clusters: one pair of steps, and tune.graph_pairs pairs
     hipGraph_t graph[MAX_GROUPS] = {}; hipGraphExec_t gexec[MAX_GROUPS] = {};
     hipGraph_t graph_n[MAX_GROUPS] = {}; hipGraphExec_t gexec_n[MAX_GROUPS] = {};
@@ -3109,16 +3149,19 @@ static int launch_graphs(bt_ctx* c, int pairs) {
     return BT_OK;
 }
 
-static int copy_back(bt_ctx* c) {
-    const size_t nc = (size_t)c->prm.n_cells;
-    const size_t ni = (size_t)c->prm.n_ions;
-    HIP_TRY(c, hipMemcpyAsync(c->buf.c_cell, c->c_cell_b, ni * nc * 8, hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->buf.c_lag, c->c_lag_b, ni * nc * 8, hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->buf.vm_cell, c->vm_b, nc * 8, hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->buf.c_env, c->c_env_b, ni * (size_t)c->kp.n_sq * 8, hipMemcpyDeviceToDevice,
-                              c->stream));
-    if (steps_fused(c))
-        HIP_TRY(c, hipMemcpyAsync(c->u, c->u_b, (size_t)c->kp.n_sq * 8, hipMemcpyDeviceToDevice, c->stream));
+// vm_keep (may be NULL) receives the caller's vm_cell from before
+static int copy_back(bt_ctx* c, double* vm_keep = nullptr) {
+    const long long nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->kp.n_sq;
+    const BackArgs a = {{{c->buf.c_cell, c->c_cell_b, nullptr, ni * nc},
+                         {c->buf.c_lag, c->c_lag_b, nullptr, ni * nc},
+                         {c->buf.vm_cell, c->vm_b, vm_keep, nc},
+                         {c->buf.c_env, c->c_env_b, nullptr, ni * ns},
+                         {c->u, c->u_b, nullptr, ns}}};
+    // (u is copied where its steps write a workspace of their own)
+    const long long most = std::max(nc, ns) * ni;
+    const unsigned nb = (unsigned)std::min<long long>((most / 2 + BLOCK - 1) / BLOCK + 1, 2048);
+    hipLaunchKernelGGL(k_copy_back, dim3(nb, steps_fused(c) ? 5 : 4), dim3(BLOCK), 0, c->stream, a);
+    HIP_TRY(c, hipGetLastError());
     return BT_OK;
 }
 
@@ -3518,6 +3561,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     alloc((void**)&c->u_b, (ns + 1) * 8);
     alloc((void**)&c->flags, 256);
     alloc((void**)&c->bad_step, 256);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->status, sizeof(Status), hipHostMallocDefault);
     alloc((void**)&c->step_ctr, 256);
     alloc((void**)&c->ctl, 2 * sizeof(TeamCtls));
     alloc((void**)&c->slots, c->slots_host.size() * sizeof(TeamSlot));
@@ -3586,6 +3630,7 @@ int bt_destroy(bt_ctx* c) {
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (void* q : c->obs_alloc) (void)hipFree(q);
+    if (c->status) (void)hipHostFree(c->status);
     delete c;
     return BT_OK;
 }
@@ -3934,11 +3979,12 @@ int bt_autotune(bt_ctx* c, int32_t n_launches, bt_tuning* chosen, double* trial_
 
 int bt_sync(bt_ctx* c, int64_t* bad_step) {
     if (!c) return BT_EINVAL;
+    hipLaunchKernelGGL(k_status, dim3(1), dim3(64), 0, c->stream, (const unsigned*)c->flags,
+                       (const unsigned long long*)c->bad_step, c->status);
+    HIP_TRY(c, hipGetLastError());
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    unsigned flags = 0;
-    unsigned long long bs = ~0ull;
-    HIP_TRY(c, hipMemcpy(&flags, c->flags, sizeof(flags), hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(&bs, c->bad_step, sizeof(bs), hipMemcpyDeviceToHost));
+    const unsigned flags = c->status->flags;
+    const unsigned long long bs = c->status->bad_step;
     if (bad_step) *bad_step = (bs == ~0ull) ? -1 : (int64_t)bs;
     if (flags & BT_FLAG_BARRIER)
         return set_err(c, BT_EHIP, "a grid barrier of the persistent step kernel gave up waiting");
@@ -4052,12 +4098,13 @@ int bt_step_observed(bt_ctx* c, int32_t n_steps, int32_t use_graph, const bt_obs
         --n_steps;
     }
     const int ahead = n_steps - 1;
+    const int odd = use_team(c) ? 0 : ahead & 1;     // (the team kernel takes either)
     if (ahead > 0) {
         // keep the graph on the caller buffers: an even number of graph steps, then eager ones
-        int rc = bt_step(c, ahead - (ahead & 1), use_graph);
+        int rc = bt_step(c, ahead - odd, use_graph);
         if (rc != BT_OK) return rc;
     }
-    int rest = (ahead & 1) + 1;           // 1 or 2 eager steps, the last one observed
+    const int rest = odd + 1;             // 1 or 2 eager steps, the last one observed
     if (rest == 2) {
         enqueue_step(c, 0);
         HIP_TRY(c, hipMemcpyAsync(c->vm_prev, c->vm_b, vbytes, hipMemcpyDeviceToDevice, c->stream));
@@ -4067,13 +4114,12 @@ int bt_step_observed(bt_ctx* c, int32_t n_steps, int32_t use_graph, const bt_obs
         enqueue_step(c, 1);
         c->capture = nullptr;
     } else {
-        HIP_TRY(c, hipMemcpyAsync(c->vm_prev, c->buf.vm_cell, vbytes, hipMemcpyDeviceToDevice, c->stream));
         if (c->phib_prev)
             HIP_TRY(c, hipMemcpyAsync(c->phib_prev, c->buf.Phi_b, pbytes, hipMemcpyDeviceToDevice, c->stream));
         c->capture = obs;
         enqueue_step(c, 0);
         c->capture = nullptr;
-        int rc = copy_back(c);
+        int rc = copy_back(c, c->vm_prev);
         if (rc == BT_OK && c->phib_staged) rc = apply_staged_boundary(c);
         if (rc != BT_OK) return rc;
     }
