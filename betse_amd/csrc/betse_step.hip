@@ -3328,53 +3328,76 @@ int64_t bt_steps_done(const bt_ctx* ctx) { return ctx ? ctx->steps_done : -1; }
 static int derive_uniform(bt_ctx* c) {
     const bt_params* p = &c->prm;
     const int nq = (int)c->clusters.size();
-    std::vector<double> dm((size_t)p->n_ions * p->n_mems), gj((size_t)p->n_mems), de((size_t)p->n_ions * p->n_squares);
-    std::vector<double> pb(c->buf.Phi_b ? (size_t)p->n_squares : 0);
-    hipError_t e = hipMemcpy(dm.data(), c->buf.Dm, dm.size() * 8, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(gj.data(), c->buf.gjopen, gj.size() * 8, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(de.data(), c->buf.D_env, de.size() * 8, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && !pb.empty()) e = hipMemcpy(pb.data(), c->buf.Phi_b, pb.size() * 8, hipMemcpyDeviceToHost);
-    if (e != hipSuccess)
+    // a row at a time through one buffer: all rows at once are 50 MB of first touches
+    // for 100k cells
+    std::vector<double> row(std::max(p->n_mems, p->n_squares));
+    auto fetch = [&](const double* src, size_t n) -> int {
+        const hipError_t e = hipMemcpy(row.data(), src, n * 8, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) return BT_OK;
         return set_err(c, BT_EHIP, std::string("reading Dm, gjopen, D_env, Phi_b: ") + hipGetErrorString(e));
-    c->any_phib = false;
-    const bool varied = c->denv_varies;
-    c->denv_varies = false;
-    for (int q = 0; q < nq; ++q) {
-        KCluster& K = c->kcl_host[q];
-        const int lo = c->cl_mem_lo[q], hi = c->cl_mem_hi[q];
+    };
+    // the value of [lo, hi) where it is one, else NaN
+    auto uniform = [&](size_t lo, size_t hi) {
+        bool same = true;
+        for (size_t k = lo; k < hi && same; ++k) same = (row[k] == row[lo]);
+        return same ? row[lo] : (double)NAN;
+    };
+    for (KCluster& K : c->kcl_host) {
         for (int i = 0; i < BT_MAX_IONS; ++i) K.dm_u[i] = K.denv_u[i] = NAN;
         K.gjo_u = NAN;
         K.still_mem = 0;
-        if (hi > lo) {
-            for (int i = 0; i < p->n_ions; ++i) {
-                const double* d = dm.data() + (size_t)i * p->n_mems;
-                bool same = true;
-                for (int m = lo; m < hi && same; ++m) same = (d[m] == d[lo]);
-                K.dm_u[i] = same ? d[lo] : NAN;
-            }
-            bool same = true;
-            for (int m = lo; m < hi && same; ++m) same = (gj[m] == gj[lo]);
-            K.gjo_u = same ? gj[lo] : NAN;
-            for (int i = 0; i < p->n_ions; ++i)
-                if (K.dm_u[i] == 0.0 && i != c->kp.i_na && i != c->kp.i_k && i != c->kp.i_ca && c->kp.ion_chan[i] < 0)
-                    K.still_mem |= 1u << i;
-        }
-        const size_t k0 = (size_t)c->clusters[q].sq_off;
-        const size_t k1 = k0 + (size_t)c->clusters[q].grid_ny * c->clusters[q].grid_nx;
-        for (int i = 0; i < p->n_ions; ++i) {
-            const double* d = de.data() + (size_t)i * p->n_squares;
-            bool same = true;
-            for (size_t k = k0; k < k1 && same; ++k) same = (d[k] == d[k0]);
-            K.denv_u[i] = same ? d[k0] : NAN;
-            c->denv_varies = c->denv_varies || !same;
-        }
         K.phib = 0;
-        for (size_t k = k0; k < k1 && !pb.empty() && !K.phib; ++k) K.phib = (pb[k] != 0.0);
-        if (K.phib) K.still_mem |= PHIB_BIT;
-        if (K.phib && p->n_chan > 0)
-            return set_err(c, BT_EINVAL, "an applied boundary voltage (Phi_b) with voltage-gated channels is not "
-                                         "supported (their gating rates are per cell)");
-        c->any_phib = c->any_phib || K.phib;
+    }
+    int rc = BT_OK;
+    for (int i = 0; i <= p->n_ions; ++i) {
+        const bool gj = (i == p->n_ions);
+        rc = gj ? fetch(c->buf.gjopen, p->n_mems) : fetch(c->buf.Dm + (size_t)i * p->n_mems, p->n_mems);
+        if (rc != BT_OK) return rc;
+        for (int q = 0; q < nq; ++q) {
+            KCluster& K = c->kcl_host[q];
+            const int lo = c->cl_mem_lo[q], hi = c->cl_mem_hi[q];
+            if (hi <= lo) continue;
+            const double u = uniform(lo, hi);
+            if (gj) {
+                K.gjo_u = u;
+                continue;
+            }
+            K.dm_u[i] = u;
+            if (u == 0.0 && i != c->kp.i_na && i != c->kp.i_k && i != c->kp.i_ca && c->kp.ion_chan[i] < 0)
+                K.still_mem |= 1u << i;
+        }
+    }
+    const bool varied = c->denv_varies;
+    c->denv_varies = false;
+    auto squares = [&](int q, size_t& k0, size_t& k1) {
+        k0 = (size_t)c->clusters[q].sq_off;
+        k1 = k0 + (size_t)c->clusters[q].grid_ny * c->clusters[q].grid_nx;
+    };
+    size_t k0, k1;
+    for (int i = 0; i < p->n_ions; ++i) {
+        rc = fetch(c->buf.D_env + (size_t)i * p->n_squares, p->n_squares);
+        if (rc != BT_OK) return rc;
+        for (int q = 0; q < nq; ++q) {
+            squares(q, k0, k1);
+            const double u = uniform(k0, k1);
+            c->kcl_host[q].denv_u[i] = u;
+            c->denv_varies = c->denv_varies || isnan(u);
+        }
+    }
+    c->any_phib = false;
+    if (c->buf.Phi_b) {
+        rc = fetch(c->buf.Phi_b, p->n_squares);
+        if (rc != BT_OK) return rc;
+        for (int q = 0; q < nq; ++q) {
+            KCluster& K = c->kcl_host[q];
+            squares(q, k0, k1);
+            for (size_t k = k0; k < k1 && !K.phib; ++k) K.phib = (row[k] != 0.0);
+            if (K.phib) K.still_mem |= PHIB_BIT;
+            if (K.phib && p->n_chan > 0)
+                return set_err(c, BT_EINVAL, "an applied boundary voltage (Phi_b) with voltage-gated channels is not "
+                                             "supported (their gating rates are per cell)");
+            c->any_phib = c->any_phib || K.phib;
+        }
     }
     // the captured step graphs hold the env kernel of the other kind
     if (c->denv_varies != varied) drop_graphs(c);
