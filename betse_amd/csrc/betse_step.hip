@@ -2749,10 +2749,8 @@ static KCluster derive_cluster(const bt_params& p, const bt_cluster& b) {
     return k;
 }
 
-// Default wavefronts per tile of k_mem_cell: two (ions split between them)
-// while one wavefront per tile would leave the SIMDs with few waves to switch
-// between (step us with two and one: 2,193 tiles 20.2 and 20.5, 3,849 tiles 27.3
-// and 24.7); pairs of steps per replayed graph (fewer graph launches).
+// tiles from which one wavefront per tile fills the SIMDs (default_mem_waves); pairs
+// of steps per replayed graph (fewer graph launches).
 constexpr int BT_MEM_WG_TILES = 3000;
 constexpr int BT_GRAPH_PAIRS = 8;
 constexpr int BT_MAX_GRAPH_PAIRS = 64;
@@ -2814,6 +2812,26 @@ static void launch_mem_cell(bt_ctx* c, const MemCellArgs& a, hipStream_t st, int
         case 7: launch_mem_cell_t<7>(c, a, st, nt); break;
         default: launch_mem_cell_t<8>(c, a, st, nt); break;
     }
+}
+
+// Default wavefronts per tile of k_mem_cell: two (ions split between them) while one
+// would leave the SIMDs with few waves to switch between (step us with two and one,
+// no channels: 2,193 tiles 20.2 and 20.5, 3,849 tiles 27.3 and 24.7). With channels the
+// two share a tile's LDS rows, so that more waves fit a CU, and two stay the better form
+// (two channels: 5,225 tiles 42.1 and 45.1, 10,486 tiles 65.1 and 69.2; three: 10,486
+// tiles 83.4 and 89.7, 17,556 tiles 146.5 and 157.8) except where one per tile fits all
+// tiles at once and two do not (two channels, FP32 flux, 3,628 tiles 34.0 and 31.7,
+// 4,387 tiles 35.9 and 34.0; three, 3,274 tiles 45.4 and 42.7).
+static int default_mem_waves(const bt_ctx* c) {
+    if (c->n_tiles < BT_MEM_WG_TILES) return 2;
+    if (c->prm.n_chan == 0) return 1;
+    // tiles resident at once, by LDS (given out in pieces of 1,280 bytes, 160 KB per CU)
+    auto resident = [&](int waves) {
+        const size_t rows = (size_t)(waves + 1) * c->prm.n_ions * TMB + (waves > 1 ? BT_TILE_CELLS : 0);
+        const size_t lds = (rows + mem_chan_lds(c->prm.n_chan, c->tile_nc)) * sizeof(double) + (BT_TILE_CELLS + 2) * sizeof(int);
+        return (int)(160 * 1024 / ((lds + 1279) / 1280 * 1280)) * N_XCD * TEAM_BLOCKS;
+    };
+    return c->n_tiles > resident(2) && c->n_tiles <= resident(1) ? 1 : 2;
 }
 
 static inline int grid_blocks(int n) { return (n + BLOCK - 1) / BLOCK; }
@@ -3631,7 +3649,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     alloc((void**)&c->sq_live, sizeof(LiveRec) * (lrec.empty() ? 1 : lrec.size()));
     alloc((void**)&c->live_flag, ns);
     c->n_live = (int)sq_live.size();
-    c->tune.mem_waves = (c->n_tiles < BT_MEM_WG_TILES) ? 2 : 1;
+    c->tune.mem_waves = default_mem_waves(c);
     c->tune.env_ions_per_block = (c->n_env_tiles < ENV_SPLIT_TILES) ? std::min(2, p->n_ions) : p->n_ions;
     c->tune.exchange_form = (c->n_live < EX_SPLIT_SQUARES) ? 0 : 1;
     if (c->tune.exchange_form == 1 && fused_allowed(c, &c->tune)) c->tune.exchange_form = BT_EXCHANGE_FUSED;
