@@ -2295,12 +2295,12 @@ constexpr unsigned TEAM_NONE = ~0u;          // team size word: no slot left, le
 constexpr unsigned TEAM_SPINS = 1u << 22;    // polls (over a second) before a wait gives up
 // The work of a slot, in cell tiles (an env tile costs about four), up to which the
 // team kernel is the default. us per step, team against replayed graphs (FP64):
-//   plain     4 cell + 1 env tiles   9.1 / 15.8     145 + 16  12.3 / 16.2
-//             61 + 16               10.9 / 15.9     226 + 25  17.7 / 16.1
-//             8 clusters of 200-400 cells 10.8 / 16.1, 32 of 60-200 13.7 / 17.9,
-//             64 of 60-200 18.5 / 16.6
-//   ordered   4 + 1                 15.1 / 19.6     61 + 9    19.4 / 20.3
-//   (channels or a Ca pump)         37 + 16 18.8 / 19.5   61 + 16 20.6 / 19.9
+//   plain     4 cell + 1 env tiles   7.2 / 15.9     145 + 16  13.5 / 16.2
+//             37 + 16                8.8 / 17.3     193 + 25  16.7 / 16.3
+//             8 clusters of 200-400 cells 9.5 / 16.2, of 1,000-1,600 13.3 / 19.0,
+//             48 of 60-200 cells 13.7 / 16.7, 64 of them 18.5 / 16.5
+//   ordered   4 + 1                 15.2 / 19.0     61 + 9    18.6 / 20.0
+//   (channels or a Ca pump)         61 + 16 19.1 / 19.7   93 + 9 20.2 / 19.6
 // Beyond, one XCD's 32 CUs have more to do than eight times as many save.
 constexpr int TEAM_TILES = 220;
 constexpr int TEAM_TILES_ORDERED = 100;
