@@ -2275,6 +2275,12 @@ k_residual(const double* c, const double* c_prev, const int32_t* cell_cluster, u
 // its slot done a team claims the next. A wait of about a second sets
 // BT_FLAG_BARRIER and the block leaves.
 //
+// A NaN stops its slot at once. Of several slots the others have run on, or ahead,
+// by then, so each slot first keeps a copy of its state, and a second launch
+// (TEAM_FINISH) puts the slots back and steps them to the earliest step that
+// produced a NaN, where replayed steps of the whole batch would have stopped;
+// without a NaN it computes v_env and E. It costs a call 9 us.
+//
 // One block is one CU's 16 wavefronts. Phases of a step: environment (a block per
 // env tile and ion group, its quarters sharing the ions) and membranes (one or three
 // wavefronts per cell tile), side by side where no membrane law reads the
@@ -2315,9 +2321,22 @@ struct TeamCtls {
     unsigned next_slot, pad[31];
 };
 
-// A slot's share of the work lists, its cells and its squares.
+// A slot's share of the work lists, its cells, squares and membranes.
 struct TeamSlot {
-    int t0, nt, e0, ne, l0, nl, c0, c1, k0, k1;
+    int t0, nt, e0, ne, l0, nl, c0, c1, k0, k1, m0, m1;
+};
+
+// A copy of what steps change in place, from before a launch (all null where one
+// slot holds every cluster); c_env_b: the env state of odd steps, of which a step
+// that is halted leaves a part as it was.
+struct TeamSave {
+    double* c_cell; double* c_lag; double* vm; double* c_env; double* c_env_b; double* u; double* gates;
+};
+
+enum TeamMode {
+    TEAM_RUN,                                // steps; with one slot also v_env and E
+    TEAM_FINISH,                             // after TEAM_RUN of several slots: v_env and E, or, halted, as TEAM_REWIND
+    TEAM_REWIND                              // after steps that left some clusters past a NaN's step: all back to it
 };
 
 struct TeamArgs {
@@ -2334,6 +2353,10 @@ struct TeamArgs {
     int n_steps;
     long long step0;                         // index of the first step
     int ordered;                             // the membrane laws read the post-diffusion env
+    int mode;                                // a TeamMode
+    int n_env_tiles;
+    int fused;                               // TEAM_REWIND: the steps had the exchange in the env kernel
+    TeamSave save;
     KParams P;
 };
 
@@ -2390,7 +2413,7 @@ __global__ void __launch_bounds__(TB)
 k_step_team(TeamArgs) {
     extern __shared__ double lds[];
     __shared__ unsigned s_word;
-    __shared__ int s_rank, s_size, s_slot;
+    __shared__ int s_rank, s_size, s_slot, s_stop;
     auto args = [] {
         table<TeamArgs> p = (table<TeamArgs>)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(p));
@@ -2401,16 +2424,40 @@ k_step_team(TeamArgs) {
     const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | 20);
     TeamCtl* const T = args()->ctl->team + xcd;
     unsigned* const flags = args()->mem[0].flags;
-    const int n_slots = args()->n_slots, n_blocks = args()->n_blocks;
+    const int n_slots = args()->n_slots, n_blocks = args()->n_blocks, mode = args()->mode;
     if (blockIdx.x == 0)
         for (int i = tid; i < (int)(sizeof(TeamCtls) / sizeof(unsigned)); i += TB)
             reinterpret_cast<unsigned*>(args()->ctl_next)[i] = 0u;
+    // v_env and E of the state at the end of the steps, by env tiles first, first + by, ...
+    auto fields = [&](int first, int by, int last, bool counts) {
+        const table<TeamArgs> TA = args();
+        for (int it = first; it < last; it += by) {
+            env_field_tile<false, false, false, false, false, true>(TA->field[0], TA->P, it, 0, 0, tid, lds, -1, 0, false);
+            lds_barrier();
+        }
+        if (counts && tid < MAX_GROUPS) const_cast<long long*>(TA->mem[0].step_ctr)[tid] = TA->step0 + TA->n_steps;
+    };
+    if (mode == TEAM_FINISH) {
+        if (tid == 0) s_word = agent_load(flags);
+        __syncthreads();
+        if (s_word == 0u) {                      // (nothing sets a flag in this launch)
+            fields(blockIdx.x, gridDim.x, args()->n_env_tiles, blockIdx.x == 0);
+            return;
+        }
+    }
     if (tid == 0) {
+        // the step of a NaN counted from this launch's first: below zero, an earlier
+        // launch halted the run (bad_step is written before the flag)
+        const unsigned f = agent_load(flags);
+        long long stop = -1;
+        if (f != 0u) stop = (long long)ld<true>(args()->mem[0].bad_step) - args()->step0;
+        const bool run = !(f & BT_FLAG_BARRIER) && (f != 0u ? stop >= 0 : mode == TEAM_RUN);
+        s_stop = (f != 0u && mode != TEAM_RUN) ? (int)stop : -1;
         int size = 0;
         const unsigned t = atomicAdd(&T->reg, 1u);
         if (!(t & TEAM_CLOSED)) {
             if (t == 0) {
-                const unsigned slot = halted(flags) ? TEAM_NONE : atomicAdd(&args()->ctl->next_slot, 1u);
+                const unsigned slot = run ? atomicAdd(&args()->ctl->next_slot, 1u) : TEAM_NONE;
                 if (slot >= (unsigned)n_slots) {
                     atomicOr(&T->reg, TEAM_CLOSED);
                     __hip_atomic_store(&T->size, TEAM_NONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2437,6 +2484,7 @@ k_step_team(TeamArgs) {
     const int rank = __builtin_amdgcn_readfirstlane(s_rank), nb = __builtin_amdgcn_readfirstlane(s_size);
     if (nb == 0) return;
     int slot = __builtin_amdgcn_readfirstlane(s_slot);
+    const int stop = __builtin_amdgcn_readfirstlane(s_stop);    // the step to go back to, if any
     unsigned target = 0;
     const int wave = __builtin_amdgcn_readfirstlane(tid / TMB), lane = tid % TMB;
 
@@ -2514,11 +2562,38 @@ k_step_team(TeamArgs) {
                 lds_barrier();
             }
         };
+        // the slot's part of the buffers that steps change in place
+        auto each_row = [&](auto row) {
+            const table<TeamArgs> TA = args();
+            const size_t C = TA->P.n_cells, Q = TA->P.n_sq, M = TA->P.n_mems;
+            for (int i = 0; i < TA->P.n_ions; ++i) {
+                row(TA->mem[0].c_cell_in + i * C, TA->save.c_cell + i * C, S->c0, S->c1);
+                row(TA->mem[0].c_lag_in + i * C, TA->save.c_lag + i * C, S->c0, S->c1);
+                row(TA->field[0].c_env + i * Q, TA->save.c_env + i * Q, S->k0, S->k1);
+                row(TA->field[0].c_env_out + i * Q, TA->save.c_env_b + i * Q, S->k0, S->k1);
+            }
+            row(TA->mem[0].vm_in, TA->save.vm, S->c0, S->c1);
+            row(TA->field[0].u, TA->save.u, S->k0, S->k1);
+            if (CHAN)
+                for (int g = 0; g < 2 * TA->P.n_chan; ++g) row(TA->mem[0].gates + g * M, TA->save.gates + g * M, S->m0, S->m1);
+        };
+        const bool several = args()->save.c_cell != nullptr, rewind = stop >= 0;
         unsigned word = 1;
+        if (rewind || (several && mode == TEAM_RUN)) {
+            each_row([&](const double* x, double* kept, int lo, int hi) {
+                double* const to = rewind ? const_cast<double*>(x) : kept;
+                const double* const from = rewind ? kept : x;
+                for (int k = lo + rank * TB + tid; k < hi; k += nb * TB) to[k] = ld<true>(from + k);
+            });
+            // (all copied before any changes)
+            word = team_sync(T, target += nb, flags, &s_word);
+            if (word == 0) return;
+        }
         int s = 0;
-        for (; s < n_steps; ++s) {
+        for (; s < ((mode == TEAM_RUN || rewind) ? n_steps : 0); ++s) {
             const int par = s & 1;
-            env_phase(par);
+            // (where the exchange is in the env kernel, a NaN's step has no env phase)
+            if (s != stop || !args()->fused) env_phase(par);
             if (ordered) {
                 word = team_sync(T, target += nb, flags, &s_word);
                 if (word == 0) return;
@@ -2528,29 +2603,25 @@ k_step_team(TeamArgs) {
             mem_phase(par);
             word = team_sync(T, target += nb, flags, &s_word);
             if (word == 0) return;
-            if (word & TEAM_STOP) break;
+            if ((word & TEAM_STOP) || s == stop) break;
             exchange_phase(par);
             word = team_sync(T, target += nb, flags, &s_word);
             if (word == 0) return;
         }
         const table<TeamArgs> TA = args();
-        if (word & TEAM_STOP) {
-            if (rank == 0 && tid == 0) {
-                atomicOr(flags, 1u);
+        const bool stopped = (word & TEAM_STOP) || rewind;
+        if (stopped) {
+            if (rank == 0 && tid == 0 && !rewind) {
                 atomicMin(TA->mem[0].bad_step, (unsigned long long)(TA->step0 + s));
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                atomicOr(flags, 1u);
             }
-        } else {
-            // v_env and E of the state
-            const int ne = S->ne;
-            for (int it = rank; it < ne; it += nb) {
-                env_field_tile<false, false, false, false, false, true>(TA->field[0], TA->P, S->e0 + it, 0, 0, tid, lds, -1, 0,
-                                                                        false);
-                lds_barrier();
-            }
-            if (slot == 0 && rank == 0 && tid < MAX_GROUPS)
-                const_cast<long long*>(TA->mem[0].step_ctr)[tid] = TA->step0 + n_steps;
+            if (rewind && slot == 0 && rank == 0 && tid < MAX_GROUPS)
+                const_cast<long long*>(TA->mem[0].step_ctr)[tid] = TA->step0 + stop;
+        } else if (!several) {
+            fields(S->e0 + rank, nb, S->e0 + S->ne, rank == 0);
         }
-        if (n_steps & 1) {
+        if ((n_steps & 1) && (mode == TEAM_RUN || rewind)) {
             // the state from the workspace to the caller's buffers (halted or not,
             // as after replayed steps)
             auto back = [&](double* dst, const double* src, int lo, int hi) {
@@ -2565,13 +2636,20 @@ k_step_team(TeamArgs) {
             }
             back(TA->mem[1].vm_out, TA->mem[1].vm_in, c0, c1);
         }
+        if (stopped) {
+            // the next slot starts without the stop, once every block has read it
+            word = team_sync(T, target += nb, flags, &s_word);
+            if (word == 0) return;
+            if (rank == 0 && tid == 0)
+                __hip_atomic_fetch_and(&T->bar, ~TEAM_STOP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
         // the next slot, claimed by the team's first block
         if (rank == 0 && tid == 0) {
             const unsigned next = atomicAdd(&TA->ctl->next_slot, 1u);
             __hip_atomic_store(&T->slot, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         word = team_sync(T, target += nb, flags, &s_word);
-        if (word == 0 || (word & TEAM_STOP)) return;
+        if (word == 0) return;
         if (tid == 0) s_slot = (int)min(agent_load(&T->slot), 0x7fffffffu);
         __syncthreads();
         slot = __builtin_amdgcn_readfirstlane(s_slot);
@@ -2634,6 +2712,7 @@ struct bt_ctx {
     // a launch and one that it leaves zeroed for the next
     std::vector<TeamSlot> slots_host;
     TeamSlot* slots = nullptr; TeamCtls* ctl = nullptr; int ctl_at = 0;
+    double* save = nullptr;            // TeamSave's copy of the state
     bool team_fits = false;            // small enough for the team kernel to be the faster one
     bool team_warm = false;            // it has been launched
     long long steps_done = 0;
@@ -3018,12 +3097,37 @@ static const void* team_kernel(const bt_ctx* c) {
     }
 }
 
-// n_steps steps, v_env and E of the last, and the state in the caller's buffers,
-// in launches of the team kernel
-static int launch_team(bt_ctx* c, int n_steps) {
-    const void* k = team_kernel(c);
-    if (!k) return set_err(c, BT_EINVAL, "no persistent step kernel for this problem");
-    TeamArgs ta;
+// the state's copy that clusters are put back from (ensure_save)
+static TeamSave save_pointers(const bt_ctx* c) {
+    const size_t nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->kp.n_sq;
+    TeamSave s;
+    s.c_cell = c->save;
+    s.c_lag = s.c_cell + ni * nc;
+    s.vm = s.c_lag + ni * nc;
+    s.c_env = s.vm + nc;
+    s.c_env_b = s.c_env + ni * ns;
+    s.u = s.c_env_b + ni * ns;
+    s.gates = s.u + ns;
+    return s;
+}
+static int ensure_save(bt_ctx* c) {
+    if (c->save) return BT_OK;
+    const size_t nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->prm.n_squares;
+    const size_t n = (2 * ni + 1) * nc + (2 * ni + 1) * ns + 2 * (size_t)c->prm.n_chan * c->prm.n_mems;
+    HIP_TRY(c, hipMalloc((void**)&c->save, n * sizeof(double)));
+    return BT_OK;
+}
+
+// a launch of the team kernel without what one launch differs from the next in
+struct TeamLaunch {
+    const void* kernel;
+    size_t lds;
+    TeamArgs args;
+};
+static int team_launch_of(bt_ctx* c, TeamLaunch& tl) {
+    tl.kernel = team_kernel(c);
+    if (!tl.kernel) return set_err(c, BT_EINVAL, "no persistent step kernel for this problem");
+    TeamArgs& ta = tl.args;
     for (int par = 0; par < 2; ++par) {
         const StepArgs a = step_args(c, par, nullptr, 0);
         ta.field[par] = a.field;
@@ -3034,6 +3138,9 @@ static int launch_team(bt_ctx* c, int n_steps) {
     ta.slots = c->slots;
     ta.n_slots = (int)c->slots_host.size();
     ta.ordered = (c->prm.n_chan > 0 || c->kp.i_ca >= 0) ? 1 : 0;
+    ta.fused = 0;
+    ta.n_env_tiles = c->n_env_tiles;
+    ta.save = TeamSave{};
     int ne = 1, nt = 1;
     for (const TeamSlot& q : c->slots_host) {
         ne = std::max(ne, q.ne);
@@ -3060,18 +3167,39 @@ static int launch_team(bt_ctx* c, int n_steps) {
     ta.split = (nt <= mem_blocks * (TW / TSPLIT)) ? 1 : 0;
     const size_t per = (size_t)team_wave_lds(ni, c->prm.n_chan, c->tile_nc, ta.split != 0) * sizeof(double);
     ta.mem_slots = (int)std::min<size_t>(ta.split ? TW / TSPLIT : TW, (159 * 1024) / per);
-    const size_t lds = (size_t)team_lds(ni, c->prm.n_chan, c->tile_nc, ta.mem_slots, ta.split != 0) * sizeof(double);
-    HIP_TRY(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    for (int done = 0; done < n_steps; done += ta.n_steps) {
-        ta.n_steps = std::min(n_steps - done, TEAM_STEPS);
-        ta.step0 = c->steps_done + done;
-        ta.ctl = c->ctl + c->ctl_at;
-        c->ctl_at ^= 1;
-        ta.ctl_next = c->ctl + c->ctl_at;
-        void* args[] = {(void*)&ta};
-        HIP_TRY(c, hipLaunchKernel(k, dim3(N_XCD * ta.n_blocks), dim3(TB), args, lds, c->stream));
-    }
+    tl.lds = (size_t)team_lds(ni, c->prm.n_chan, c->tile_nc, ta.mem_slots, ta.split != 0) * sizeof(double);
+    HIP_TRY(c, hipFuncSetAttribute(tl.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tl.lds));
     return BT_OK;
+}
+static int launch_team_mode(bt_ctx* c, TeamLaunch& tl, int mode, long long step0, int n_steps) {
+    TeamArgs& ta = tl.args;
+    ta.mode = mode;
+    ta.step0 = step0;
+    ta.n_steps = n_steps;
+    ta.ctl = c->ctl + c->ctl_at;
+    c->ctl_at ^= 1;
+    ta.ctl_next = c->ctl + c->ctl_at;
+    void* args[] = {(void*)&ta};
+    HIP_TRY(c, hipLaunchKernel(tl.kernel, dim3(N_XCD * ta.n_blocks), dim3(TB), args, tl.lds, c->stream));
+    return BT_OK;
+}
+
+// n_steps steps, v_env and E of the last, and the state in the caller's buffers,
+// in launches of the team kernel
+static int launch_team(bt_ctx* c, int n_steps) {
+    TeamLaunch tl;
+    int rc = team_launch_of(c, tl);
+    const bool several = tl.args.n_slots > 1;
+    if (rc == BT_OK && several) {
+        rc = ensure_save(c);
+        if (rc == BT_OK) tl.args.save = save_pointers(c);
+    }
+    for (int done = 0, n = 0; rc == BT_OK && done < n_steps; done += n) {
+        n = std::min(n_steps - done, TEAM_STEPS);
+        rc = launch_team_mode(c, tl, TEAM_RUN, c->steps_done + done, n);
+        if (rc == BT_OK && several) rc = launch_team_mode(c, tl, TEAM_FINISH, c->steps_done + done, n);
+    }
+    return rc;
 }
 
 // whether bt_step runs its steps in the team kernel
@@ -3540,7 +3668,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
         const int nq = n_clusters;
         if (c->cl_tile0.empty()) {
             c->slots_host.push_back(TeamSlot{0, b->n_tiles, 0, c->n_env_tiles, 0, (int)sq_live.size(), 0, p->n_cells, 0,
-                                             p->n_squares});
+                                             p->n_squares, 0, p->n_mems});
         } else {
             // a cluster's cost: its cell tiles and env tiles (about equal times)
             auto cost = [&](int q) {
@@ -3578,7 +3706,8 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
                 c->slots_host.push_back(TeamSlot{c->cl_tile0[qa], c->cl_tile0[qz] - c->cl_tile0[qa], c->cl_env0[qa],
                                                  c->cl_env0[qz] - c->cl_env0[qa], c->cl_live0[qa],
                                                  c->cl_live0[qz] - c->cl_live0[qa], (int)c->cl_cell0[qa],
-                                                 (int)c->cl_cell0[qz], cl[qa].sq_off, k1});
+                                                 (int)c->cl_cell0[qz], cl[qa].sq_off, k1, mp[c->cl_cell0[qa]],
+                                                 mp[c->cl_cell0[qz]]});
                 qa = qz;
             }
         }
@@ -3658,6 +3787,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     c->tune.persistent = 0;
     c->tune.streams = 1;
     c->serial_groups = pick_serial_groups(c);
+    if (e == hipSuccess && use_team(c) && c->slots_host.size() > 1 && ensure_save(c) != BT_OK) e = hipErrorOutOfMemory;
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, lrec.data(), sizeof(LiveRec) * lrec.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
@@ -3704,7 +3834,7 @@ int bt_destroy(bt_ctx* c) {
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     void* ptrs[] = {c->tiles, c->mrec, c->rvol, c->c_cell_b, c->c_lag_b, c->vm_b, c->c_mid, c->fsa, c->fch, c->u, c->u_b, c->rates, c->c_env_b,
                     c->sq_live, c->live_flag, c->flags, c->bad_step, c->step_ctr, c->kcl, c->env_tiles,
-                    c->vm_prev, c->net, c->ctl, c->slots, c->phib_stage, c->phib_prev};
+                    c->vm_prev, c->net, c->ctl, c->slots, c->save, c->phib_stage, c->phib_prev};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (void* q : c->obs_alloc) (void)hipFree(q);

@@ -1,0 +1,84 @@
+"""After a NaN every cluster of a batch is at the step that produced the first of
+them, whichever way the steps ran: with NaNs that come up at different steps in
+different clusters, the state, the gates and the fields are those of separate
+launches of the three kernels over the whole batch, bit for bit."""
+
+import numpy as np
+import pytest
+
+from betse_amd.batch import batched_worlds
+from betse_amd.channels import draw_channel_state
+from betse_amd.exceptions import BetseSimUnstableException
+from tests.test_gpu_configs import batch, say
+
+pytestmark = pytest.mark.gpu
+
+SEPARATE = {"persistent": 0}
+
+
+def everything(b):
+    b.stream.synchronize()
+    keys = ("c_cell", "c_lag", "vm_cell", "c_env", "E_x", "E_y", "v_env") + (("gates",) if len(b.states[0].channel_specs) else ())
+    return {k: b._dev[k].cpu().numpy().copy() for k in keys}
+
+
+def far_square(b, cluster):
+    """A square without membranes, in from the world's edge (which is reset every
+    step): a NaN there reaches a membrane's square some steps later."""
+    soff = b.offsets[2]
+    ny, nx = b.worlds[cluster][1].X.shape
+    sp = b._dev["sq_ptr"].cpu().numpy()
+    k0 = int(soff[cluster])
+    empty = [r * nx + c for r in range(2, ny - 2) for c in range(2, nx - 2)
+             if sp[k0 + r * nx + c + 1] == sp[k0 + r * nx + c]]
+    return k0 + empty[0]
+
+
+def plant(b, cells, squares):
+    for q in cells:
+        b._dev["c_cell"][1, int(b.offsets[0][q]) + 3] = float("nan")
+    for q in squares:
+        b._dev["c_env"][0, far_square(b, q)] = float("nan")
+    b.torch.cuda.synchronize()
+
+
+def halted_states(worlds, flux_mode, tunings, n, cells, squares, first=None, use_graph=True):
+    runs = []
+    for tuning in tunings:
+        say(f"case: {len(worlds)} clusters, {flux_mode}, {n} steps, NaN in the cells of {cells}, in the env of "
+            f"{squares}, tuning {tuning}")
+        b = batch(worlds, flux_mode, tuning=tuning)
+        b.step_n(6)
+        plant(b, cells, squares)
+        with pytest.raises(BetseSimUnstableException) as e:
+            b.step_n(n)
+        st = everything(b)
+        with pytest.raises(BetseSimUnstableException) as e2:
+            b.step_n(4)
+        assert e2.value.step == e.value.step
+        for k, v in everything(b).items():
+            assert np.array_equal(v, st[k], equal_nan=True), k
+        runs.append((e.value.step, st))
+        b.close()
+    say(f"  first NaN at step {[r[0] for r in runs]}")
+    for step, st in runs[1:]:
+        assert step == runs[0][0]
+        for k, v in st.items():
+            assert np.array_equal(v, runs[0][1][k], equal_nan=True), k
+    return runs[0][0]
+
+
+@pytest.mark.parametrize("n", [40, 41])
+@pytest.mark.parametrize("cells,squares", [([2], []), ([], [0, 9]), ([], [5, 18])])
+def test_slots_stop_at_the_first_nan(cells, squares, n):
+    worlds = batched_worlds(n_clusters=19, cells_range=(10, 200), grid_range=(16, 33), seed=24)
+    step = halted_states(worlds, "fp64", (SEPARATE, None), n, cells, squares)
+    assert (step == 6) == bool(cells)
+
+
+@pytest.mark.parametrize("n", [40, 41])
+def test_slots_with_channels_stop_at_the_first_nan(n):
+    worlds = batched_worlds(n_clusters=9, cells_range=(10, 90), grid_range=(16, 24), seed=5, base="tiny_channels")
+    for p, c in worlds:
+        draw_channel_state(p, c.n_cells, c.n_mems)
+    assert halted_states(worlds, "fp32", (SEPARATE, None), n, [], [1, 7]) > 6
