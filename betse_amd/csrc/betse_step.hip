@@ -2202,7 +2202,7 @@ struct BackSeg {
     double* dst; const double* src; double* keep; long long n;
 };
 struct BackArgs {
-    BackSeg s[5];
+    BackSeg s[6];
 };
 __global__ void __launch_bounds__(BLOCK)
 k_copy_back(BackArgs a) {
@@ -3097,24 +3097,27 @@ static const void* team_kernel(const bt_ctx* c) {
     }
 }
 
-// the state's copy that clusters are put back from (ensure_save)
-static TeamSave save_pointers(const bt_ctx* c) {
+// the state's copy that clusters are put back from; returns its length in doubles
+static size_t save_layout(const bt_ctx* c, TeamSave* s) {
     const size_t nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->kp.n_sq;
-    TeamSave s;
-    s.c_cell = c->save;
-    s.c_lag = s.c_cell + ni * nc;
-    s.vm = s.c_lag + ni * nc;
-    s.c_env = s.vm + nc;
-    s.c_env_b = s.c_env + ni * ns;
-    s.u = s.c_env_b + ni * ns;
-    s.gates = s.u + ns;
-    return s;
+    size_t at = 0;
+    auto part = [&](size_t n) {                  // (whole 16 bytes each: k_copy_back's wide form)
+        double* p = c->save + at;
+        at += (n + 1) / 2 * 2;
+        return p;
+    };
+    s->c_cell = part(ni * nc);
+    s->c_lag = part(ni * nc);
+    s->vm = part(nc);
+    s->c_env = part(ni * ns);
+    s->c_env_b = part(ni * ns);
+    s->u = part(ns);
+    s->gates = part(2 * (size_t)c->prm.n_chan * c->prm.n_mems);
+    return at;
 }
 static int ensure_save(bt_ctx* c) {
-    if (c->save) return BT_OK;
-    const size_t nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->prm.n_squares;
-    const size_t n = (2 * ni + 1) * nc + (2 * ni + 1) * ns + 2 * (size_t)c->prm.n_chan * c->prm.n_mems;
-    HIP_TRY(c, hipMalloc((void**)&c->save, n * sizeof(double)));
+    TeamSave s;
+    if (!c->save) HIP_TRY(c, hipMalloc((void**)&c->save, save_layout(c, &s) * sizeof(double)));
     return BT_OK;
 }
 
@@ -3192,7 +3195,7 @@ static int launch_team(bt_ctx* c, int n_steps) {
     const bool several = tl.args.n_slots > 1;
     if (rc == BT_OK && several) {
         rc = ensure_save(c);
-        if (rc == BT_OK) tl.args.save = save_pointers(c);
+        if (rc == BT_OK) save_layout(c, &tl.args.save);
     }
     for (int done = 0, n = 0; rc == BT_OK && done < n_steps; done += n) {
         n = std::min(n_steps - done, TEAM_STEPS);
@@ -3236,8 +3239,17 @@ static bool streams_allowed(const bt_ctx* c, int G) { return G <= BT_MAX_STREAMS
 // 143.5 and 132.1, 400 MB 170.5 and 161.8, 468 MB (500k cells) 200.4 and 186.3
 // (three: 185.5): smaller groups also fill the GPU less well, so the second one
 // starts at 1.2 times the cache.
+//
+// When a NaN halts one group the others have finished the call or not begun it, so a
+// call first copies the state, and ends with a launch that puts all clusters at the
+// NaN's step (TEAM_REWIND; nothing without one): 85 us for 500k cells, paid back after
+// GROUP_MIN_PAIRS pairs of steps (us per step in groups and all at once, 16 steps 182.8
+// and 184.5, 50 steps 175.0 and 182.6, 200 steps 171.8 and 181.9).
 constexpr double GROUP_BYTES = 256.0 * (1 << 20);
+constexpr int GROUP_MIN_PAIRS = 8;
+constexpr int GROUP_PAIRS = 512;             // pairs of steps between two copies
 static int pick_serial_groups(const bt_ctx* c) {
+    if (!team_kernel(c)) return 1;               // (which puts the clusters back after a NaN)
     const long long ni = c->prm.n_ions;
     const long long moving = ni - (c->kcl_host.empty() ? 0 : __builtin_popcount(c->kcl_host[0].still_mem & 0xffu));
     const long long fb = c->prm.flux_mode == BT_FLUX_FP32 ? 4 : 8;
@@ -3332,20 +3344,55 @@ static int launch_graphs(bt_ctx* c, int pairs) {
     return BT_OK;
 }
 
+// one launch of k_copy_back over segments of the step's state
+static int launch_copy(bt_ctx* c, const BackArgs& a, int n_segs) {
+    const long long most = (long long)std::max(c->prm.n_cells, c->kp.n_sq) * c->prm.n_ions;
+    const unsigned nb = (unsigned)std::min<long long>((most / 2 + BLOCK - 1) / BLOCK + 1, 2048);
+    hipLaunchKernelGGL(k_copy_back, dim3(nb, n_segs), dim3(BLOCK), 0, c->stream, a);
+    HIP_TRY(c, hipGetLastError());
+    return BT_OK;
+}
+
 // vm_keep (may be NULL) receives the caller's vm_cell from before
 static int copy_back(bt_ctx* c, double* vm_keep = nullptr) {
     const long long nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->kp.n_sq;
+    // (u is copied where its steps write a workspace of their own)
     const BackArgs a = {{{c->buf.c_cell, c->c_cell_b, nullptr, ni * nc},
                          {c->buf.c_lag, c->c_lag_b, nullptr, ni * nc},
                          {c->buf.vm_cell, c->vm_b, vm_keep, nc},
                          {c->buf.c_env, c->c_env_b, nullptr, ni * ns},
                          {c->u, c->u_b, nullptr, ns}}};
-    // (u is copied where its steps write a workspace of their own)
-    const long long most = std::max(nc, ns) * ni;
-    const unsigned nb = (unsigned)std::min<long long>((most / 2 + BLOCK - 1) / BLOCK + 1, 2048);
-    hipLaunchKernelGGL(k_copy_back, dim3(nb, steps_fused(c) ? 5 : 4), dim3(BLOCK), 0, c->stream, a);
-    HIP_TRY(c, hipGetLastError());
-    return BT_OK;
+    return launch_copy(c, a, steps_fused(c) ? 5 : 4);
+}
+
+// whether replayed steps run group after group
+static bool one_after_the_other(const bt_ctx* c) { return c->tune.streams <= 1 && n_step_groups(c) > 1; }
+
+// `pairs` replayed pairs of steps; in groups one after the other, the clusters are
+// put at the step of a NaN afterwards
+static int launch_pairs(bt_ctx* c, int pairs) {
+    if (!one_after_the_other(c)) return launch_graphs(c, pairs);
+    TeamLaunch tl;
+    int rc = ensure_save(c);
+    if (rc == BT_OK) rc = team_launch_of(c, tl);
+    if (rc != BT_OK) return rc;
+    TeamSave& q = tl.args.save;
+    save_layout(c, &q);
+    tl.args.fused = steps_fused(c) ? 1 : 0;
+    const long long nc = c->prm.n_cells, ni = c->prm.n_ions, ns = c->kp.n_sq;
+    const BackArgs a = {{{q.c_cell, c->buf.c_cell, nullptr, ni * nc},
+                         {q.c_lag, c->buf.c_lag, nullptr, ni * nc},
+                         {q.vm, c->buf.vm_cell, nullptr, nc},
+                         {q.c_env, c->buf.c_env, nullptr, ni * ns},
+                         {q.c_env_b, c->c_env_b, nullptr, ni * ns},
+                         {q.u, c->u, nullptr, ns}}};
+    for (int done = 0, n = 0; rc == BT_OK && done < pairs; done += n) {
+        n = std::min(pairs - done, GROUP_PAIRS);
+        rc = launch_copy(c, a, 6);
+        if (rc == BT_OK) rc = launch_graphs(c, n);
+        if (rc == BT_OK) rc = launch_team_mode(c, tl, TEAM_REWIND, c->steps_done + 2LL * done, 2 * n);
+    }
+    return rc;
 }
 
 // scalar arguments of bt_create / bt_validate
@@ -3787,7 +3834,8 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     c->tune.persistent = 0;
     c->tune.streams = 1;
     c->serial_groups = pick_serial_groups(c);
-    if (e == hipSuccess && use_team(c) && c->slots_host.size() > 1 && ensure_save(c) != BT_OK) e = hipErrorOutOfMemory;
+    if (e == hipSuccess && ((use_team(c) && c->slots_host.size() > 1) || c->serial_groups > 1) && ensure_save(c) != BT_OK)
+        e = hipErrorOutOfMemory;
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, lrec.data(), sizeof(LiveRec) * lrec.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
@@ -3915,13 +3963,13 @@ int bt_step(bt_ctx* c, int32_t n_steps, int32_t use_graph) {
         use_graph = 0;
     }
     int pairs = n_steps / 2;
-    if (use_graph && pairs > 0) {
+    if (use_graph && pairs > 0 && (!one_after_the_other(c) || pairs >= GROUP_MIN_PAIRS)) {
         // a graph of tune.graph_pairs pairs of steps for the bulk, one of a
         // single pair for the rest; both are captured and instantiated on the
         // first call that replays graphs, so later calls only launch them
         int rc = capture_graphs(c);
         if (rc != BT_OK) return rc;
-        rc = launch_graphs(c, pairs);
+        rc = launch_pairs(c, pairs);
         if (rc != BT_OK) return rc;
     } else {
         for (int s = 0; s < pairs; ++s) {
@@ -4043,7 +4091,7 @@ int bt_capture_graphs(bt_ctx* c) {
     HIP_TRY(c, hipMalloc((void**)&save, sbytes));
     hipError_t e = state_copy(c, regions, save, false);
     if (e == hipSuccess) {
-        rc = team ? launch_team(c, 2) : launch_graphs(c, c->tune.graph_pairs > 1 ? c->tune.graph_pairs + 1 : 1);
+        rc = team ? launch_team(c, 2) : launch_pairs(c, c->tune.graph_pairs > 1 ? c->tune.graph_pairs + 1 : 1);
         c->team_warm = c->team_warm || (team && rc == BT_OK);
         if (rc == BT_OK) e = state_copy(c, regions, save, true);
     }

@@ -226,8 +226,8 @@ int bt_destroy(bt_ctx* ctx);
  * (BT_EXCHANGE_FUSED, all ions per block) on all but small problems wherever that
  * is allowed, whatever exchange_form and env_ions_per_block say; single kernels (bt_time_kernel) run
  * as the fields say. A batch larger than the Infinity Cache is stepped in
- * groups of clusters one after the other within a bt_step call; a NaN then
- * halts every group at the end of that call. */
+ * groups of clusters one after the other within a bt_step call; after a NaN
+ * all of them are put at its step. */
 typedef struct {
     int32_t mem_waves;          /* k_mem_cell wavefronts per cell tile: 1, or 2 (each a contiguous block of ions) */
     int32_t env_ions_per_block; /* ions per k_env_field block, 1..n_ions (n_ions: one block per 16x16 tile) */

@@ -42,7 +42,7 @@ def plant(b, cells, squares):
     b.torch.cuda.synchronize()
 
 
-def halted_states(worlds, flux_mode, tunings, n, cells, squares, first=None, use_graph=True):
+def halted_states(worlds, flux_mode, tunings, n, cells, squares):
     runs = []
     for tuning in tunings:
         say(f"case: {len(worlds)} clusters, {flux_mode}, {n} steps, NaN in the cells of {cells}, in the env of "
@@ -82,3 +82,46 @@ def test_slots_with_channels_stop_at_the_first_nan(n):
     for p, c in worlds:
         draw_channel_state(p, c.n_cells, c.n_mems)
     assert halted_states(worlds, "fp32", (SEPARATE, None), n, [], [1, 7]) > 6
+
+
+@pytest.fixture(scope="module")
+def large():
+    return batched_worlds(n_clusters=90, cells_range=(3800, 5000), grid_range=(100, 128), seed=11)
+
+
+@pytest.mark.parametrize("n", [40, 41])
+@pytest.mark.parametrize("cells,squares", [([2], []), ([80], []), ([], [3, 77])])
+def test_groups_stop_at_the_first_nan(large, cells, squares, n):
+    """A batch beyond the Infinity Cache, stepped in groups of clusters one after
+    the other. (Separate launches skip what of the NaN's step starts after it, so the
+    states to compare are those of a run without a NaN.) A step writes the workspace
+    and the caller's buffers in turn, and an odd call ends in the workspace."""
+    say(f"case: {len(large)} clusters in groups, {n} steps, NaN in the cells of {cells}, in the env of {squares}")
+    b = batch(large, "fp64")
+    b.step_n(6)
+    before = everything(b)
+    plant(b, cells, squares)
+    with pytest.raises(BetseSimUnstableException) as e:
+        b.step_n(n)
+    got, off, soff = everything(b), b.offsets[0], b.offsets[2]
+    b.close()
+    s = e.value.step - 6
+    written = s % 2 == (n + 1) % 2            # the step of the NaN wrote the buffers that the call ends in
+    b = batch(large, "fp64")
+    b.use_graph = False
+    b.step_n(6 + s + written)
+    clean = everything(b)
+    b.close()
+    say(f"  first NaN at step {e.value.step}")
+    assert (s == 0) == bool(cells)
+    for q in range(len(large)):
+        if q in cells + squares:
+            continue
+        for k in ("c_cell", "c_lag", "vm_cell"):
+            c = slice(int(off[q]), int(off[q + 1]))
+            assert np.array_equal(got[k][..., c], clean[k][..., c]), (q, k)
+        c = slice(int(soff[q]), int(soff[q + 1]))
+        if not written:
+            assert np.array_equal(got["c_env"][:, c], clean["c_env"][:, c]), q
+        for k in ("v_env", "E_x", "E_y"):
+            assert np.array_equal(got[k][c], before[k][c]), (q, k)
