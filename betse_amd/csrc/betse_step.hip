@@ -3535,7 +3535,10 @@ static int derive_uniform(bt_ctx* c) {
         for (size_t k = lo; k < hi && same; ++k) same = (row[k] == row[lo]);
         return same ? row[lo] : (double)NAN;
     };
-    for (KCluster& K : c->kcl_host) {
+    // (taken over as a whole at the end: after an error the context goes on as it was)
+    std::vector<KCluster> kcl = c->kcl_host;
+    bool denv_varies = false, any_phib = false;
+    for (KCluster& K : kcl) {
         for (int i = 0; i < BT_MAX_IONS; ++i) K.dm_u[i] = K.denv_u[i] = NAN;
         K.gjo_u = NAN;
         K.still_mem = 0;
@@ -3547,7 +3550,7 @@ static int derive_uniform(bt_ctx* c) {
         rc = gj ? fetch(c->buf.gjopen, p->n_mems) : fetch(c->buf.Dm + (size_t)i * p->n_mems, p->n_mems);
         if (rc != BT_OK) return rc;
         for (int q = 0; q < nq; ++q) {
-            KCluster& K = c->kcl_host[q];
+            KCluster& K = kcl[q];
             const int lo = c->cl_mem_lo[q], hi = c->cl_mem_hi[q];
             if (hi <= lo) continue;
             const double u = uniform(lo, hi);
@@ -3560,8 +3563,6 @@ static int derive_uniform(bt_ctx* c) {
                 K.still_mem |= 1u << i;
         }
     }
-    const bool varied = c->denv_varies;
-    c->denv_varies = false;
     auto squares = [&](int q, size_t& k0, size_t& k1) {
         k0 = (size_t)c->clusters[q].sq_off;
         k1 = k0 + (size_t)c->clusters[q].grid_ny * c->clusters[q].grid_nx;
@@ -3573,27 +3574,29 @@ static int derive_uniform(bt_ctx* c) {
         for (int q = 0; q < nq; ++q) {
             squares(q, k0, k1);
             const double u = uniform(k0, k1);
-            c->kcl_host[q].denv_u[i] = u;
-            c->denv_varies = c->denv_varies || isnan(u);
+            kcl[q].denv_u[i] = u;
+            denv_varies = denv_varies || isnan(u);
         }
     }
-    c->any_phib = false;
     if (c->buf.Phi_b) {
         rc = fetch(c->buf.Phi_b, p->n_squares);
         if (rc != BT_OK) return rc;
         for (int q = 0; q < nq; ++q) {
-            KCluster& K = c->kcl_host[q];
+            KCluster& K = kcl[q];
             squares(q, k0, k1);
             for (size_t k = k0; k < k1 && !K.phib; ++k) K.phib = (row[k] != 0.0);
             if (K.phib) K.still_mem |= PHIB_BIT;
             if (K.phib && p->n_chan > 0)
                 return set_err(c, BT_EINVAL, "an applied boundary voltage (Phi_b) with voltage-gated channels is not "
                                              "supported (their gating rates are per cell)");
-            c->any_phib = c->any_phib || K.phib;
+            any_phib = any_phib || K.phib;
         }
     }
     // the captured step graphs hold the env kernel of the other kind
-    if (c->denv_varies != varied) drop_graphs(c);
+    if (c->denv_varies != denv_varies) drop_graphs(c);
+    c->kcl_host.swap(kcl);
+    c->denv_varies = denv_varies;
+    c->any_phib = any_phib;
     return BT_OK;
 }
 
