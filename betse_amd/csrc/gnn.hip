@@ -1070,6 +1070,7 @@ int64_t bt_gnn_cache_len(int32_t hidden, int32_t n_layers, int32_t n, int32_t ke
 }
 
 int64_t bt_gnn_backward_len(int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers, int32_t n) {
+    if (n < 1) return 0;                                        // (bt_gnn_backward refuses it)
     int64_t len = (int64_t)n * hidden * (n_layers + 4);         // dz of every layer, dH, two of G
     const int64_t H = hidden;
     const int64_t sums = (n + COL_ROWS - 1) / COL_ROWS;

@@ -444,7 +444,8 @@ int bt_gnn_adam_all(float* const* p, const float* const* g, float* const* m, flo
  * bt_gnn_forward leaves in cache (bt_gnn_cache_len floats, 16-byte aligned),
  * with keep, what the backward pass reads; n nodes of f_in features in, n of
  * f_out in y. bt_gnn_backward reads the first n of the cache's cache_n nodes
- * and writes every gradient; ws: bt_gnn_backward_len floats, 16-byte aligned. */
+ * and writes every gradient; ws: bt_gnn_backward_len floats, 16-byte aligned.
+ * Without nodes (n < 1) the length is 0 and both passes return BT_EINVAL. */
 int bt_gnn_layered(int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers);
 int64_t bt_gnn_cache_len(int32_t hidden, int32_t n_layers, int32_t n, int32_t keep);
 int64_t bt_gnn_backward_len(int32_t f_in, int32_t f_out, int32_t hidden, int32_t n_layers, int32_t n);
