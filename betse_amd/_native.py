@@ -153,6 +153,8 @@ SIGNATURES = {
     "bt_refresh_params": (ctypes.c_int, [_vp]),
     "bt_stage_boundary": (ctypes.c_int, [_vp, _vp]),
     "bt_get_tuning": (ctypes.c_int, [_vp, ctypes.POINTER(BtTuning)]),
+    "bt_running_tuning": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(BtTuning),
+                                         ctypes.POINTER(ctypes.c_int32)]),
     "bt_set_tuning": (ctypes.c_int, [_vp, ctypes.POINTER(BtTuning)]),
     "bt_autotune": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(BtTuning), ctypes.POINTER(ctypes.c_double),
                                     ctypes.c_int32]),

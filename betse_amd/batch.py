@@ -199,9 +199,19 @@ class BatchSimulator(DeviceFetch):
         self._check(self._lib.bt_get_tuning(self._ctx, ctypes.byref(t)))
         return t.as_dict()
 
+    def running_tuning(self) -> dict:
+        """The launch variants the steps run with (``bt_running_tuning``: those of
+        ``get_tuning`` once any are forced), and into how many groups of clusters
+        stepped one after the other (``serial_groups``)."""
+        t, groups = _native.BtTuning(), ctypes.c_int32(1)
+        self._check(self._lib.bt_running_tuning(self._ctx, 1 if self.use_graph else 0, ctypes.byref(t),
+                                                ctypes.byref(groups)))
+        return dict(t.as_dict(), serial_groups=groups.value)
+
     def set_tuning(self, tuning: dict) -> None:
         """Force the step kernels' launch variants (``bt_set_tuning``); keys of
-        ``_native.BtTuning``, missing ones keep their current value."""
+        ``_native.BtTuning``, missing ones keep the value ``get_tuning`` reports.
+        Until the first call the steps run as ``running_tuning`` reports."""
         cur = self.get_tuning()
         cur.update(tuning)
         t = _native.BtTuning(**cur)

@@ -3052,7 +3052,7 @@ static hipStream_t group_stream(bt_ctx* c, int G, int g) {
 // which: -1 all, 0 membrane/cell, 1 env field+diffusion, 2 exchange, 3 field only
 static void enqueue_step(bt_ctx* c, int parity, int which = -1, int G = 1, int g = 0) {
     const bt_obs* ob = c->capture;
-    const bool fused = (which < 0) ? steps_fused(c) : c->tune.exchange_form == BT_EXCHANGE_FUSED;
+    const bool fused = steps_fused(c);
     const StepArgs a = step_args(c, parity, ob, which < 0 ? 1 : 0, G, g, fused);
     const Span sp = group_span(c, G, g);
     hipStream_t st = group_stream(c, G, g);
@@ -3995,6 +3995,18 @@ int bt_step(bt_ctx* c, int32_t n_steps, int32_t use_graph) {
 int bt_get_tuning(const bt_ctx* c, bt_tuning* out) {
     if (!c || !out) return BT_EINVAL;
     *out = c->tune;
+    return BT_OK;
+}
+
+int bt_running_tuning(const bt_ctx* c, int32_t use_graph, bt_tuning* out, int32_t* serial_groups) {
+    if (!c || !out || !serial_groups) return BT_EINVAL;
+    *out = c->tune;
+    out->persistent = use_team(c) ? 1 : 0;
+    if (steps_fused(c)) {
+        out->exchange_form = BT_EXCHANGE_FUSED;
+        out->env_ions_per_block = c->prm.n_ions;
+    }
+    *serial_groups = (use_graph && !out->persistent && one_after_the_other(c)) ? n_step_groups(c) : 1;
     return BT_OK;
 }
 

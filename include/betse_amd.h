@@ -224,8 +224,9 @@ int bt_destroy(bt_ctx* ctx);
  * only the division of the work between wavefronts and blocks changes. Until
  * one of the two is called, whole steps run with the exchange in the env kernel
  * (BT_EXCHANGE_FUSED, all ions per block) on all but small problems wherever that
- * is allowed, whatever exchange_form and env_ions_per_block say; single kernels (bt_time_kernel) run
- * as the fields say. A batch larger than the Infinity Cache is stepped in
+ * is allowed, and small problems in the persistent kernel, whatever
+ * exchange_form, env_ions_per_block and persistent say: bt_get_tuning reports the
+ * fields, bt_running_tuning what runs. A batch larger than the Infinity Cache is stepped in
  * groups of clusters one after the other within a bt_step call; after a NaN
  * all of them are put at its step. */
 typedef struct {
@@ -286,6 +287,10 @@ int bt_stage_boundary(bt_ctx* ctx, const double* Phi_b_next);
 int bt_capture_graphs(bt_ctx* ctx);
 
 int bt_get_tuning(const bt_ctx* ctx, bt_tuning* out);
+/* The variants that bt_step runs (with use_graph as there); given to
+ * bt_set_tuning they are what it goes on running. *serial_groups: into how many
+ * groups of clusters, stepped one after the other, long calls split a batch. */
+int bt_running_tuning(const bt_ctx* ctx, int32_t use_graph, bt_tuning* out, int32_t* serial_groups);
 int bt_set_tuning(bt_ctx* ctx, const bt_tuning* tuning);
 
 /* Time each kernel variant over n_launches launches (HIP events on the
