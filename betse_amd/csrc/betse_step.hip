@@ -3205,10 +3205,11 @@ static int launch_team(bt_ctx* c, int n_steps) {
     return rc;
 }
 
-// whether bt_step runs its steps in the team kernel
-static bool use_team(const bt_ctx* c) {
+// whether bt_step runs its steps in the team kernel: where the caller forced it, or
+// picked for a small problem in place of replayed graphs
+static bool use_team(const bt_ctx* c, int use_graph) {
     if (!c->auto_pick) return c->tune.persistent != 0;
-    return c->team_fits && team_kernel(c) != nullptr;
+    return use_graph && c->team_fits && team_kernel(c) != nullptr;
 }
 
 static void drop_graphs(bt_ctx* c) {
@@ -3837,7 +3838,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     c->tune.persistent = 0;
     c->tune.streams = 1;
     c->serial_groups = pick_serial_groups(c);
-    if (e == hipSuccess && ((use_team(c) && c->slots_host.size() > 1) || c->serial_groups > 1) && ensure_save(c) != BT_OK)
+    if (e == hipSuccess && ((use_team(c, 1) && c->slots_host.size() > 1) || c->serial_groups > 1) && ensure_save(c) != BT_OK)
         e = hipErrorOutOfMemory;
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, lrec.data(), sizeof(LiveRec) * lrec.size(), hipMemcpyHostToDevice);
@@ -3952,7 +3953,7 @@ int bt_step(bt_ctx* c, int32_t n_steps, int32_t use_graph) {
         }
         return bt_step(c, n_steps - 1, use_graph);
     }
-    if (use_team(c)) {
+    if (use_team(c, use_graph)) {
         // (a captured launch would be replayed on control words that are not its
         // own: under the caller's capture the steps are separate launches)
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -4001,7 +4002,7 @@ int bt_get_tuning(const bt_ctx* c, bt_tuning* out) {
 int bt_running_tuning(const bt_ctx* c, int32_t use_graph, bt_tuning* out, int32_t* serial_groups) {
     if (!c || !out || !serial_groups) return BT_EINVAL;
     *out = c->tune;
-    out->persistent = use_team(c) ? 1 : 0;
+    out->persistent = use_team(c, use_graph) ? 1 : 0;
     if (steps_fused(c)) {
         out->exchange_form = BT_EXCHANGE_FUSED;
         out->env_ions_per_block = c->prm.n_ions;
@@ -4089,7 +4090,7 @@ static hipError_t state_copy(bt_ctx* c, const std::vector<std::pair<void*, size_
 int bt_capture_graphs(bt_ctx* c) {
     if (!c) return BT_EINVAL;
     // (steps that run in the team kernel replay no graphs: it is launched once)
-    const bool team = use_team(c);
+    const bool team = use_team(c, 1);
     bool fresh = team && !c->team_warm;
     for (int g = 0; g < n_step_groups(c) && !team; ++g)
         fresh = fresh || !c->gexec[g] || (c->tune.graph_pairs > 1 && !c->gexec_n[g]);
@@ -4369,7 +4370,7 @@ int bt_step_observed(bt_ctx* c, int32_t n_steps, int32_t use_graph, const bt_obs
         --n_steps;
     }
     const int ahead = n_steps - 1;
-    const int odd = use_team(c) ? 0 : ahead & 1;     // (the team kernel takes either)
+    const int odd = use_team(c, use_graph) ? 0 : ahead & 1;     // (the team kernel takes either)
     if (ahead > 0) {
         // keep the graph on the caller buffers: an even number of graph steps, then eager ones
         int rc = bt_step(c, ahead - odd, use_graph);

@@ -241,7 +241,7 @@ typedef struct {
                                    blocks of each XCD form a team that steps a share of the clusters (barriers
                                    between a step's phases within the XCD; 5 or 6 ions, no reaction network);
                                    0: replayed step graphs, or the persistent kernel where a context's tuning has
-                                   been left alone and the clusters are small */
+                                   been left alone, the clusters are small and bt_step is called with use_graph */
     int32_t streams;            /* 1..BT_MAX_STREAMS: with replayed graphs, the clusters of a batch are split
                                    into this many groups of about equal cells, each stepped by its own graphs
                                    on its own stream, so that one group's kernels run in the ramps and tails of
@@ -317,8 +317,10 @@ int bt_update_v(bt_ctx* ctx);
 /* Enqueue n_steps iterations of the _run_sim_core_loop body (sim.py:1169-1366):
  * NaK pump, per-ion GHK + gap-junction fluxes, env Nernst-Planck update,
  * Ca pump, voltage-gated channels (networks.py:3115-3215), cell/env
- * concentration update, update_V, NaN checks. Steps are
- * replayed from a captured hipGraph when use_graph != 0. Asynchronous. */
+ * concentration update, update_V, NaN checks. With use_graph != 0 the steps are
+ * replayed from captured hipGraphs, or run in the persistent kernel where that is
+ * picked for a small problem; with 0 every kernel of every step is a launch of its
+ * own. A forced persistent kernel (bt_tuning) runs them either way. Asynchronous. */
 int bt_step(bt_ctx* ctx, int32_t n_steps, int32_t use_graph);
 
 /* Attach a reaction network to the step (NULL net detaches it). c_net is the

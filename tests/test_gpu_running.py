@@ -46,3 +46,21 @@ def test_kernels_are_timed_as_the_steps_run_them():
     say(f"case: kernels of fused steps, env {env * 1e3:.1f} us, exchange {ex * 1e3:.1f} us")
     assert ex < 0.2 * env
     b.close()
+
+
+def test_without_graphs_every_kernel_is_a_launch():
+    """use_graph = 0 on a small problem: separate launches, with the same bits."""
+    worlds = batched_worlds(seed=13, **SMALL)
+    states = []
+    for use_graph in (True, False):
+        b = batch(worlds, "fp64")
+        b.use_graph = use_graph
+        say(f"case: use_graph {use_graph}, running {b.running_tuning()}")
+        assert b.running_tuning()["persistent"] == int(use_graph)
+        b.step_n(23)
+        states.append(state(b))
+        b.set_tuning({"persistent": 1})
+        assert b.running_tuning()["persistent"] == 1
+        b.close()
+    for k, v in states[0].items():
+        assert np.array_equal(v, states[1][k]), k
