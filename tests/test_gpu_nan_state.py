@@ -77,6 +77,14 @@ def test_slots_stop_at_the_first_nan(cells, squares, n):
 
 
 @pytest.mark.parametrize("n", [40, 41])
+@pytest.mark.parametrize("cells,squares", [([0], []), ([], [0])])
+def test_one_cluster_stops_at_its_nan(cells, squares, n):
+    worlds = batched_worlds(n_clusters=1, cells_range=(60, 70), grid_range=(33, 34), seed=2)
+    step = halted_states(worlds, "fp64", (SEPARATE, None, {"persistent": 1}), n, cells, squares)
+    assert (step == 6) == bool(cells)
+
+
+@pytest.mark.parametrize("n", [40, 41])
 def test_slots_with_channels_stop_at_the_first_nan(n):
     worlds = batched_worlds(n_clusters=9, cells_range=(10, 90), grid_range=(16, 24), seed=5, base="tiny_channels")
     for p, c in worlds:
