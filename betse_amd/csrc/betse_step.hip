@@ -3252,10 +3252,13 @@ constexpr int GROUP_PAIRS = 512;             // pairs of steps between two copie
 static int pick_serial_groups(const bt_ctx* c) {
     if (!team_kernel(c)) return 1;               // (which puts the clusters back after a NaN)
     const long long ni = c->prm.n_ions;
-    const long long moving = ni - (c->kcl_host.empty() ? 0 : __builtin_popcount(c->kcl_host[0].still_mem & 0xffu));
+    long long flux_values = 0;                   // (a still ion's row is not written)
+    for (size_t q = 0; q < c->kcl_host.size(); ++q)
+        flux_values += (long long)std::max(c->cl_mem_hi[q] - c->cl_mem_lo[q], 0) *
+                       (ni - __builtin_popcount(c->kcl_host[q].still_mem & 0xffu));
     const long long fb = c->prm.flux_mode == BT_FLUX_FP32 ? 4 : 8;
     const long long bytes = (long long)c->prm.n_cells * (32 * ni + 40) +
-                            (long long)c->prm.n_mems * (long long)(sizeof(MemRec) + 8 + fb * moving) +
+                            (long long)c->prm.n_mems * (long long)(sizeof(MemRec) + 8) + fb * flux_values +
                             (long long)c->prm.n_squares * (16 * ni + 21);
     int G = (int)std::min(ceil((double)bytes / GROUP_BYTES - 0.2), (double)MAX_GROUPS);
     while (G > 1 && !groups_allowed(c, G)) --G;

@@ -31,3 +31,19 @@ def test_groups_are_the_whole_batch(worlds, flux_mode, copies, groups):
         b.close()
     for k in runs[0]:
         assert np.array_equal(runs[0][k], runs[1][k]), k
+
+
+def test_the_split_does_not_depend_on_the_order_of_the_clusters(worlds):
+    """A cluster in which fewer ions move, first and last, in a batch of just over 2.2
+    times the cache."""
+    p, cells = worlds[0]
+    p = p.copy()
+    p.mem_perms = dict(p.mem_perms, Cl=0.0)
+    rest = (worlds * 2)[1:]
+    groups = []
+    for w in ([(p, cells)] + rest, rest + [(p, cells)]):
+        b = batch(w, "fp32")
+        groups.append(b.running_tuning()["serial_groups"])
+        say(f"case: a cluster without Cl flux at {'the start' if w[0][0] is p else 'the end'}: {groups[-1]} groups")
+        b.close()
+    assert groups == [3, 3]
