@@ -225,7 +225,9 @@ __device__ __forceinline__ v4s bf16x4(v4f x) {
 
 // s / d for an integer d < 2^26, r = 1.0 / d: a quotient of 24 bits by d is never so
 // near the middle of two floats that the product's error of 2^-52 could cross it, so
-// it rounds as the division does (three instructions instead of eleven)
+// it rounds as the division does (three instructions instead of eleven). Below 2^-126,
+// where floats have fewer bits, a quotient can lie in the middle and then be rounded up
+// where the division rounds down, or down for up (the first such d is 98).
 __device__ __forceinline__ float div_int(float s, double r) { return (float)((double)s * r); }
 
 __device__ __forceinline__ v4f mfma16(v4s a, v4s b, v4f c) {
@@ -266,6 +268,14 @@ __device__ __forceinline__ void stage_weights(v4s* s, const float* W, int sk, in
     }
 }
 
+// The lanes of a wavefront exchange values through LDS: what they stored before is what
+// they load after. (It executes in order; this keeps the compiler from reordering.)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // A wavefront's 16 nodes by H = 16 HB columns in two layouts: rows, where lane l
 // holds columns 4 c4 .. 4 c4 + 3 (c4 = l % LR) of node it RI + l / LR in element it,
 // consecutive lanes on consecutive addresses; and operands, where it holds columns
@@ -292,15 +302,19 @@ struct Tile {
     // rows to BF16 operands (half 0 or 1 of the LDS)
     __device__ __forceinline__ void operands(v4s (&o)[HB], const v4f (&x)[HB], int half) {
         v4s_lds* t = b + half * LDS;
+        wave_sync();
 #pragma unroll
         for (int it = 0; it < HB; ++it) t[(it * RI + g) * PITCH + c4] = bf16x4(x[it]);
+        wave_sync();
 #pragma unroll
         for (int ks = 0; ks < HB; ++ks) o[ks] = t[node * PITCH + 4 * ks + kq];
     }
     // results to rows
     __device__ __forceinline__ void rows(v4f (&x)[HB], const v4f (&acc)[HB]) {
+        wave_sync();
 #pragma unroll
         for (int ct = 0; ct < HB; ++ct) f[node * PITCH + 4 * ct + kq] = acc[ct];
+        wave_sync();
 #pragma unroll
         for (int it = 0; it < HB; ++it) x[it] = f[(it * RI + g) * PITCH + c4];
     }

@@ -443,7 +443,8 @@ int bt_gnn_adam(float* p, const float* g, float* m, float* v, int64_t count, flo
 int bt_gnn_adam_all(float* const* p, const float* const* g, float* const* m, float* const* v, const int64_t* counts,
                     int32_t n_tensors, float lr, float b1, float b2, float eps, int32_t t, void* stream);
 /* Whole passes of the network, a kernel per layer: bit for bit the results of
- * the calls above composed layer by layer. bt_gnn_layered: 1 where they exist
+ * the calls above composed layer by layer (but for means over 98 neighbours or more
+ * that lie below 2^-126 and midway between two floats). bt_gnn_layered: 1 where they exist
  * (hidden 16, 32 or 64, f_out <= 16, f_in <= 128, n_layers 1..15), else 0 and
  * the passes return BT_EINVAL, as they do for n * hidden >= 2^30. params and grads (host arrays of device
  * pointers): W_in, b_in, then W and b of each layer, then W_out, b_out.
