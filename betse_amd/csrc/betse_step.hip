@@ -3604,6 +3604,16 @@ static int derive_uniform(bt_ctx* c) {
     return BT_OK;
 }
 
+// the caller's membranes and volumes as k_mem_cell reads them
+static hipError_t take_geometry(bt_ctx* c) {
+    const bt_buffers& b = c->buf;
+    const int nm = c->prm.n_mems, nc = c->prm.n_cells;
+    hipLaunchKernelGGL(k_mem_records, dim3(grid_blocks(nm)), dim3(BLOCK), 0, c->stream, b.nn_mem, b.nn_cell, b.mem_sq,
+                       b.mem_pos, c->mrec, nm);
+    hipLaunchKernelGGL(k_reciprocal, dim3(grid_blocks(nc)), dim3(BLOCK), 0, c->stream, b.cell_vol, c->rvol, nc);
+    return hipGetLastError();
+}
+
 int bt_refresh_params(bt_ctx* c) {
     if (!c) return BT_EINVAL;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -3612,6 +3622,8 @@ int bt_refresh_params(bt_ctx* c) {
     int rc = derive_uniform(c);
     if (rc != BT_OK) return rc;
     HIP_TRY(c, hipMemcpy(c->kcl, c->kcl_host.data(), sizeof(KCluster) * c->kcl_host.size(), hipMemcpyHostToDevice));
+    HIP_TRY(c, take_geometry(c));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
     return BT_OK;
 }
 
@@ -3846,13 +3858,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
     if (e == hipSuccess && !sq_live.empty())
         e = hipMemcpy(c->sq_live, lrec.data(), sizeof(LiveRec) * lrec.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->tiles, trec.data(), trec.size() * sizeof(TileRec), hipMemcpyHostToDevice);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_mem_records, dim3(grid_blocks(p->n_mems)), dim3(BLOCK), 0, c->stream, b->nn_mem, b->nn_cell,
-                           b->mem_sq, b->mem_pos, c->mrec, p->n_mems);
-        hipLaunchKernelGGL(k_reciprocal, dim3(grid_blocks(p->n_cells)), dim3(BLOCK), 0, c->stream, b->cell_vol, c->rvol,
-                           p->n_cells);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess) e = take_geometry(c);
     if (e == hipSuccess) e = hipMemcpy(c->live_flag, live_flag.data(), ns, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(c->kcl, c->kcl_host.data(), sizeof(KCluster) * (size_t)n_clusters, hipMemcpyHostToDevice);

@@ -187,9 +187,10 @@ typedef struct {
  * status words) on the current device. It reads tile_ptr, mem_ptr,
  * tile_cluster, sq_ptr, sq_has_mem, Dm, gjopen and D_env with blocking
  * copies, so their contents must be complete when it is called. Dm, gjopen
- * and D_env are read once here (a cluster whose values are uniform gets them
- * as constants); they do not change within a phase on this path, and a caller
- * that changes them creates a new context. Between calls the caller's state buffers hold the
+ * and D_env are read here (a cluster whose values are uniform gets them as
+ * constants), and nn_mem, nn_cell, mem_sq, mem_pos and cell_vol taken over into
+ * records of the steps' own: a caller that changes any of these between steps
+ * calls bt_refresh_params. Between calls the caller's state buffers hold the
  * state (the workspace copies are internal).
  * `stream` is a hipStream_t (may be NULL for the default stream; graphs need a
  * non-default stream). Replaces the state set-up of init_core/init_dynamics
@@ -259,7 +260,7 @@ typedef struct {
  * D_env (or Phi_b) buffers bound at bt_create, this re-derives the per-cluster
  * constants bt_create took from them (values that are one over a cluster, ions
  * without membrane flux, clusters with an applied voltage), so the next steps
- * use the new values; captured graphs stay valid. BT_EINVAL for a nonzero
+ * use the new values, and those in nn_mem, nn_cell and cell_vol; captured graphs stay valid. BT_EINVAL for a nonzero
  * Phi_b with voltage-gated channels. Synchronous. */
 int bt_refresh_params(bt_ctx* ctx);
 
