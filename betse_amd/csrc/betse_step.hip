@@ -68,8 +68,9 @@ constexpr int TY = 16, TX = 16;          // k_env_field tile
 // them per problem). Until the caller forces a variant, and where no membrane law
 // reads the post-diffusion env, whole steps from FUSE_TILES cell tiles on have the
 // exchange in the env kernel (us per step with it and, in brackets, as a launch of
-// its own with the better of the splits below: 532 tiles 17.2 (17.6), 2,193 tiles
-// 20.2 (25.5), 5,428 30.0 (36.2), 19,239 67.6 (81.6), 50,081 187 (231)). Elsewhere,
+// its own with the better of the splits below: 260 tiles 18.1 (18.2), 322 16.3 (17.1),
+// 402 17.2 (17.2), 480 16.8 (16.8), 562 16.9 (17.2), 2,193 20.2 (25.5), 5,428 30.0
+// (36.2), 19,239 67.6 (81.6), 50,081 187 (231); FP32 flux 480 tiles 16.3 (17.3)). Elsewhere,
 // below ENV_SPLIT_TILES env tiles k_env_field splits its blocks by pairs of ions
 // (measured: pairs of ions win by 35% at 256 tiles, one block per tile by 10% at
 // 1024); below EX_SPLIT_SQUARES squares with membranes k_env_exchange runs one
@@ -482,7 +483,7 @@ __device__ __forceinline__ void gate_rates(int kind, double V, double& mInf, dou
 // membrane but the tile's first that is the first of its cell, moved down by
 // one, so the number of its bits below a lane is the cell of that lane's
 // membrane within the tile; `inv_nc` = floor(2^16 / cells) + 1, whose product
-// with a t < 256 over 2^16 is t / cells (cells <= 32).
+// with a t < 2048 over 2^16 is t / cells (cells <= 32).
 struct TileRec {
     int c0, m0, n_cells, n_mems, cluster, inv_nc;
     unsigned long long starts;
@@ -537,12 +538,15 @@ struct MemLds {
     unsigned flag_bit;
 };
 constexpr int CHV = 6;        // a_m, b_m, a_h, b_h, modulator, cell concentration
+static_assert(BT_TILE_CELLS <= 32 && BT_TILE_CELLS * BT_MAX_CHAN * CHV < 2048 && BT_TILE_CELLS * BT_MAX_IONS + 4 * TMB < 2048,
+              "the quotients by inv_nc");
 
 // Synchronisation of the lanes that share a tile's LDS: the block (WSYNC
-// false: the tile's one or two wavefronts are the block; an LDS-only barrier,
-// so the tile's flux stores need not have landed) or the wavefront alone (WSYNC true: in the persistent step kernel every wavefront of a block
-// works on a tile of its own; the lanes of a wavefront run in step and its LDS
-// accesses complete in order, so a compiler fence is all it needs).
+// false: the tile's wavefronts are the block, or a team block's tiles pass the same
+// barriers; an LDS-only barrier, so the tile's flux stores need not have landed) or
+// the wavefront alone (WSYNC true: every wavefront of a team block has a tile of its
+// own; the lanes of a wavefront run in step and its LDS accesses complete in order,
+// so a compiler fence is all it needs).
 template <bool WSYNC>
 __device__ __forceinline__ void tile_sync() {
     if constexpr (WSYNC) {
@@ -557,18 +561,21 @@ __device__ __forceinline__ void tile_sync() {
 // The work of wavefront W of a k_mem_cell tile. WT >= 0 is W at compile time, so
 // that every ion index below is a constant (the per-ion kernel parameters then
 // load once, up front); WT = -1 takes it from w (the team kernel, where one code
-// for both wavefronts is worth more).
+// for the tile's three wavefronts is worth more).
 //
-// What bounds it is the vector-memory address unit: about 16 cycles for every
-// wavefront-wide gather, whatever it hits (measured 79 % busy with 36 loads and
-// 15 stores per tile). So whatever is per cell is loaded once per cell, a lane
+// A wavefront-wide gather takes the vector-memory address unit about 16 cycles,
+// whatever it hits, and with 36 loads and 15 stores per tile that unit was what bound
+// the kernel (79 % busy). So whatever is per cell is loaded once per cell, a lane
 // per (ion, cell) (one load for all ions of a tile of ten cells, where a load
 // per membrane and ion took NI), handed to the membranes through LDS, and the
 // cells' new state is summed and stored by the same lanes; a membrane's indices
-// are one 16-byte record, and the Na/K pump shares its ions' gathers: 23 vector
-// accesses a tile where there were 51 (five ions, no channels). 53k cells on the
+// are one 16-byte record, and the Na/K pump shares its ions' gathers: 17 loads and 7
+// stores a tile (five ions, no channels), the unit 63 % busy. 53k cells on the
 // FP32-flux path 13.8 -> 11.4 us; 23k cells with two channels, two wavefronts a
-// tile, 15.2 -> 13.5 us; 105k cells with three channels 51.4 -> 50.2 us.
+// tile, 15.2 -> 13.5 us; 105k cells with three channels 51.4 -> 50.2 us. What bounds it
+// now on large problems is the wavefronts a CU holds (LDS rows) and the writes to HBM:
+// wavefronts wait 54 % of their time, and 2 KB more LDS a block took the 500k-cell batch
+// from 109 to 117 us. On small ones it is one wavefront's chain.
 template <int NI, typename FT, int WG, int WT, bool OBS, bool WSYNC = false, bool SC1 = false, typename MA, typename KP>
 __device__ __forceinline__ void mem_cell_wave(MA& A, KP& P, int tile, const MemLds& L, int w = 0, bool stop = false) {
     const int W = WT >= 0 ? WT : w;
@@ -944,9 +951,6 @@ struct FieldArgs {
     long long* step_ctr = nullptr; unsigned ctr_mask = 0; int count_step = 0;
 };
 
-// RATES: also the gating rates (diffuse mode with channels). Divisions by the
-// grid spacing and by kT are products by their FP64 reciprocals (an FP64 ulp
-// each).
 // the gate-update coefficients of channel ch in a cell from the
 // cell's Vmem vmc: the channel's rates at Vmem carrying the n_ions + ch
 // nonces of the membrane stage, and update_mh (channelsabc.py:54-58),
@@ -992,14 +996,14 @@ __device__ __forceinline__ double neg_flux_sum(const void* fsa, int fsa32, size_
 }
 
 // FUSE: the membrane fluxes of FUSE_I ions of a square are summed together,
-// FUSE_W membranes of each loaded at a time (16 loads in flight)
+// FUSE_W membranes of each loaded at a time (four 16-byte loads in flight, or two of
+// FP32 fluxes)
 constexpr int FUSE_I = 2;
 constexpr int FUSE_W = 4;
 
 // Four consecutive fluxes of a row from an address aligned to one of them, by
 // 16-byte loads: the vector-memory address unit takes 16 cycles for a
-// wavefront's gather whether a lane asks for 8 bytes or 16, and it is what
-// bounds these kernels. A run may reach FSA_PAD values past a square's own
+// wavefront's gather whether a lane asks for 8 bytes or 16. A run may reach FSA_PAD values past a square's own
 // membranes (into the next square's, the next row, or the allocation's padding);
 // those are not used.
 constexpr int FSA_PAD = FUSE_W - 1;
@@ -1102,8 +1106,9 @@ __device__ __forceinline__ EnvAxis env_axis_inner(double rd2) {
 
 // One env tile's work for the ions [i_lo, i_lo + ipb) (those there are), for
 // which its tile's field is rebuilt, by thread tid of 256, with the block's LDS at
-// lds (ENV_LDS doubles). With RATES the block's threads also
-// evaluate the gating-rate items rate_first, rate_first + rate_stride, ...
+// lds (ENV_LDS doubles). With RATES (diffusion with channels) the block's threads also
+// evaluate the gating-rate items rate_first, rate_first + rate_stride, ... Divisions by
+// the grid spacing and by kT are products by their FP64 reciprocals (an FP64 ulp each).
 //
 // A thread owns one square. The divergence at a square needs the fluxes of its
 // four neighbours only, and each of those the two concentrations beside it, so
@@ -1254,9 +1259,8 @@ __device__ __forceinline__ void env_field_tile(FA& A, KP& P, int tile_id, int i_
         t[it] = ld_pair<TEAM>(A.u + so + clampi(rr, ny) * nx + clampi(cc, nx));
     }
 
-    // FUSE: the square's membrane-flux sums of every moving ion, taken here, all
-    // ions' loads in flight together, while the field's loads are too; each
-    // thread keeps its own in LDS for the ion loop
+    // FUSE: the square's membrane-flux sums of every moving ion, taken here, while the
+    // field's loads are in flight; each thread keeps its own in LDS for the ion loop
     double* s_sum = s_du + BT_MAX_IONS;
     if (FUSE && live_b != 0) {
         const unsigned moving = ~still_mem & ((1u << P.n_ions) - 1u);
@@ -1518,7 +1522,7 @@ __device__ __forceinline__ void advance_step(const ExArgs& A) {
 
 // The negated sums over a square's membranes [a, b), in membrane order, of a flux row
 // and (chan) a channel's row: both rows' next eight values are loaded together, in
-// 16-byte runs. Their latency is what this kernel takes (waves wait 75 % of the time):
+// 16-byte runs. Their latency is what this kernel takes (waves wait 69-78 % of the time):
 // 105k cells with three channels 12.9 -> 12.2 us, 23k with two 4.4 -> 3.9 (one row after
 // the other in 8-byte loads before, the halt flag waited for first).
 template <typename T>
@@ -2290,8 +2294,9 @@ constexpr int TB = 1024;                     // threads per block
 constexpr int TW = TB / TMB;                 // wavefronts per block
 static_assert(TB == TSUB * TY * TX, "a block's quarters are env tiles' threads");
 // Wavefronts that share a tile's five or six ions. The membrane phase is a chain of
-// double-precision arithmetic on few wavefronts: us per step with two / three, 362
-// cells 10.7 / 10.2, 37 tiles on 32x32 9.2 / 8.5, 145 tiles 13.0 / 12.3.
+// double-precision arithmetic on few wavefronts: us per step with two / three (one
+// process each; another day's run of the same sizes differs by up to 0.7), 362 cells
+// 10.7 / 10.2, 37 tiles on 32x32 9.2 / 8.5, 145 tiles 13.0 / 12.3.
 constexpr int TSPLIT = 3;
 constexpr int TEAM_BLOCKS = 32;              // blocks of a full team: the CUs of an XCD
 constexpr unsigned BT_FLAG_BARRIER = 2u;     // flags bit: a team barrier gave up waiting
@@ -2300,14 +2305,18 @@ constexpr unsigned TEAM_CLOSED = 1u << 31;   // registration word's bit
 constexpr unsigned TEAM_NONE = ~0u;          // team size word: no slot left, leave
 constexpr unsigned TEAM_SPINS = 1u << 22;    // polls (over a second) before a wait gives up
 // The work of a slot, in cell tiles (an env tile costs about four), up to which the
-// team kernel is the default. us per step, team against replayed graphs (FP64):
-//   plain     4 cell + 1 env tiles   7.2 / 15.9     145 + 16  13.5 / 16.2
-//             37 + 16                8.8 / 17.3     193 + 25  16.7 / 16.3
-//             8 clusters of 200-400 cells 9.5 / 16.2, of 1,000-1,600 13.3 / 19.0,
-//             48 of 60-200 cells 13.7 / 16.7, 64 of them 18.5 / 16.5
-//   ordered   4 + 1                 15.2 / 19.0     61 + 9    18.6 / 20.0
-//   (channels or a Ca pump)         61 + 16 19.1 / 19.7   93 + 9 20.2 / 19.6
-// Beyond, one XCD's 32 CUs have more to do than eight times as many save.
+// team kernel is the default. us per step, team / replayed graphs, FP64 and FP32 flux:
+//   plain     4 cell + 1 env tiles   7.6 / 16.1   7.3 / 16.0
+//             37 + 16               10.1 / 17.3   8.6 / 17.8
+//             143 + 16              12.4 / 17.9  11.1 / 17.7
+//             191 + 25              16.6 / 16.4  16.5 / 16.5
+//             8 clusters of 200-400 cells 10.1 / 16.4, 9.4 / 16.9, of 1,000-1,600 13.6 / 18.4,
+//             12.2 / 18.3; 48 of 60-200 cells 14.2 / 18.5, 14.1 / 18.3, 64 of them 14.2 / 18.9
+//   ordered   4 + 1                 16.0 / 19.3  15.0 / 19.6
+//   (channels or a Ca pump)         60 + 9 19.7 / 20.3, 18.5 / 20.5;  60 + 16 19.3 / 19.5,
+//             18.1 / 19.8;  93 + 9 21.4 / 20.1, 19.8 / 20.3
+// Beyond, one XCD's 32 CUs have about as much more to do as the launches cost (a few
+// sizes still gain: 222 + 16 16.0 / 17.6, 14.2 / 18.1).
 constexpr int TEAM_TILES = 220;
 constexpr int TEAM_TILES_ORDERED = 100;
 constexpr int TEAM_STEPS = 1 << 12;          // steps per launch: even, and a team that formed short of blocks is soon re-formed
@@ -3736,7 +3745,7 @@ int bt_create(bt_ctx** out, const bt_params* p, const bt_cluster* cl, int32_t n_
             c->slots_host.push_back(TeamSlot{0, b->n_tiles, 0, c->n_env_tiles, 0, (int)sq_live.size(), 0, p->n_cells, 0,
                                              p->n_squares, 0, p->n_mems});
         } else {
-            // a cluster's cost: its cell tiles and env tiles (about equal times)
+            // a cluster's cost in cell tiles: an env tile takes about as long as four
             auto cost = [&](int q) {
                 return c->cl_tile0[q + 1] - c->cl_tile0[q] + 4 * (c->cl_env0[q + 1] - c->cl_env0[q]);
             };
