@@ -4388,7 +4388,7 @@ int bt_step_observed(bt_ctx* c, int32_t n_steps, int32_t use_graph, const bt_obs
         --n_steps;
     }
     const int ahead = n_steps - 1;
-    const int odd = use_team(c, use_graph) ? 0 : ahead & 1;     // (the team kernel takes either)
+    const int odd = ahead & 1;
     if (ahead > 0) {
         // keep the graph on the caller buffers: an even number of graph steps, then eager ones
         int rc = bt_step(c, ahead - odd, use_graph);

@@ -133,3 +133,26 @@ def test_groups_stop_at_the_first_nan(large, cells, squares, n):
             assert np.array_equal(got["c_env"][:, c], clean["c_env"][:, c]), q
         for k in ("v_env", "E_x", "E_y"):
             assert np.array_equal(got[k][c], before[k][c]), (q, k)
+
+
+@pytest.mark.parametrize("period", [9, 10])
+@pytest.mark.parametrize("n_clusters,square_of", [(1, 0), (5, 3)])
+def test_sampled_loop_stops_at_the_first_nan(n_clusters, square_of, period):
+    """Even and odd counts of steps before a sampled one, the NaN among them."""
+    worlds = batched_worlds(n_clusters=n_clusters, cells_range=(60, 90), grid_range=(33, 36), seed=4)
+    for p, _ in worlds:
+        p.init_time_sampling = period * p.init_time_step
+        p.set_phase_time("init")
+    runs = []
+    for tuning in (SEPARATE, None):
+        b = batch(worlds, "fp64", tuning=tuning)
+        b.step_n(6)
+        plant(b, [], [square_of])
+        with pytest.raises(BetseSimUnstableException) as e:
+            b.run_loop(60)
+        runs.append((e.value.step, everything(b)))
+        b.close()
+    say(f"case: {n_clusters} clusters, sampled every {period} steps, NaN at step {[r[0] for r in runs]}")
+    assert runs[0][0] == runs[1][0]
+    for k, v in runs[0][1].items():
+        assert np.array_equal(v, runs[1][1][k], equal_nan=True), k
