@@ -2303,6 +2303,7 @@ constexpr unsigned BT_FLAG_BARRIER = 2u;     // flags bit: a team barrier gave u
 constexpr unsigned TEAM_STOP = 1u << 31;     // barrier word's bit: a NaN in the slot
 constexpr unsigned TEAM_CLOSED = 1u << 31;   // registration word's bit
 constexpr unsigned TEAM_NONE = ~0u;          // team size word: no slot left, leave
+constexpr unsigned TEAM_HALTED = 1u << 30;   // slot word's bit: an earlier launch halted the run
 constexpr unsigned TEAM_SPINS = 1u << 22;    // polls (over a second) before a wait gives up
 // The work of a slot, in cell tiles (an env tile costs about four), up to which the
 // team kernel is the default. us per step, team / replayed graphs, FP64 and FP32 flux:
@@ -2460,7 +2461,9 @@ k_step_team(TeamArgs) {
         const unsigned f = agent_load(flags);
         long long stop = -1;
         if (f != 0u) stop = (long long)ld<true>(args()->mem[0].bad_step) - args()->step0;
-        const bool run = !(f & BT_FLAG_BARRIER) && (f != 0u ? stop >= 0 : mode == TEAM_RUN);
+        // (halted, an odd count still ends with the state in the caller's buffers)
+        const bool was = f != 0u && stop < 0, back = was && mode == TEAM_RUN && (args()->n_steps & 1);
+        const bool run = !(f & BT_FLAG_BARRIER) && (f != 0u ? !was || back : mode == TEAM_RUN);
         s_stop = (f != 0u && mode != TEAM_RUN) ? (int)stop : -1;
         int size = 0;
         const unsigned t = atomicAdd(&T->reg, 1u);
@@ -2474,7 +2477,7 @@ k_step_team(TeamArgs) {
                     const unsigned long long t0 = wall_clock64();      // 100 MHz
                     while (agent_load(&T->reg) < (unsigned)n_blocks && wall_clock64() - t0 < 3000ull) {}
                     size = (int)atomicOr(&T->reg, TEAM_CLOSED);
-                    __hip_atomic_store(&T->slot, slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(&T->slot, slot | (back ? TEAM_HALTED : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __hip_atomic_store(&T->size, (unsigned)size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
@@ -2493,6 +2496,8 @@ k_step_team(TeamArgs) {
     const int rank = __builtin_amdgcn_readfirstlane(s_rank), nb = __builtin_amdgcn_readfirstlane(s_size);
     if (nb == 0) return;
     int slot = __builtin_amdgcn_readfirstlane(s_slot);
+    const bool halted_before = slot >= 0 && (slot & TEAM_HALTED);
+    if (halted_before) slot &= (int)~TEAM_HALTED;
     const int stop = __builtin_amdgcn_readfirstlane(s_stop);    // the step to go back to, if any
     unsigned target = 0;
     const int wave = __builtin_amdgcn_readfirstlane(tid / TMB), lane = tid % TMB;
@@ -2588,7 +2593,7 @@ k_step_team(TeamArgs) {
         };
         const bool several = args()->save.c_cell != nullptr, rewind = stop >= 0;
         unsigned word = 1;
-        if (rewind || (several && mode == TEAM_RUN)) {
+        if (rewind || (several && mode == TEAM_RUN && !halted_before)) {
             each_row([&](const double* x, double* kept, int lo, int hi) {
                 double* const to = rewind ? const_cast<double*>(x) : kept;
                 const double* const from = rewind ? kept : x;
@@ -2599,7 +2604,7 @@ k_step_team(TeamArgs) {
             if (word == 0) return;
         }
         int s = 0;
-        for (; s < ((mode == TEAM_RUN || rewind) ? n_steps : 0); ++s) {
+        for (; s < (((mode == TEAM_RUN && !halted_before) || rewind) ? n_steps : 0); ++s) {
             const int par = s & 1;
             // (where the exchange is in the env kernel, a NaN's step has no env phase)
             if (s != stop || !args()->fused) env_phase(par);
@@ -2618,9 +2623,9 @@ k_step_team(TeamArgs) {
             if (word == 0) return;
         }
         const table<TeamArgs> TA = args();
-        const bool stopped = (word & TEAM_STOP) || rewind;
+        const bool stopped = (word & TEAM_STOP) || rewind || halted_before;
         if (stopped) {
-            if (rank == 0 && tid == 0 && !rewind) {
+            if (rank == 0 && tid == 0 && !rewind && !halted_before) {
                 atomicMin(TA->mem[0].bad_step, (unsigned long long)(TA->step0 + s));
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 atomicOr(flags, 1u);

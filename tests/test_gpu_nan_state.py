@@ -58,13 +58,16 @@ def halted_states(worlds, flux_mode, tunings, n, cells, squares):
         assert e2.value.step == e.value.step
         for k, v in everything(b).items():
             assert np.array_equal(v, st[k], equal_nan=True), k
-        runs.append((e.value.step, st))
+        with pytest.raises(BetseSimUnstableException):
+            b.step_n(5)                  # (an odd count ends with the workspace's state in the caller's buffers)
+        runs.append((e.value.step, st, everything(b)))
         b.close()
     say(f"  first NaN at step {[r[0] for r in runs]}")
-    for step, st in runs[1:]:
+    for step, *states in runs[1:]:
         assert step == runs[0][0]
-        for k, v in st.items():
-            assert np.array_equal(v, runs[0][1][k], equal_nan=True), k
+        for st, want in zip(states, runs[0][1:]):
+            for k, v in st.items():
+                assert np.array_equal(v, want[k], equal_nan=True), k
     return runs[0][0]
 
 
@@ -156,3 +159,10 @@ def test_sampled_loop_stops_at_the_first_nan(n_clusters, square_of, period):
     assert runs[0][0] == runs[1][0]
     for k, v in runs[0][1].items():
         assert np.array_equal(v, runs[1][1][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("n_clusters", [1, 3])
+def test_a_nan_in_a_call_of_several_launches(n_clusters):
+    """More steps than one launch of the persistent kernel runs."""
+    worlds = batched_worlds(n_clusters=n_clusters, cells_range=(20, 60), grid_range=(12, 20), seed=4)
+    assert halted_states(worlds, "fp64", (SEPARATE, None), 9001, [], [n_clusters - 1]) < 40
