@@ -467,7 +467,8 @@ int bt_gnn_backward(const float* const* params, int32_t f_in, int32_t f_out, int
 
 /* Wait for the stream; return BT_OK or BT_UNSTABLE (a NaN was produced; the
  * state is frozen at the step that produced it and *bad_step receives its
- * 0-based index counted from context creation, or -1). With streams > 1
+ * 0-based index counted from context creation, or -1: the first of them, and
+ * every cluster of a batch is at that step). With streams > 1
  * (bt_tuning) the clusters of the other stream groups stop where their own
  * stream had got to within the same bt_step call. */
 int bt_sync(bt_ctx* ctx, int64_t* bad_step);
