@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 
 from betse_amd.batch import BatchSimulator, batched_worlds
+from betse_amd.cells import Cells
 from betse_amd.channels import draw_channel_state
+from betse_amd.parameters import Parameters
 from tests.test_gpu_configs import say, state
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +70,18 @@ def test_channels(n_clusters, cells, grid, flux_mode):
     small = n_clusters > 1
     tiles = compare_forms(worlds, flux_mode, ALL if small else [(TEAM, True, 1), (GRAPHS, True, 0), (None, False, 0)])
     assert small or tiles > 160
+
+
+@pytest.mark.parametrize("flux_mode", ["fp64", "fp32"])
+def test_channels_of_triangular_cells(flux_mode):
+    """Tiles of 21 cells (three membranes each) with three channels: a block's LDS
+    holds fewer tiles than it has wavefronts."""
+    p = Parameters.preset("tiny_full")
+    p.network, p.cluster_radius, p.grid_size = None, 380e-6, 33
+    a, n = 10e-6, 44                      # cells around the vertices of a honeycomb
+    i, j = np.meshgrid(np.arange(-n, n), np.arange(-n, n), indexing="ij")
+    x, y = 1.5 * a * i.ravel(), np.sqrt(3) * a * (j + 0.5 * (i % 2)).ravel()
+    cells = Cells.make_world(p, points=np.stack([np.concatenate([x, x + a]), np.concatenate([y, y])], axis=1))
+    assert set(cells.num_mems.tolist()) == {3}
+    draw_channel_state(p, cells.n_cells, cells.n_mems)
+    assert compare_forms([(p, cells)], flux_mode, [(TEAM, True, 1), (GRAPHS, True, 0), (None, False, 0)]) > 160
